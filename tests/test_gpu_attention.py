@@ -100,6 +100,26 @@ def test_decode_request_order(dev, B):
         assert torch.equal(gotp.cpu(), got.cpu()[perm]), f"B={B} splits {splits}: permuted batch differs"
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("splits", [2, 31, 32, 33, 64])
+def test_decode_merge_of_many_splits(dev, splits, D):
+    """The merge takes partials in rounds of 32: counts at, below and past a round, requests whose
+    contexts leave most splits empty (those write no partial: the workspace holds NaN before), and
+    a head count that leaves lanes of the merge without a head."""
+    print(f"decode merge splits={splits} D={D}", flush=True)
+    ctx = torch.tensor([0, 127, 128, 129, 4095, 4200, 8191])
+    a = wl.attn_batch(ctx, torch.ones(7, dtype=torch.int32), Hq=6, Hkv=2, D=D, page_size=16, seed=splits)
+    pb = a["batch"]
+    ws = torch.full((WS_BYTES // 4,), float("nan"), device=dev)
+    w = attention.BatchDecodeWithPagedKVCacheWrapper(ws, "NHD")
+    w.plan(pb.kv_indptr.to(dev), pb.kv_indices.to(dev), pb.kv_last_page_len.to(dev), 6, 2, D, 16)
+    w._plan["splits"] = splits
+    got = w.run(a["q"].to(dev), a["cache"].to(dev))
+    want = _want(a)
+    assert_bf16_close(N(got), want, what="decode merge")
+    _tight(got, want, "decode merge")
+
+
 def test_decode_page_size_one_long_context(dev):
     """Page size 1: a 1500-token context spans several 510-page windows of the staged table."""
     a = wl.attn_batch(torch.tensor([1499, 700, 3]), torch.ones(3, dtype=torch.int32), Hq=8, Hkv=2,
