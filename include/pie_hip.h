@@ -421,6 +421,43 @@ int pie_hip_attention_prefill(const pie_bf16* q, int64_t q_tok_stride, int64_t q
                               pie_bf16* out, int64_t o_tok_stride, int64_t o_head_stride,
                               void* stream);
 
+/*
+ * The prefill form with items cut over their kv range, for batches that would leave most of the
+ * chip idle (a few query tokens over long contexts). pie_hip_attention_prefill_split_plan takes the
+ * plan's arguments, the run's window_left, the device's compute units (0: 256) and the bytes of
+ * the workspace that will hold the plan, then (mode 2) the packed mask and the extents, each
+ * 16-byte aligned, then the run's scratch. It writes the same plan and, after it, a list with the
+ * longest items cut, where that pays and plan_capacity (8 words more per piece) and the workspace
+ * hold it: split[5] = {word of the cut items, their number (0: no cut), word of the merge list,
+ * its entries, scratch bytes}. pie_hip_attention_prefill_split takes pie_hip_attention_prefill's
+ * arguments, that array and 16-byte-aligned scratch. Runs of one plan share its scratch: for
+ * head_dim 128 overlapping runs are refused as above; for 64 and 256 a run that is captured, or made
+ * while another stream's run uses the scratch, runs the uncut items.
+ */
+int pie_hip_attention_prefill_split_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
+                                         const int32_t* kv_last_page_len, int64_t batch,
+                                         int64_t page_size, int64_t num_qo_heads,
+                                         int64_t num_kv_heads, int64_t head_dim, int32_t mode,
+                                         int64_t window_left, int64_t num_cus,
+                                         int64_t workspace_bytes, int32_t* plan,
+                                         int64_t plan_capacity, int64_t* plan_words,
+                                         int64_t* num_items, int64_t* mask_bytes,
+                                         int64_t* mask_words, int64_t* split);
+int pie_hip_attention_prefill_split(const pie_bf16* q, int64_t q_tok_stride, int64_t q_head_stride,
+                                    const pie_bf16* k_cache, const pie_bf16* v_cache,
+                                    int64_t page_stride, int64_t slot_stride, int64_t head_stride,
+                                    int64_t num_pages, const int32_t* qo_indptr,
+                                    const int32_t* kv_indptr, const int32_t* kv_indices,
+                                    const int32_t* kv_last_page_len, int64_t num_qo_heads,
+                                    int64_t num_kv_heads, int64_t head_dim, int64_t page_size,
+                                    float sm_scale, int32_t mode, int64_t window_left,
+                                    const float* sinks, const uint32_t* packed_mask,
+                                    const int32_t* mask_extent, const int32_t* plan,
+                                    int64_t num_items, int64_t mask_offsets_word,
+                                    const int64_t* split, void* scratch, int64_t scratch_bytes,
+                                    pie_bf16* out, int64_t o_tok_stride, int64_t o_head_stride,
+                                    void* stream);
+
 
 /*
  * Sampling from probabilities, one draw per row: flashinfer.sampling.sampling_from_probs (mode 0),

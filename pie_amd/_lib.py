@@ -56,6 +56,11 @@ SIGNATURES: dict[str, list] = {
     "pie_hip_attention_prefill": [vp, i64, i64, vp, vp, i64, i64, i64, i64, vp, vp, vp, vp, i64,
                                   i64, i64, i64, f32, i32, i64, vp, vp, vp, vp, i64, i64, vp, i64,
                                   i64, vp],
+    "pie_hip_attention_prefill_split_plan": [vp, vp, vp, i64, i64, i64, i64, i64, i32, i64, i64, i64,
+                                             vp, i64, vp, vp, vp, vp, vp],
+    "pie_hip_attention_prefill_split": [vp, i64, i64, vp, vp, i64, i64, i64, i64, vp, vp, vp, vp, i64,
+                                        i64, i64, i64, f32, i32, i64, vp, vp, vp, vp, i64, i64, vp, vp,
+                                        i64, vp, i64, i64, vp],
     "pie_hip_sample": [vp, i64, i64, i64, i64, vp, i32, vp, i32, vp, f32, vp, f32, vp, u64, u64, vp, vp],
     "pie_hip_scaled_softmax": [vp, i32, i64, i64, i64, vp, f32, vp, i64, vp],
     "pie_hip_group_begin": [],

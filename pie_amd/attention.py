@@ -227,15 +227,18 @@ class BatchPrefillWithPagedKVCacheWrapper:
         mode = 2 if mask is not None else (1 if causal else 0)
         G = num_qo_heads // num_kv_heads
         T = int(qo_h[-1]) if batch else 0
-        n_items = T * G // 64 + batch + 1
-        # header, 8-word items, the persistent schedule (slot offsets, one word per (kv head,
-        # item) unit), mask offsets
-        cap = 16 + 8 * n_items + (4096 + n_items * num_kv_heads) + 4 * batch + 8
-        plan = np.zeros(cap, dtype=np.int32)
+        ws_bytes = self._workspace.numel() * self._workspace.element_size()
+        cus = _num_cus(dev) if dev.type == "cuda" else 0
+        n_items = T * G // 128 + batch + 1
+        # header, 8-word items, mask offsets, and for a split list the items again, at most ~2
+        # pieces per work group the device runs at once beyond one each, and a merge entry each
+        cap = 16 + 8 * n_items + 4 * batch + 8 + 8 * (2 * n_items + 4 * (cus or 256))
+        plan = np.empty(cap, dtype=np.int32)
         words, items, mbytes, mwords = C.c_int64(0), C.c_int64(0), C.c_int64(0), C.c_int64(0)
-        _lib.call("pie_hip_attention_prefill_plan", qo_h.data_ptr(), kv_h.data_ptr(), ll_h.data_ptr(),
-                  batch, page_size, num_qo_heads, num_kv_heads, head_dim_qk, mode, plan.ctypes.data, cap,
-                  C.byref(words), C.byref(items), C.byref(mbytes), C.byref(mwords))
+        split = (C.c_int64 * 5)()
+        _lib.call("pie_hip_attention_prefill_split_plan", qo_h.data_ptr(), kv_h.data_ptr(), ll_h.data_ptr(),
+                  batch, page_size, num_qo_heads, num_kv_heads, head_dim_qk, mode, window_left, cus, ws_bytes,
+                  plan.ctypes.data, cap, C.byref(words), C.byref(items), C.byref(mbytes), C.byref(mwords), split)
         if mode == 2:
             if mask.dtype not in (torch.bool, torch.uint8):
                 raise ValueError(f"{name}: custom_mask must be bool, got {mask.dtype}")
@@ -244,13 +247,15 @@ class BatchPrefillWithPagedKVCacheWrapper:
                 raise ValueError(f"{name}: custom_mask has {mask.numel()} entries, the batch needs "
                                  f"{mbytes.value} (sum of qo_len * kv_len)")
             mask = mask.to(dev).contiguous()
-        # workspace layout: [plan words | packed mask words | per-token extents] (mode 2), each
-        # 16-byte aligned
+        # workspace layout: [plan words | packed mask words | per-token extents (mode 2) | partial
+        # results of split items], each 16-byte aligned
         nbytes = (words.value * 4 + 15) // 16 * 16
         mask_off = nbytes
         ext_off = mask_off + (mwords.value * 4 + 15) // 16 * 16
         need = ext_off + T * 4 if mode == 2 else nbytes
-        ws_bytes = self._workspace.numel() * self._workspace.element_size()
+        scratch_off = (need + 15) // 16 * 16
+        if split[4] and scratch_off + split[4] > ws_bytes:
+            split[1] = split[4] = 0
         if need > ws_bytes:
             raise ValueError(f"{name}: the plan needs {need} bytes of workspace, have {ws_bytes}")
         ws8 = self._workspace.view(torch.uint8)
@@ -270,7 +275,8 @@ class BatchPrefillWithPagedKVCacheWrapper:
                           last_page_len=tables[3], batch=batch, T=T, Hq=num_qo_heads,
                           Hkv=num_kv_heads, D=head_dim_qk, P=page_size, mode=mode, packed=packed, extent=extent,
                           window_left=window_left,
-                          plan=plan_d, items=items.value, woff_word=int(plan[4]),
+                          plan=plan_d, items=items.value, woff_word=int(plan[4]), split=split,
+                          scratch=ws8[scratch_off: scratch_off + split[4]],
                           sm_scale=(1.0 / math.sqrt(head_dim_qk)) if sm_scale is None else sm_scale)
 
     begin_forward = plan
@@ -307,15 +313,16 @@ class BatchPrefillWithPagedKVCacheWrapper:
         packed = p["packed"]
         if p["mode"] == 2 and packed is None:  # a mask over zero positions: nothing is visible
             return out.zero_()
-        _lib.call("pie_hip_attention_prefill", q.data_ptr(), q.stride(0), q.stride(1), kp, vp, ps,
+        scratch = p["scratch"]
+        _lib.call("pie_hip_attention_prefill_split", q.data_ptr(), q.stride(0), q.stride(1), kp, vp, ps,
                   ss, hs, npages, p["qo_indptr"].data_ptr(), p["indptr"].data_ptr(),
                   p["indices"].data_ptr(), p["last_page_len"].data_ptr(), Hq, Hkv, D, P,
                   float(p["sm_scale"]), p["mode"], p["window_left"],
                   None if _sinks is None else _sinks.data_ptr(),
                   packed.data_ptr() if packed is not None else None,
                   p["extent"].data_ptr() if p["extent"] is not None else None,
-                  p["plan"].data_ptr(), p["items"], p["woff_word"], out.data_ptr(), out.stride(0),
-                  out.stride(1), _stream(q))
+                  p["plan"].data_ptr(), p["items"], p["woff_word"], p["split"], scratch.data_ptr(),
+                  scratch.numel(), out.data_ptr(), out.stride(0), out.stride(1), _stream(q))
         return out
 
     forward = run

@@ -7,7 +7,8 @@
 // query token i attends kv positions t <= kv_len - qo_len + i (or where the custom mask is set),
 // head h reads kv head h / (Hq/Hkv), scores are q.k * sm_scale, output is softmax(scores) @ v.
 //
-// MI355X mapping. Both kernels run the matrix products on MFMA v_mfma_f32_16x16x32_bf16:
+// MI355X mapping. Decode runs the matrix products on MFMA v_mfma_f32_16x16x32_bf16 (prefill, below,
+// on v_mfma_f32_32x32x16_bf16 with the output transposed):
 //   S^T = K Q^T   A = 16 kv tokens x 32 head dims (straight from HBM into registers: lane
 //                 (n, g) holds token n's dims 8(4s+g)..+8 at step s, one 64-byte run per token
 //                 per step), B = 16 query rows (the same dims permutation), C = S^T tile with
@@ -617,47 +618,63 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(PagedKV kv, int window_
 
 // ------------------------------------------------------------------------------ prefill
 // Work item: request b, first packed query row row0 (row R = query token R / G, head R % G of
-// the kv head's group). A work group of prefill_waves<D> waves owns prefill_rows<D> rows
-// (prefill_row_tiles<D> 16-row MFMA row tiles per wave) and streams the request's kv tokens in 32-token tiles: the four waves load each K
-// and V tile cooperatively (three tiles ahead through registers, then into LDS, chunk-swizzled,
-// double-buffered),
-// then every wave reads the K and V MFMA operands it needs into registers before the next
-// tile's loads are issued, and runs both row tiles against them.
+// the kv head's group). A work group of four waves owns kPrefillRows = 128 rows, 32 per wave, and
+// streams the request's kv tokens in tiles of prefill_tile<D> tokens; the four waves load each K
+// and V tile cooperatively into registers (two tiles ahead) and then into LDS (chunk-swizzled,
+// double-buffered).
 // Visibility: mode 0 every cached position, 1 causal (t <= kv_len - qo_len + i), 2 the custom
 // mask, bit-packed by attn_pack_mask_kernel: query token i of request b reads 32-bit word
 // w (kv positions 32w..32w+31) at packed + word_off[b] + i * ceil(kv_len / 32) + w.
-// Work-group shape of attn_prefill_kernel: 4 waves of two 16-row MFMA row tiles (one for D = 256,
-// whose accumulators would not fit twice). Head dim 128 runs attn_prefill32_kernel (32 rows per
-// wave, same 128-row work items).
+//
+// The products run on v_mfma_f32_32x32x16_bf16, the output transposed:
+//   S^T = K Q^T    A = 32 kv tokens x 16 dims (lane (t, kg): token t's dims 8(2s+kg)..+8 at
+//                  step s, from LDS), B = 32 query rows (lane (r, kg): row r, the same dims)
+//   O^T = V^T P^T  A = 32 dims x 16 tokens (two transpose reads of 4 V rows each),
+//                  B = P^T: lane (r, kg) holds row r's probabilities of tokens
+//                  16j + 8(e/4) + 4kg + e%4, exactly 8 consecutive registers of S^T's C layout
+// so every lane owns one query row r = lane % 32 in both products: its running max, sum and
+// rescale factor are its own (one exchange with lane ^ 32 for the max), and no factor has to be
+// broadcast to other lanes.
+//
+// What bounds it (rocprofv3 counters, 8 x 8192 tokens at head dim 128): MFMA 37% busy, VALU 40%, LDS
+// 28%, no bank conflicts; a wave waits 36% of its time, for the tile's loads (without them the
+// kernel takes 22% less) and at the barrier. Work groups of four 32-row waves in 64-token tiles,
+// each MFMA's V operands read a step ahead, against the four 2 x 16-row waves on 16x16x32 MFMAs in
+// 32-token tiles before: head dim 64, 4 x 4000 tokens 1,531 -> 827 us (674 TFLOP/s); head dim 256
+// (one 16-row tile per wave before) 1,858 -> 922 us (568 TFLOP/s). At head dim 256 one wave fits a
+// SIMD and nothing runs under its softmax.
+constexpr int kPrefillRows = 128;
+// kv tokens per tile: 64, or 32 at head dim 256, whose accumulators fill the registers
 template <int D>
-constexpr int prefill_waves() { return 4; }
+constexpr int prefill_tile() { return D == 256 ? 32 : 64; }
+// work groups per CU the registers are budgeted for
 template <int D>
-constexpr int prefill_row_tiles() { return D == 256 ? 1 : 2; }
-template <int D>
-constexpr int prefill_min_waves() { return D == 256 ? 1 : 2; }
-template <int D>
-constexpr int prefill_rows() { return 16 * prefill_waves<D>() * prefill_row_tiles<D>(); }
+constexpr int prefill_groups() { return D == 256 ? 1 : 2; }
 constexpr int kPlanHeader = 16;  // plan words before the items: [0] items, [1] batch, [2] rows per item
+// Plan word 2: rows per item; head dim 256 sets another value, so that its plans and those of
+// the other head dims do not drive each other's kernels.
+constexpr int plan_rows_word(int64_t D) { return D == 256 ? kPrefillRows | (1 << 16) : kPrefillRows; }
+constexpr int kPlanChunkWord = 5;  // kv tokens per piece of a split item
 // Plan words the head-dim-128 kernel uses as counters: the next unit of each XCD's queue, and
 // the work groups that have finished (the last one sets all nine back to zero).
 constexpr int kPlanQueueWord = 8, kPlanDoneWord = 7;
-// words per work item: request b, first packed row, and the request's q0 (first query token),
+// words per work item: request b, first packed row, the request's q0 (first query token),
 // qo_len, kv_len and first page-table slot, so the kernels' prologue reads one 32-byte item
-// instead of chasing b through qo_indptr / kv_indptr / kv_last_page_len; two pad words
+// instead of chasing b through qo_indptr / kv_indptr / kv_last_page_len; then, for an item split
+// over its kv range, the piece's index and 1 + its partial-result slot (0: not split)
 constexpr int kPlanItemWords = 8;
+// words per merge entry of a split plan: first packed row, q0, qo_len, first slot, pieces
+constexpr int kPlanMergeWords = 8;
 
 // XCD-aware order of the prefill grid: work groups are dispatched round-robin over the 8 XCDs
 // (id mod 8), each with its own L2, so XCD x takes the contiguous run [x * per, (x + 1) * per) of
 // the (kv head, item) units. The plan lists each request's items together, so the work groups an
 // XCD runs at one time mostly read the same request's K/V prefix through one L2. Returns the
-// unit's plan item and sets kvh, or nullptr for the padding work groups past the last unit.
-__device__ __forceinline__ const int32_t* prefill_unit(const int32_t* plan, int n_items, int n_kv_heads,
-                                                       int& kvh) {
-  const int units = n_items * n_kv_heads, per = (units + 7) / 8;
+// unit's number, or -1 for the padding work groups past the last unit.
+__device__ __forceinline__ int prefill_unit(int units) {
+  const int per = (units + 7) / 8;
   const int u = (int)(blockIdx.x & 7u) * per + (int)(blockIdx.x >> 3);
-  if (u >= units) return nullptr;
-  kvh = u / n_items;
-  return plan + kPlanHeader + kPlanItemWords * (u - kvh * n_items);
+  return u < units ? u : -1;
 }
 
 // attn_mask_extent_kernel marks a query token whose mask row is exactly causal (positions
@@ -670,7 +687,8 @@ constexpr int kExtentCausal = 1 << 30;
 __device__ __forceinline__ void mask_rows_extent(const int32_t* __restrict__ extent, int q0, int row0, int rows,
                                                  int G, int nrows, int& ext, bool& causal) {
   __shared__ int s_ext, s_mixed;
-  if (threadIdx.x == 0) { s_ext = 0; s_mixed = 0; }
+  const int zero = opaque_v(0);  // a constant pair would be kept in registers over the caller's loop
+  if (threadIdx.x == 0) { s_ext = zero; s_mixed = zero; }
   __syncthreads();
   const int r = row0 + (int)threadIdx.x;
   if ((int)threadIdx.x < nrows && r < rows) {
@@ -683,9 +701,9 @@ __device__ __forceinline__ void mask_rows_extent(const int32_t* __restrict__ ext
   causal = s_mixed == 0;
 }
 
-// A plan made for another head_dim (its rows per item differ) cannot drive this kernel: every
-// work group fills the whole output (the plan's tokens, all q heads) with NaN instead, so the
-// mistake shows in the result rather than leaving the output unwritten.
+// A plan made for another head_dim cannot drive this kernel: every work group fills the whole
+// output (the plan's tokens, all q heads) with NaN instead, so the mistake shows in the result
+// rather than leaving the output unwritten.
 template <int D>
 __device__ void prefill_plan_mismatch(const int32_t* __restrict__ plan, const int32_t* __restrict__ qo_indptr,
                                       int Hq, uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs) {
@@ -700,282 +718,6 @@ __device__ void prefill_plan_mismatch(const int32_t* __restrict__ plan, const in
   }
 }
 
-template <int D>
-__global__ __launch_bounds__(64 * prefill_waves<D>(), prefill_min_waves<D>()) void attn_prefill_kernel(
-    const uint16_t* __restrict__ q, int64_t q_ts, int64_t q_hs, PagedKV kv,
-    const int32_t* __restrict__ qo_indptr, int G, float scale_log2, const int32_t* __restrict__ plan,
-    int n_items, int n_kv_heads,
-    int mode_in, int window_left, const uint32_t* __restrict__ packed,
-    const int64_t* __restrict__ word_off, const int32_t* __restrict__ extent,
-    uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const float* __restrict__ sinks) {
-  using W = WaveAttn<D>;
-  constexpr int NS = W::NS, NB = W::NB, CH = D / 8, RPI = 64 / CH;
-  constexpr int RT = prefill_row_tiles<D>(), kPrefillRows = prefill_rows<D>();
-  constexpr int NW = prefill_waves<D>(), NT = 64 * NW;  // waves, threads
-  constexpr int TILE = kTileTokens * D;  // elements of one K or V tile
-  constexpr int kSmemLoop = 2 * 2 * TILE * 2;
-  constexpr int kSmemOut = kPrefillRows * D * 2;
-  constexpr int kSmem = kSmemLoop > kSmemOut ? kSmemLoop : kSmemOut;
-  __shared__ __attribute__((aligned(16))) char smem[kSmem];
-  __shared__ int32_t ptab[kPageWin];
-
-  if (plan[2] != kPrefillRows) {
-    prefill_plan_mismatch<D>(plan, qo_indptr, G * n_kv_heads, out, o_ts, o_hs);
-    return;
-  }
-  int kvh;
-  const int32_t* item = prefill_unit(plan, n_items, n_kv_heads, kvh);
-  if (!item) return;  // padding work group
-  const int b = item[0], row0 = item[1], q0 = item[2], qo_len = item[3], kv_len = item[4];
-  const int page0 = item[5];
-  const int lane = threadIdx.x & 63, w = uniform(threadIdx.x >> 6);
-  const int n = lane & 15, g = lane >> 4;
-  const int rows = qo_len * G;
-  int mode = mode_in, mext = 0;  // a custom mask that is causal for all the rows: the causal path
-  if (mode_in == 2) {
-    bool causal;
-    mask_rows_extent(extent, q0, row0, rows, G, kPrefillRows, mext, causal);
-    mode = uniform(causal ? 1 : 2);  // wave-uniform (a scalar register), like the argument
-  }
-
-  // this lane's query rows (row n of each of the wave's row tiles)
-  W st[RT];
-  int lim[RT], tok[RT], lo[RT];  // visible positions of the row: lo..lim (and the mask)
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    st[rt].init();
-    const int R = row0 + 16 * RT * w + 16 * rt + n;
-    const bool valid = R < rows;
-    const int i = valid ? R / G : 0, hg = valid ? R - i * G : 0;
-    tok[rt] = i;
-    lim[rt] = !valid ? -1 : mode == 1 ? min(kv_len - qo_len + i, kv_len - 1) : kv_len - 1;
-    lo[rt] = window_left >= 0 ? kv_len - qo_len + i - window_left : 0;
-    const uint16_t* qp = q + (int64_t)(q0 + i) * q_ts + (int64_t)(kvh * G + hg) * q_hs;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const u32x4_t z = {0u, 0u, 0u, 0u};
-      st[rt].qb[s] = valid ? ld16v(qp + 8 * (4 * s + g)) : z;
-    }
-  }
-  // kv positions any row of this work group can see (mode 2: the furthest set mask bit of its
-  // rows' query tokens, from attn_mask_extent_kernel)
-  const int last_row = min(rows, row0 + kPrefillRows) - 1;
-  int kv_end = mode == 1 ? min(kv_len, kv_len - qo_len + last_row / G + 1) : kv_len;
-  if (mode == 2) kv_end = min(kv_len, mext);
-  // sliding window: no row of the work group sees positions before its first row's window
-  // (tiles start 32-aligned so mask words line up)
-  const int kv_begin = window_left >= 0 ? max(0, kv_len - qo_len + row0 / G - window_left) & ~31 : 0;
-  int wave_lo = 0;  // the largest window start of the wave's rows (uniform)
-  if (window_left >= 0) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) wave_lo = max(wave_lo, lim[rt] < 0 ? 0 : lo[rt]);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) wave_lo = max(wave_lo, __builtin_amdgcn_ds_bpermute((lane ^ o) << 2, wave_lo));
-    wave_lo = uniform(wave_lo);
-  }
-  // mode 2: this lane's rows' mask words; modes 0/1: the last kv position every row of the wave
-  // sees (tiles ending at or before it need no per-element visibility test)
-  const uint32_t* mword[RT];
-  const int nw = (kv_len + 31) / 32;
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) mword[rt] = mode == 2 ? packed + word_off[b] + (int64_t)tok[rt] * nw : nullptr;
-  int wave_lim = 0x7fffffff;
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) wave_lim = min(wave_lim, lim[rt] < 0 ? 0x7fffffff : lim[rt]);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) wave_lim = min(wave_lim, __builtin_amdgcn_ds_bpermute((lane ^ o) << 2, wave_lim));
-  wave_lim = uniform(wave_lim);
-  __shared__ int window_bad;
-  __shared__ uint32_t mwt[2][RT][NT];  // mode 2: mask words of the tiles in LDS, per lane
-
-  uint16_t* kt = reinterpret_cast<uint16_t*>(smem);  // [2 buffers][K, V][32][D]
-  constexpr int WR = kTileTokens / NW;  // rows of each K / V tile one wave loads
-  constexpr int NL = WR / RPI;          // load instructions per wave for them
-  static_assert(NL >= 1 && WR % RPI == 0, "tile rows per wave");
-  // A tile in flight in registers: this wave's rows 8w..8w+7 of K and V (chunk-swizzled as they
-  // will sit in LDS).
-  struct Slot { u32x4_t k[NL], v[NL]; uint32_t mw[RT]; };
-  const int win = max(kTileTokens, (kPageWin - 2) * kv.page_size / kTileTokens * kTileTokens);
-  for (int wt0 = kv_begin; wt0 < kv_end; wt0 += win) {
-    const int wt1 = min(kv_end, wt0 + win);
-    const int lp0 = (int)kv.pdiv.div((uint32_t)wt0);
-    const int npg = (int)kv.pdiv.div((uint32_t)(wt1 - 1)) - lp0 + 1;
-    const int ntiles = (wt1 - wt0 + kTileTokens - 1) / kTileTokens;
-    if (threadIdx.x == 0) window_bad = 0;
-    __syncthreads();  // the previous window's lookups and LDS tiles are done
-    for (int i = threadIdx.x; i < npg; i += NT) {
-      const int pg = kv.indices[page0 + lp0 + i];
-      ptab[i] = pg;
-      if ((unsigned)pg >= (unsigned)kv.num_pages) window_bad = 1;
-    }
-    __syncthreads();
-    const bool all_pages_ok = window_bad == 0;
-    auto gload = [&](Slot& sl, int tile) {
-      const int t0 = wt0 + tile * kTileTokens;
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const int r = WR * w + RPI * i + lane / CH;
-        bool ok;
-        const uint64_t off = kv_offset_lds(kv, ptab, lp0, min(t0 + r, wt1 - 1), kvh, ok);
-        sl.k[i] = ld16v(kv.k + off + 8 * ((lane % CH) ^ chunk_swizzle<D>(r)));
-        sl.v[i] = ld16v(kv.v + off + 8 * ((lane % CH) ^ v_swizzle<D>(r)));
-      }
-      if (mode == 2) {
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) sl.mw[rt] = mword[rt][t0 >> 5];
-      }
-    };
-    auto lwrite = [&](const Slot& sl, int tile) {
-      uint16_t* kd = kt + (tile & 1) * 2 * TILE;
-      if (mode == 2) {  // each lane keeps its own rows' mask words with the tile (no sharing)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) mwt[tile & 1][rt][threadIdx.x] = sl.mw[rt];
-      }
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        *reinterpret_cast<u32x4_t*>(kd + (WR * w + RPI * i) * D + 8 * lane) = sl.k[i];
-        *reinterpret_cast<u32x4_t*>(kd + TILE + (WR * w + RPI * i) * D + 8 * lane) = sl.v[i];
-      }
-    };
-    auto compute = [&](int tile) {
-      const int t0 = wt0 + tile * kTileTokens;
-      const uint16_t* kd = kt + (tile & 1) * 2 * TILE;
-      // tokens of this tile on valid pages (bit r = token t0 + r); tested only in windows that
-      // hold an out-of-range page id
-      uint64_t tv = 0xffffffffull;
-      if (!all_pages_ok) {
-        bool pok = false;
-        if (lane < kTileTokens && t0 + lane < wt1) kv_offset_lds(kv, ptab, lp0, t0 + lane, kvh, pok);
-        tv = __builtin_amdgcn_ballot_w64(pok);
-      }
-      const bool full = mode != 2 && all_pages_ok && t0 + kTileTokens - 1 <= wave_lim && t0 >= wave_lo;
-      u32x4_t ka[2][NS];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int r = 16 * u + n;
-        const int z = chunk_swizzle<D>(r);
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-          ka[u][s] = *reinterpret_cast<const u32x4_t*>(kd + r * D + 8 * ((4 * s + g) ^ z));
-      }
-      u32x4_t pa[RT];
-      float a[RT][4];
-      bool rs[RT];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        uint32_t vm = 0xFFu;
-        if (mode == 2) {
-          // bit 16u+4g+i of the row's word is token t0+16u+4g+i
-          const uint32_t mw = mwt[tile & 1][rt][threadIdx.x] & (uint32_t)tv;
-          vm = ((mw >> (4 * g)) & 15u) | (((mw >> (16 + 4 * g)) & 15u) << 4);
-          if (lim[rt] < 0) vm = 0;
-        } else if (!full) {
-          vm = 0;
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int r = 16 * u + 4 * g + i;
-              vm |= (uint32_t)(t0 + r <= lim[rt] && ((tv >> r) & 1ull)) << (4 * u + i);
-            }
-        }
-        if (t0 < wave_lo) {  // the tile crosses some row's window start
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (t0 + 16 * u + 4 * g + i < lo[rt]) vm &= ~(1u << (4 * u + i));
-        }
-        if (__builtin_amdgcn_ballot_w64(vm != 0xFFu) == 0) vm = 0xFFu;  // keep the fast path visible
-        float sc[2][4];
-        st[rt].scores(ka, vm, scale_log2, sc);
-        pa[rt] = st[rt].softmax(sc, lane, a[rt], rs[rt]);
-      }
-      // PV: the V operand of each 16-dim block comes straight from LDS (transpose reads)
-      const int j = (lane >> 2) & 3, qq = lane & 3;
-      const int r0 = 4 * g + j, r1 = r0 + 16;
-      const uint16_t* b0 = kd + TILE + r0 * D + 4 * (qq & 1);
-      const uint16_t* b1 = kd + TILE + r1 * D + 4 * (qq & 1);
-      const int z0 = v_swizzle<D>(r0), z1 = v_swizzle<D>(r1);
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int lc = 2 * nb + (qq >> 1);
-        const uint2 lo = lds_read_tr16(b0 + 8 * (lc ^ z0));
-        const uint2 hi = lds_read_tr16(b1 + 8 * (lc ^ z1));
-        const u32x4_t vb = {lo.x, lo.y, hi.x, hi.y};
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) st[rt].pv(pa[rt], vb, a[rt], rs[rt], nb);
-      }
-    };
-    // Two register slots alternate (no copies, which would force waits on loads in flight):
-    // tile k+3's loads are issued while tile k is computed and land in LDS two steps later.
-    Slot sa, sb;
-    gload(sa, 0);
-    if (ntiles > 1) gload(sb, 1);
-    lwrite(sa, 0);
-    if (ntiles > 2) gload(sa, 2);
-    __syncthreads();
-    for (int k = 0;;) {
-      compute(k);
-      if (k + 1 < ntiles) {
-        lwrite(sb, k + 1);
-        if (k + 3 < ntiles) gload(sb, k + 3);
-      }
-      __syncthreads();
-      if (++k >= ntiles) break;
-      compute(k);
-      if (k + 1 < ntiles) {
-        lwrite(sa, k + 1);
-        if (k + 3 < ntiles) gload(sa, k + 3);
-      }
-      __syncthreads();
-      if (++k >= ntiles) break;
-    }
-  }
-
-  // normalise and stage the bf16 rows in LDS ([kPrefillRows][D]), then write 16-byte chunks
-  float inv[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    float L = st[rt].row_sum(lane);
-    const int R = row0 + 16 * RT * w + 16 * rt + n;
-    if (sinks && R < rows) L += sink_mass(sinks, kvh * G + R % G, st[rt].m);
-    inv[rt] = L > 0.f ? 1.f / L : 0.f;
-  }
-  __syncthreads();
-  uint16_t* ot = reinterpret_cast<uint16_t*>(smem);
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float f = lane_read(inv[rt], 4 * g + i);
-      const int row = 16 * RT * w + 16 * rt + 4 * g + i;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) ot[row * D + 16 * nb + n] = to_bf1(st[rt].o[nb][i] * f);
-    }
-  __syncthreads();
-  for (int u = threadIdx.x; u < kPrefillRows * CH; u += NT) {
-    const int row = u / CH, c = u % CH;
-    const int R = row0 + row;
-    if (R >= rows) continue;
-    const int i = R / G, hg = R - i * G;
-    st16(out + (int64_t)(q0 + i) * o_ts + (int64_t)(kvh * G + hg) * o_hs + 8 * c,
-         *reinterpret_cast<const uint4*>(ot + row * D + 8 * c));
-  }
-}
-
-
-// ------------------------------------------------------------------------------ prefill, D = 128
-// The same work items, visibility rules, K/V tile pipeline and masks as attn_prefill_kernel, with
-// the products on v_mfma_f32_32x32x16_bf16 and the output computed transposed:
-//   S^T = K Q^T    A = 32 kv tokens x 16 dims (lane (t, kg): token t's dims 8(2s+kg)..+8 at
-//                  step s, from LDS), B = 32 query rows (lane (r, kg): row r, the same dims)
-//   O^T = V^T P^T  A = 32 dims x 16 tokens (two transpose reads of 4 V rows each),
-//                  B = P^T: lane (r, kg) holds row r's probabilities of tokens
-//                  16j + 8(e/4) + 4kg + e%4, exactly 8 consecutive registers of S^T's C layout
-// so every lane owns one query row r = lane % 32 in both products: its running max, sum and
-// rescale factor are its own (one exchange with lane ^ 32 for the max), and no factor has to be
-// broadcast to other lanes. Each wave owns 32 rows; a work group of 4 waves, 128 rows.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ f32x16_t mfma_32x32x16(const u32x4_t& a, const u32x4_t& b, f32x16_t c) {
@@ -987,10 +729,416 @@ __device__ __forceinline__ f32x16_t mfma_32x32x16(const u32x4_t& a, const u32x4_
 #define sched_group(mask, n) __builtin_amdgcn_sched_group_barrier((mask), (n), 0)
 
 // V-row swizzle for this kernel's transpose reads: one read takes 4 consecutive rows x 4 chunks
-// per half-wave, so rows r..r+3 XOR chunk bits 2-3 with r mod 4.
-__device__ __forceinline__ int v32_swizzle(int r) { return (r & 3) << 2; }
+// (64 bytes) per half-wave, and the 4 rows must fall on different 64-byte bank groups: rows of
+// 256 bytes or more XOR chunk bits 2-3 with r mod 4, rows of 128 bytes chunk bit 2 with bit 1 of r.
+template <int D>
+__device__ __forceinline__ int v32_swizzle(int r) { return D == 64 ? ((r >> 1) & 1) << 2 : (r & 3) << 2; }
 
+// v of lane ^ 32
+__device__ __forceinline__ float other_half(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  return __builtin_bit_cast(float, (threadIdx.x & 32) ? r[0] : r[1]);
+}
 
+// Partial results of a split item (piece slot s, kv head h): 128 rows of D fp32 outputs
+// (normalised) at part_o + (s * n_kv_heads + h) * 128 * D and their log2-sum-exps at
+// part_lse + (s * n_kv_heads + h) * 128; attn_prefill_merge_kernel combines an item's pieces.
+template <int D>
+__global__ __launch_bounds__(256, prefill_groups<D>()) void attn_prefill_kernel(
+    const uint16_t* __restrict__ q, int64_t q_ts, int64_t q_hs, PagedKV kv,
+    const int32_t* __restrict__ qo_indptr, int G, float scale_log2, const int32_t* __restrict__ plan,
+    int items_word, int n_items, int n_kv_heads,
+    int mode_in, int window_left, const uint32_t* __restrict__ packed,
+    const int64_t* __restrict__ word_off, const int32_t* __restrict__ extent,
+    uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs, const float* __restrict__ sinks,
+    float* __restrict__ part_o, float* __restrict__ part_lse) {
+  constexpr int TT = prefill_tile<D>(), H2 = TT / 32;  // tile tokens, 32-token halves
+  constexpr int NS = D / 16;  // QK k-steps
+  constexpr int NB = D / 32;  // 32-dim output blocks
+  constexpr int CH = D / 8, RPI = 64 / CH;  // 16-byte chunks per row, rows per load instruction
+  constexpr int NT = 256;
+  constexpr int TILE = TT * D;
+  constexpr int WR = TT / 4;    // rows of each K / V tile one wave loads
+  constexpr int NL = WR / RPI;  // load instructions for them
+  static_assert(NL >= 1 && WR % RPI == 0, "tile rows per wave");
+  __shared__ __attribute__((aligned(16))) char smem[2 * 2 * TILE * 2];
+  __shared__ int32_t ptab[kPageWin];
+  __shared__ int window_bad;
+
+  if (plan[2] != plan_rows_word(D)) {
+    prefill_plan_mismatch<D>(plan, qo_indptr, G * n_kv_heads, out, o_ts, o_hs);
+    return;
+  }
+  const int u = prefill_unit(n_items * n_kv_heads);
+  if (u < 0) return;  // padding work group
+  const int kvh = u / n_items;
+  const int32_t* item = plan + items_word + kPlanItemWords * (u - kvh * n_items);
+  const int b = uniform(item[0]), row0 = uniform(item[1]), q0 = uniform(item[2]), qo_len = uniform(item[3]);
+  const int kv_len = uniform(item[4]), page0 = uniform(item[5]), piece = uniform(item[6]), slot = uniform(item[7]) - 1;
+  const int lane = threadIdx.x & 63, w = uniform(threadIdx.x >> 6);
+  const int r32 = lane & 31, kg = lane >> 5;
+  const int rows = qo_len * G;
+  int mode = mode_in, mext = 0;  // a custom mask that is causal for all the rows: the causal path
+  if (mode_in == 2) {
+    bool causal;
+    mask_rows_extent(extent, q0, row0, rows, G, kPrefillRows, mext, causal);
+    mode = uniform(causal ? 1 : 2);  // wave-uniform (a scalar register), like the argument
+    mext = uniform(mext);
+  }
+
+  // this lane's query row
+  const int R = row0 + 32 * w + r32;
+  const bool valid = R < rows;
+  const int row_tok = valid ? R / G : -1;
+  // the positions a row (its query token; -1: no row) sees: lo..lim (and the mask)
+  const auto row_lim = [&](int t) { return t < 0 ? -1 : mode == 1 ? kv_len - qo_len + t : kv_len - 1; };
+  const auto row_lo = [&](int t) { return window_left >= 0 ? kv_len - qo_len + t - window_left : 0; };
+  u32x4_t qb[NS];
+  {
+    const int tok = max(row_tok, 0), hg = valid ? R - tok * G : 0;
+    const uint16_t* qp = q + (int64_t)(q0 + tok) * q_ts + (int64_t)(kvh * G + hg) * q_hs;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const u32x4_t z = {0u, 0u, 0u, 0u};
+      qb[s] = valid ? ld16v(qp + 8 * (2 * s + kg)) : z;
+    }
+  }
+  f32x16_t o[NB];
+#pragma unroll
+  for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[bb][i] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+
+  // kv positions any row of this work group can see (mode 2: the furthest set mask bit of its
+  // rows' query tokens, from attn_mask_extent_kernel); a sliding window hides positions before
+  // its first row's window (tiles start 32-aligned so mask words line up)
+  const int last_row = min(rows, row0 + kPrefillRows) - 1;
+  int kv_end = mode == 1 ? min(kv_len, kv_len - qo_len + last_row / G + 1) : kv_len;
+  if (mode == 2) kv_end = min(kv_len, mext);
+  int kv_begin = window_left >= 0 ? max(0, kv_len - qo_len + row0 / G - window_left) & ~31 : 0;
+  if (slot >= 0) {
+    const int chunk = uniform(plan[kPlanChunkWord]);
+    kv_begin += piece * chunk;
+    kv_end = min(kv_end, kv_begin + chunk);
+  }
+  const int nw = (kv_len + 31) / 32;
+  const uint32_t* mword = mode == 2 ? packed + word_off[b] + (int64_t)max(row_tok, 0) * nw : nullptr;
+  // uniform bounds of the wave's rows: tiles inside [wave_lo, wave_lim] need no per-element test,
+  // tiles past wave_hi are seen by none of them
+  // (a row's limits grow with its token, so the wave's first and last rows give them)
+  const int wr0 = row0 + 32 * w, wr1 = min(wr0 + 31, rows - 1);
+  const bool wave_rows = wr0 < rows;
+  const int wtok0 = wave_rows ? wr0 / G : -1, wtok1 = wave_rows ? wr1 / G : -1;
+  const int wave_lim = wave_rows ? row_lim(wtok0) : 0x7fffffff, wave_hi = row_lim(wtok1);
+  const int wave_lo = wave_rows ? row_lo(wtok1) : 0;
+
+  uint16_t* kt = reinterpret_cast<uint16_t*>(smem);  // [2 buffers][K, V][TT][D]
+  // A tile in flight in registers: this wave's rows WR*w.. of K and V (chunk-swizzled as they will
+  // sit in LDS), and the mask words of this lane's row.
+  struct Slot { u32x4_t k[NL], v[NL]; uint32_t mw[H2]; };
+  // Pages of at least WR tokens (a multiple of it) hold the wave's rows of a tile together: one
+  // uniform page lookup and a scalar base address per tile. Load i's rows are RPI*i further on, a
+  // scalar too, and its lanes' chunks differ from load 0's by XORs of constants, with cache rows
+  // that are whole multiples of D elements apart.
+  const bool one_page = kv.page_size % WR == 0 && kv.slot_stride % D == 0 && kv.slot_stride < (1 << 26);
+  const auto k_xor = [](int i) { return (uint32_t)(D == 256 ? 32 * i : 64 * i); };  // bytes
+  const auto v_xor = [](int i) { return (uint32_t)(D == 256 ? 128 * (i & 1) : 0); };
+  uint32_t koff, voff;
+  {
+    const int rl = lane / CH, r = WR * w + rl;
+    koff = 2u * ((uint32_t)rl * (uint32_t)kv.slot_stride + 8u * ((lane % CH) ^ chunk_swizzle<D>(r)));
+    voff = 2u * ((uint32_t)rl * (uint32_t)kv.slot_stride + 8u * ((lane % CH) ^ v32_swizzle<D>(r)));
+  }
+  const uint32_t step = 2u * RPI * (uint32_t)kv.slot_stride;
+  // LDS byte offsets of this lane's operands in a tile: k step 0 of half 0 (step s: ^ 32s), and V
+  // block 0 of the first transpose read (block bb: ^ 64bb). Transpose-read source lanes: group
+  // G16 = lane / 16 reads rows 16j + 8h + 4kg + (lane%16)/4 (h: first or second 4 tokens), dims
+  // 32bb + 16(G16%2) + 4(lane%4)
+  uint32_t kl0, vl0;
+  {
+    kl0 = 2u * r32 * D + 16u * (kg ^ chunk_swizzle<D>(r32));
+    const int r = 4 * kg + ((lane >> 2) & 3), dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    vl0 = 2u * (TILE + r * D + 8 * ((dim >> 3) ^ v32_swizzle<D>(r)) + (dim & 7));
+  }
+  const int win = max(TT, (kPageWin - 2) * kv.page_size / TT * TT);
+  for (int wt0 = kv_begin; wt0 < kv_end; wt0 += win) {
+    const int wt1 = min(kv_end, wt0 + win);
+    const int lp0 = (int)kv.pdiv.div((uint32_t)wt0);
+    const int npg = (int)kv.pdiv.div((uint32_t)(wt1 - 1)) - lp0 + 1;
+    const int ntiles = (wt1 - wt0 + TT - 1) / TT;
+    if (threadIdx.x == 0) window_bad = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < npg; i += NT) {
+      const int pg = kv.indices[page0 + lp0 + i];
+      ptab[i] = pg;
+      if ((unsigned)pg >= (unsigned)kv.num_pages) window_bad = 1;
+    }
+    __syncthreads();
+    const bool all_pages_ok = uniform(window_bad) == 0;
+    // the wave's first token of a tile (in the last tile at most the last whole group of WR rows)
+    const auto wave_tok = [&](int tile) { return min(wt0 + tile * TT + WR * w, (wt1 - 1) & ~(WR - 1)); };
+    int next_page = one_page ? ptab[(int)kv.pdiv.div((uint32_t)wave_tok(0)) - lp0] : 0;
+    // Tiles are loaded in order, 0, 1, ...; the next tile's page id is read from LDS one tile ahead.
+    auto gload = [&](Slot& sl, int tile) {
+      const int t0 = wt0 + tile * TT;
+      if (one_page) {
+        const int tb = wave_tok(tile);
+        const int slot0 = tb - (int)kv.pdiv.div((uint32_t)tb) * kv.page_size;
+        const int page = uniform(next_page);
+        next_page = ptab[(int)kv.pdiv.div((uint32_t)wave_tok(tile + 1)) - lp0];
+        const uint32_t pg = (unsigned)page < (unsigned)kv.num_pages ? (uint32_t)page : 0u;
+        const int64_t base = (int64_t)pg * kv.page_stride + (int64_t)slot0 * kv.slot_stride + (int64_t)kvh * kv.head_stride;
+        const auto kb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kv.k + base), 0, 0x7fffffff, 0x00020000);
+        const auto vb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kv.v + base), 0, 0x7fffffff, 0x00020000);
+        const uint32_t ko = (uint32_t)opaque_v((int)koff);
+        uint32_t back[NL];
+#pragma unroll
+        for (int i = 0; i < NL; ++i) back[i] = 0;
+        if (t0 + TT > wt1) {  // the last tile: rows past the end read the last row (their probability is 0)
+#pragma unroll
+          for (int i = 0; i < NL; ++i)
+            back[i] = 2u * (uint32_t)max(0, RPI * i + lane / CH - (wt1 - 1 - tb)) * (uint32_t)kv.slot_stride;
+        }
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+          sl.k[i] = __builtin_amdgcn_raw_buffer_load_b128(kb, (int)((ko ^ k_xor(i)) + i * step - back[i]), 0, 0);
+          sl.v[i] = __builtin_amdgcn_raw_buffer_load_b128(vb, (int)((voff ^ v_xor(i)) + i * step - back[i]), 0, 0);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+          const int r = WR * w + RPI * i + lane / CH;
+          bool ok;
+          const uint64_t off = kv_offset_lds(kv, ptab, lp0, min(t0 + r, wt1 - 1), kvh, ok);
+          sl.k[i] = ld16v(kv.k + off + 8 * ((lane % CH) ^ chunk_swizzle<D>(r)));
+          sl.v[i] = ld16v(kv.v + off + 8 * ((lane % CH) ^ v32_swizzle<D>(r)));
+        }
+      }
+      if (mode == 2) {
+#pragma unroll
+        for (int h = 0; h < H2; ++h) sl.mw[h] = mword[min((t0 >> 5) + h, nw - 1)];
+      }
+    };
+    uint32_t mcur[H2];  // the mask words of the tile being computed
+#pragma unroll
+    for (int h = 0; h < H2; ++h) mcur[h] = 0;
+    auto lwrite = [&](const Slot& sl, int tile) {
+      uint16_t* kd = kt + (tile & 1) * 2 * TILE;
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        *reinterpret_cast<u32x4_t*>(kd + (WR * w + RPI * i) * D + 8 * lane) = sl.k[i];
+        *reinterpret_cast<u32x4_t*>(kd + TILE + (WR * w + RPI * i) * D + 8 * lane) = sl.v[i];
+      }
+      if (mode == 2) {
+#pragma unroll
+        for (int h = 0; h < H2; ++h) mcur[h] = sl.mw[h];
+      }
+    };
+    auto compute = [&](int tile) {
+      const int t0 = wt0 + tile * TT;
+      if (t0 > wave_hi) return;  // no row of the wave sees the tile
+      const uint32_t buf = (tile & 1) * 4 * TILE;  // bytes
+      const uint32_t kl = (uint32_t)opaque_v((int)(buf + kl0));
+      // S^T: token 32h + r32 of the tile against this lane group's 32 rows
+      f32x16_t sacc[H2];
+#pragma unroll
+      for (int h = 0; h < H2; ++h)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sacc[h][i] = 0.f;
+      {
+        // K operands read four ahead of the MFMAs. The schedule is pinned: left to itself the
+        // compiler reads two ahead and exposes the LDS latency several times per tile.
+        u32x4_t kr[NS][H2];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+          for (int h = 0; h < H2; ++h)
+            kr[s][h] = *reinterpret_cast<const u32x4_t*>(smem + ((kl ^ (32 * s)) + 64 * h * D));
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+          for (int h = 0; h < H2; ++h) sacc[h] = mfma_32x32x16(kr[s][h], qb[s], sacc[h]);
+        sched_group(0x100, 4);
+#pragma unroll
+        for (int s = 0; s < NS * H2 - 4; ++s) { sched_group(0x008, 1); sched_group(0x100, 1); }
+        sched_group(0x008, 4);
+      }
+      // V operands, read 16 tokens ahead of their MFMAs (the first ones here, over the softmax)
+      const uint32_t vl = (uint32_t)opaque_v((int)(buf + vl0));
+      u32x4_t va[2][NB];
+      const auto read_v = [&](int j) {
+#pragma unroll
+        for (int bb = 0; bb < NB; ++bb) {
+          uint2 hv[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            hv[h] = lds_read_tr16(reinterpret_cast<const uint16_t*>(smem + ((vl ^ (64 * bb)) + (32 * j + 16 * h) * D)));
+          va[j & 1][bb] = u32x4_t{hv[0].x, hv[0].y, hv[1].x, hv[1].y};
+        }
+      };
+      read_v(0);
+      // visibility of token tt(i) = 32h + 8(i/4) + 4kg + i%4 for this lane's row: mask bits by
+      // shifts, then the per-element bounds only in tiles that cross a row's limit or window start
+      uint32_t vis[H2];
+#pragma unroll
+      for (int h = 0; h < H2; ++h) vis[h] = 0xffffu;
+      if (mode == 2) {
+#pragma unroll
+        for (int h = 0; h < H2; ++h) {
+          vis[h] = 0;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) vis[h] |= ((mcur[h] >> (8 * c + 4 * kg)) & 15u) << (4 * c);
+        }
+      }
+      if (!all_pages_ok || t0 + TT - 1 > wave_lim || t0 < wave_lo) {
+        uint64_t tv = ~0ull;
+        if (!all_pages_ok) {
+          bool pok = false;
+          if (lane < TT && t0 + lane < wt1) kv_offset_lds(kv, ptab, lp0, t0 + lane, kvh, pok);
+          tv = __builtin_amdgcn_ballot_w64(pok);
+        }
+        // compared against the constants 32h + 8(i/4) + i%4, so that nothing per element stays live
+        const int hi = row_lim(row_tok) - t0 - 4 * kg, first = row_lo(row_tok) - t0 - 4 * kg;
+        tv >>= 4 * kg;
+#pragma unroll
+        for (int h = 0; h < H2; ++h)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int c = 32 * h + 8 * (i >> 2) + (i & 3);
+            if (!(c <= hi && c >= first && ((tv >> c) & 1ull))) vis[h] &= ~(1u << i);
+          }
+      }
+      // Scores stay raw (q.k) until the exponent, where one fma applies the scale: the row maximum
+      // is taken over raw scores, negated when the scale is negative (a uniform branch), with
+      // hidden entries set to the raw value that scales to -inf (the scale is never 0 here).
+      const bool neg = scale_log2 < 0.f;
+      bool seen_all = true;
+#pragma unroll
+      for (int h = 0; h < H2; ++h) seen_all = seen_all && vis[h] == 0xffffu;
+      if (__builtin_amdgcn_ballot_w64(!seen_all) != 0) {
+        const float hidden = neg ? INFINITY : -INFINITY;
+#pragma unroll
+        for (int h = 0; h < H2; ++h)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sacc[h][i] = ((vis[h] >> i) & 1u) ? sacc[h][i] : hidden;
+      }
+      float mx = -INFINITY;
+      if (!neg) {
+        float mh[4 * H2];
+#pragma unroll
+        for (int h = 0; h < H2; ++h)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            mh[4 * h + c] = fmaxf(fmaxf(sacc[h][4 * c], sacc[h][4 * c + 1]), fmaxf(sacc[h][4 * c + 2], sacc[h][4 * c + 3]));
+#pragma unroll
+        for (int c = 0; c < 4 * H2; ++c) mx = fmaxf(mx, mh[c]);
+      } else {
+#pragma unroll
+        for (int h = 0; h < H2; ++h)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) mx = fmaxf(mx, -sacc[h][i]);
+      }
+      mx = fmaxf(mx, other_half(mx)) * fabsf(scale_log2);
+      // lazy maximum (kLazyMax)
+      if (__builtin_amdgcn_ballot_w64(mx > m_run + kLazyMax) != 0) {
+        const bool grow = mx > m_run + kLazyMax;
+        const float alpha = grow ? fast_exp2(m_run - mx) : 1.f;
+        if (grow) m_run = mx;
+        l_run *= alpha;
+#pragma unroll
+        for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[bb][i] *= alpha;
+      }
+      const float m_use = m_run == -INFINITY ? 0.f : m_run;
+      // O^T += V^T P^T, 16 tokens at a time. Step j's MFMAs, the next step's V reads and its
+      // exponentials are independent, and pinned together: the reads first, then an equal share of
+      // the exponentials behind each MFMA. Left to itself the compiler reads each V operand right
+      // before its MFMA and waits for it there.
+      float ps[2 * H2];
+      u32x4_t pb[2];
+      const auto probs = [&](int j) {
+        float sc[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sc[i] = fast_exp2(fmaf(sacc[j >> 1][8 * (j & 1) + i], scale_log2, -m_use));
+        // the row's partial sum as a tree (a chain of dependent adds sat on the critical path)
+        ps[j] = ((sc[0] + sc[1]) + (sc[2] + sc[3])) + ((sc[4] + sc[5]) + (sc[6] + sc[7]));
+        pb[j & 1] = u32x4_t{pack_bf2(sc[0], sc[1]), pack_bf2(sc[2], sc[3]), pack_bf2(sc[4], sc[5]), pack_bf2(sc[6], sc[7])};
+      };
+      probs(0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 2 * H2; ++j) {
+        const bool more = j + 1 < 2 * H2;
+        if (more) { read_v(j + 1); probs(j + 1); }
+#pragma unroll
+        for (int bb = 0; bb < NB; ++bb) o[bb] = mfma_32x32x16(va[j & 1][bb], pb[j & 1], o[bb]);
+        if (more) sched_group(0x100, 2 * NB);
+#pragma unroll
+        for (int bb = 0; bb < NB; ++bb) {
+          sched_group(0x008, 1);
+          
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (H2 == 2) l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);
+      else l_run += ps[0] + ps[1];
+    };
+    Slot sl;
+    gload(sl, 0);
+    lwrite(sl, 0);
+    if (ntiles > 1) gload(sl, 1);
+    __syncthreads();
+    for (int k = 0;;) {
+      compute(k);
+      if (k + 1 < ntiles) {
+        lwrite(sl, k + 1);
+        if (k + 2 < ntiles) gload(sl, k + 2);
+      }
+      __syncthreads();
+      if (++k >= ntiles) break;
+    }
+  }
+  // normalise and write: o[bb][i] is dim 32bb + 8(i/4) + 4kg + i%4 of row R; lanes r and r^32
+  // together cover 8 consecutive dims
+  float L = l_run + other_half(l_run);
+  // the row again, so that nothing of it is kept over the loop
+  const int le = opaque_v((int)(threadIdx.x & 63)), re = 32 * w + (le & 31), Re = row0 + re, ge = le >> 5;
+  if (slot >= 0) {
+    if (Re < rows) {
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      const int64_t pr = ((int64_t)slot * n_kv_heads + kvh) * kPrefillRows + re;
+      float* op = part_o + pr * D;
+#pragma unroll
+      for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          *reinterpret_cast<float4*>(op + 32 * bb + 8 * c + 4 * ge) =
+              make_float4(o[bb][4 * c] * inv, o[bb][4 * c + 1] * inv, o[bb][4 * c + 2] * inv, o[bb][4 * c + 3] * inv);
+      if (ge == 0) part_lse[pr] = L > 0.f ? m_run + log2f(L) : -INFINITY;
+    }
+  } else if (Re < rows) {
+    const int tok = Re / G, hg = Re - tok * G;
+    L += sink_mass(sinks, kvh * G + hg, m_run);
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    uint16_t* op = out + (int64_t)(q0 + tok) * o_ts + (int64_t)(kvh * G + hg) * o_hs;
+#pragma unroll
+    for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint2 v = {pack_bf2(o[bb][4 * c] * inv, o[bb][4 * c + 1] * inv),
+                         pack_bf2(o[bb][4 * c + 2] * inv, o[bb][4 * c + 3] * inv)};
+        *reinterpret_cast<uint2*>(op + 32 * bb + 8 * c + 4 * ge) = v;
+      }
+  }
+}
+
+// Head dim 128 with more units than the chip runs at once: the same products and work items in
+// 32-token tiles with two tiles in flight in registers, on persistent work groups.
+// Long prompts run alike on either kernel (8 x 8192 tokens: 4.76 ms here, 4.68 in
+// attn_prefill_kernel); short ones, where a tile's overhang past the causal limit counts, are
+// faster here (64 x U[1, 2048]: 963 against 980 us; 128 x 512: 623 against 659 us).
 template <int D>
 __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(
     const uint16_t* __restrict__ q, int64_t q_ts, int64_t q_hs, PagedKV kv,
@@ -1014,7 +1162,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(
   // queue is empty. XCD x's queue is the contiguous run [x * per, (x + 1) * per) of the units, in
   // plan order (each request's items together), so the work groups of one XCD share the K/V
   // prefix they read through its L2; a work group whose queue is empty takes from the others.
-  if (plan[2] != kRows) {
+  if (plan[2] != plan_rows_word(D)) {
     prefill_plan_mismatch<D>(plan, qo_indptr, G * n_kv_heads, out, o_ts, o_hs);
     return;
   }
@@ -1117,7 +1265,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(
         bool ok;
         const uint64_t off = kv_offset_lds(kv, ptab, lp0, min(t0 + r, wt1 - 1), kvh, ok);
         sl.k[i] = ld16v(kv.k + off + 8 * ((lane % CH) ^ chunk_swizzle<D>(r)));
-        sl.v[i] = ld16v(kv.v + off + 8 * ((lane % CH) ^ v32_swizzle(r)));
+        sl.v[i] = ld16v(kv.v + off + 8 * ((lane % CH) ^ v32_swizzle<D>(r)));
       }
       if (mode == 2) sl.mw = mword[t0 >> 5];
     };
@@ -1230,7 +1378,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(
           for (int h = 0; h < 2; ++h) {
             const int r = 16 * j + 8 * h + 4 * kg + jj;
             const int dim = 32 * bb + 16 * (g16 & 1) + 4 * qq;
-            const int c = (dim >> 3) ^ v32_swizzle(r);
+            const int c = (dim >> 3) ^ v32_swizzle<D>(r);
             hv[h] = lds_read_tr16(vbase + r * D + 8 * c + (dim & 7));
           }
           const u32x4_t va = {hv[0].x, hv[0].y, hv[1].x, hv[1].y};
@@ -1284,6 +1432,34 @@ __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(
     for (int x = 0; x < 8; ++x) atomicExch(&counters[kPlanQueueWord + x], 0);
     atomicExch(&counters[kPlanDoneWord], 0);
   }
+}
+
+// Combines the pieces of split items: work group x takes (merge entry, kv head) x and 512 / D of
+// its 128 rows.
+template <int D>
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
+    const int32_t* __restrict__ merges, int n_kv_heads, int G, const float* __restrict__ part_o,
+    const float* __restrict__ part_lse, uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs,
+    const float* __restrict__ sinks) {
+  constexpr int CH = D / 8;
+  const int e = blockIdx.x / n_kv_heads, kvh = blockIdx.x - e * n_kv_heads;
+  const int32_t* m = merges + kPlanMergeWords * e;
+  const int row0 = m[0], q0 = m[1], rows = m[2] * G, slot = m[3], pieces = m[4];
+  const int lane = threadIdx.x & 63, c = lane % CH;
+  const int rl0 = blockIdx.y * (64 / CH);
+  if (row0 + rl0 >= rows) return;
+  const int R = min(row0 + rl0 + lane / CH, rows - 1);  // lanes past the last row repeat it
+  const int64_t first = ((int64_t)slot * n_kv_heads + kvh) * kPrefillRows + (R - row0);
+  const int64_t step = (int64_t)n_kv_heads * kPrefillRows;
+  float acc[8], L, M;
+  merge_partials<D>(part_o + first * D + 8 * c, step * D, part_lse + first, step, pieces, acc, L, M);
+  if (threadIdx.x >= 64 || row0 + rl0 + lane / CH >= rows) return;
+  const int tok = R / G, hq = kvh * G + (R - tok * G);
+  if (M != -INFINITY) L += sink_mass(sinks, hq, M);
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[i] *= inv;
+  st16(out + (int64_t)(q0 + tok) * o_ts + (int64_t)hq * o_hs + 8 * c, pack8(acc));
 }
 
 }  // namespace pie
@@ -1473,17 +1649,28 @@ extern "C" int pie_hip_attention_decode_noalloc(
 }
 
 // Host: the prefill work list. Reads host copies of qo_indptr, kv_indptr and kv_last_page_len
-// (as flashinfer's plan does); lists (request, first row) items of prefill_rows<D> packed rows,
+// (as flashinfer's plan does); lists (request, first row) items of kPrefillRows packed rows,
 // those that see the most kv positions first, and for mode 2 the byte offset of every
-// request's [qo_len, kv_len] mask block (int64, 8-byte aligned in the plan).
-extern "C" int pie_hip_attention_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
-                                              const int32_t* kv_last_page_len, int64_t batch,
-                                              int64_t page_size, int64_t num_qo_heads,
-                                              int64_t num_kv_heads, int64_t head_dim, int32_t mode,
-                                              int32_t* plan,
-                                              int64_t plan_capacity, int64_t* plan_words,
-                                              int64_t* num_items, int64_t* mask_bytes,
-                                              int64_t* mask_words) {
+// request's [qo_len, kv_len] mask block (int64, 8-byte aligned in the plan). With `split`, a second
+// list after them cuts the items that would outlast the rest of the launch over their kv range.
+struct PrefillSplit {
+  int64_t window_left, num_cus, workspace_bytes;
+  int64_t items_word = 0, num_items = 0, merges_word = 0, num_merges = 0, scratch_bytes = 0;
+};
+
+// The rule of the split list. Without it a request's rows walk its whole context in one work group:
+// 13 drafted tokens each over 4 contexts of 1-9k tokens took 253 us on 32 work groups and take 32 us
+// in 256-to-320-token pieces; one 700-token prompt 100 us, and 30 us. A launch fills num_cus * groups work groups; their mean share of the
+// kv tokens (over all items and kv heads) is the length a piece aims at, at least kSplitMinChunk,
+// below which a piece is mostly set-up. Items are cut only when the longest exceeds its pieces by
+// kSplitMinGain tokens: less than that the merge launch costs more than the cut saves.
+constexpr int64_t kSplitMinChunk = 256, kSplitMinGain = 512;
+
+static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_last_page_len,
+                             int64_t batch, int64_t page_size, int64_t num_qo_heads, int64_t num_kv_heads,
+                             int64_t head_dim, int32_t mode, int32_t* plan, int64_t plan_capacity,
+                             int64_t* plan_words, int64_t* num_items, int64_t* mask_bytes, int64_t* mask_words,
+                             PrefillSplit* split) {
   PIE_REQUIRE(qo_indptr && kv_indptr && kv_last_page_len && plan && plan_words && num_items && mask_bytes &&
                   mask_words,
               "prefill_plan: null argument");
@@ -1495,8 +1682,7 @@ extern "C" int pie_hip_attention_prefill_plan(const int32_t* qo_indptr, const in
   PIE_REQUIRE(head_dim == 64 || head_dim == 128 || head_dim == 256,
               "prefill_plan: head_dim %lld not in {64, 128, 256}", (long long)head_dim);
   const int64_t G = num_qo_heads / num_kv_heads;
-  const int64_t kPrefillRows = head_dim == 256 ? prefill_rows<256>() : prefill_rows<128>();
-  struct Item { int32_t b, row0, q0, qo, kv, page0; int64_t work, req_work; };
+  struct Item { int32_t b, row0, q0, qo, kv, page0; int64_t work, req_work, span; };
   std::vector<Item> items;
   std::vector<int64_t> moff((size_t)batch + 1, 0), woff((size_t)batch + 1, 0);
   int64_t mtotal = 0, wtotal = 0;
@@ -1514,8 +1700,11 @@ extern "C" int pie_hip_attention_prefill_plan(const int32_t* qo_indptr, const in
     for (int64_t r0 = 0; r0 < qo * G; r0 += kPrefillRows) {
       const int64_t last = std::min(qo * G, r0 + kPrefillRows) - 1;
       const int64_t seen = mode == 1 ? std::max<int64_t>(0, std::min(kv, kv - qo + last / G + 1)) : kv;
+      // the kernel's kv range: from the first row's window start, 32-aligned
+      const int64_t wl = split ? split->window_left : -1;
+      const int64_t begin = wl >= 0 ? std::max<int64_t>(0, kv - qo + r0 / G - wl) / 32 * 32 : 0;
       items.push_back(Item{(int32_t)b, (int32_t)r0, qo_indptr[b], (int32_t)qo, (int32_t)kv, kv_indptr[b],
-                           seen, kv * qo});
+                           seen, kv * qo, std::max<int64_t>(0, seen - begin)});
     }
   }
   // Each request's items stay together (they share its K/V prefix, which the kernels' XCD-aware
@@ -1532,49 +1721,152 @@ extern "C" int pie_hip_attention_prefill_plan(const int32_t* qo_indptr, const in
   woff[(size_t)batch] = wtotal;
   const int64_t moff_word = words, woff_word = words + 2 * (batch + 1);
   if (mode == 2) words += 4 * (batch + 1);
-  *plan_words = words;
   *num_items = (int64_t)items.size();
   *mask_bytes = mtotal;
   *mask_words = wtotal;
+  int64_t chunk = 0;
+  if (split && !items.empty()) {
+    int64_t total = 0, longest = 0;
+    for (const Item& it : items) {
+      total += it.span;
+      longest = std::max(longest, it.span);
+    }
+    const int64_t groups = (head_dim == 256 ? prefill_groups<256>() : prefill_groups<128>()) *
+                           (split->num_cus > 0 ? split->num_cus : 256);
+    chunk = std::max(kSplitMinChunk, (total * num_kv_heads + groups - 1) / groups);
+    chunk = (chunk + 63) / 64 * 64;
+    for (; longest >= chunk + kSplitMinGain; chunk *= 2) {  // longer pieces where the scratch is short
+      int64_t pieces = 0, cut = 0, whole = 0;
+      for (const Item& it : items) {
+        const int64_t n = (it.span + chunk - 1) / chunk;
+        if (n > 1) { pieces += n; ++cut; } else ++whole;
+      }
+      const int64_t all = words + kPlanItemWords * (pieces + whole) + kPlanMergeWords * cut;
+      const int64_t scratch = pieces * num_kv_heads * kPrefillRows * (head_dim + 1) * 4;
+      const int64_t masks = mode == 2 ? (wtotal * 4 + 15) / 16 * 16 + qo_indptr[batch] * 4ll : 0;
+      if (all <= plan_capacity && (all * 4 + 15) / 16 * 16 + (masks + 15) / 16 * 16 + scratch <= split->workspace_bytes &&
+          (pieces + whole) * num_kv_heads < (1ll << 31)) {
+        split->items_word = words;
+        split->num_items = pieces + whole;
+        split->merges_word = words + kPlanItemWords * (pieces + whole);
+        split->num_merges = cut;
+        split->scratch_bytes = scratch;
+        words = all;
+        break;
+      }
+    }
+  }
+  *plan_words = words;
   PIE_REQUIRE(words <= plan_capacity, "prefill_plan: needs %lld words, capacity %lld",
               (long long)words, (long long)plan_capacity);
   for (int i = 0; i < kPlanHeader; ++i) plan[i] = 0;
   plan[0] = (int32_t)items.size();
   plan[1] = (int32_t)batch;
-  plan[2] = (int32_t)kPrefillRows;
+  plan[2] = plan_rows_word(head_dim);
   plan[3] = (int32_t)moff_word;  // mode 2: int64 byte offsets of the mask blocks [batch + 1]
   plan[4] = (int32_t)woff_word;  // mode 2: int64 offsets of the packed mask words [batch + 1]
+  plan[kPlanChunkWord] = split && split->num_items ? (int32_t)chunk : 0;
   // [7] and [8, 16): the persistent kernel's work counters (zero between launches)
+  const auto put = [](int32_t* p, const Item& it, int32_t piece, int32_t slot1) {
+    const int32_t w8[kPlanItemWords] = {it.b, it.row0, it.q0, it.qo, it.kv, it.page0, piece, slot1};
+    memcpy(p, w8, sizeof(w8));
+  };
   int32_t* p = plan + kPlanHeader;
-  for (const Item& it : items) {
-    const int32_t w8[kPlanItemWords] = {it.b, it.row0, it.q0, it.qo, it.kv, it.page0, 0, 0};
-    for (int i = 0; i < kPlanItemWords; ++i) *p++ = w8[i];
-  }
+  for (const Item& it : items) { put(p, it, 0, 0); p += kPlanItemWords; }
   if (mode == 2) {
     memcpy(plan + moff_word, moff.data(), sizeof(int64_t) * (size_t)(batch + 1));
     memcpy(plan + woff_word, woff.data(), sizeof(int64_t) * (size_t)(batch + 1));
   }
+  if (split && split->num_items) {
+    int32_t slot = 0;
+    int32_t* m = plan + split->merges_word;
+    p = plan + split->items_word;
+    for (const Item& it : items) {
+      const int32_t n = (int32_t)((it.span + chunk - 1) / chunk);
+      if (n <= 1) { put(p, it, 0, 0); p += kPlanItemWords; continue; }
+      const int32_t w8[kPlanMergeWords] = {it.row0, it.q0, it.qo, slot, n, 0, 0, 0};
+      memcpy(m, w8, sizeof(w8));
+      m += kPlanMergeWords;
+      for (int32_t i = 0; i < n; ++i) { put(p, it, i, ++slot); p += kPlanItemWords; }
+    }
+  }
   return PIE_HIP_OK;
 }
 
+extern "C" int pie_hip_attention_prefill_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
+                                              const int32_t* kv_last_page_len, int64_t batch,
+                                              int64_t page_size, int64_t num_qo_heads,
+                                              int64_t num_kv_heads, int64_t head_dim, int32_t mode,
+                                              int32_t* plan,
+                                              int64_t plan_capacity, int64_t* plan_words,
+                                              int64_t* num_items, int64_t* mask_bytes,
+                                              int64_t* mask_words) {
+  return prefill_plan_impl(qo_indptr, kv_indptr, kv_last_page_len, batch, page_size, num_qo_heads, num_kv_heads,
+                           head_dim, mode, plan, plan_capacity, plan_words, num_items, mask_bytes, mask_words,
+                           nullptr);
+}
+
+extern "C" int pie_hip_attention_prefill_split_plan(
+    const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_last_page_len, int64_t batch,
+    int64_t page_size, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int32_t mode,
+    int64_t window_left, int64_t num_cus, int64_t workspace_bytes, int32_t* plan, int64_t plan_capacity,
+    int64_t* plan_words, int64_t* num_items, int64_t* mask_bytes, int64_t* mask_words, int64_t* split) {
+  PIE_REQUIRE(split, "prefill_split_plan: null argument");
+  PrefillSplit sp{window_left, num_cus, workspace_bytes};
+  const int rc = prefill_plan_impl(qo_indptr, kv_indptr, kv_last_page_len, batch, page_size, num_qo_heads,
+                                   num_kv_heads, head_dim, mode, plan, plan_capacity, plan_words, num_items,
+                                   mask_bytes, mask_words, &sp);
+  if (rc) return rc;
+  split[0] = sp.items_word;
+  split[1] = sp.num_items;
+  split[2] = sp.merges_word;
+  split[3] = sp.num_merges;
+  split[4] = sp.scratch_bytes;
+  return PIE_HIP_OK;
+}
+
+struct PrefillLaunch {
+  hipStream_t st;
+  const uint16_t* q;
+  int64_t q_ts, q_hs;
+  PagedKV kv;
+  const int32_t* qo_indptr;
+  int G, Hkv;
+  float sl2;
+  const int32_t* plan;
+  int items_word, n_items, mode, window_left;
+  const uint32_t* packed;
+  const int64_t* woff;
+  const int32_t* extent;
+  uint16_t* out;
+  int64_t o_ts, o_hs;
+  const float* sinks;
+  int merges_word, n_merges;
+  float *part_o, *part_lse;
+};
+
 template <int D>
-static void launch_prefill(hipStream_t st, dim3 grid, const uint16_t* q, int64_t q_ts, int64_t q_hs,
-                           const PagedKV& kv, const int32_t* qo_indptr, int G, float sl2,
-                           const int32_t* plan, int mode, int window_left, const uint32_t* packed,
-                           const int64_t* woff, const int32_t* extent, uint16_t* out, int64_t o_ts,
-                           int64_t o_hs, const float* sinks) {
-  // attn_prefill32_kernel scales raw scores inside the exponent, where a zero scale would turn a
-  // hidden (-inf) score into NaN; 1e-30 gives the same result (every exponent rounds to 2^0).
-  const dim3 xgrid(8 * ((grid.x * grid.y + 7) / 8));  // (kv head, item) units, padded to 8 XCDs
-  if constexpr (D == 128)
-    hipLaunchKernelGGL(attn_prefill32_kernel<128>, dim3(8 * ((2 * num_cus() + 7) / 8)), dim3(256), 0, st, q, q_ts,
-                       q_hs, kv, qo_indptr, G,
-                       sl2 == 0.f ? 1e-30f : sl2, plan, (int)grid.x, (int)grid.y, mode, window_left, packed,
-                       woff, extent, out, o_ts, o_hs, sinks);
-  else
-    hipLaunchKernelGGL(attn_prefill_kernel<D>, xgrid, dim3(64 * prefill_waves<D>()), 0, st, q, q_ts, q_hs, kv,
-                       qo_indptr, G, sl2, plan, (int)grid.x, (int)grid.y, mode, window_left, packed, woff,
-                       extent, out, o_ts, o_hs, sinks);
+static void launch_prefill(const PrefillLaunch& a) {
+  // the kernel scales raw scores inside the exponent, where a zero scale would turn a hidden
+  // (-inf) score into NaN; 1e-30 gives the same result (every exponent rounds to 2^0)
+  const float sl2 = a.sl2 == 0.f ? 1e-30f : a.sl2;
+  const int64_t units = (int64_t)a.n_items * a.Hkv;
+  if constexpr (D == 128) {
+    const int fit = 8 * ((prefill_groups<D>() * num_cus() + 7) / 8);  // work groups the chip runs at once
+    if (!a.n_merges && units > fit) {
+      hipLaunchKernelGGL(attn_prefill32_kernel<D>, dim3(fit), dim3(256), 0, a.st, a.q, a.q_ts, a.q_hs, a.kv,
+                         a.qo_indptr, a.G, sl2, a.plan, a.n_items, a.Hkv, a.mode, a.window_left, a.packed, a.woff,
+                         a.extent, a.out, a.o_ts, a.o_hs, a.sinks);
+      return;
+    }
+  }
+  const unsigned grid = (unsigned)(8 * ((units + 7) / 8));  // one work group per unit, padded to 8 XCDs
+  hipLaunchKernelGGL(attn_prefill_kernel<D>, dim3(grid), dim3(256), 0, a.st, a.q, a.q_ts, a.q_hs, a.kv, a.qo_indptr,
+                     a.G, sl2, a.plan, a.items_word, a.n_items, a.Hkv, a.mode, a.window_left, a.packed, a.woff,
+                     a.extent, a.out, a.o_ts, a.o_hs, a.sinks, a.part_o, a.part_lse);
+  if (a.n_merges)
+    hipLaunchKernelGGL(attn_prefill_merge_kernel<D>, dim3(a.n_merges * a.Hkv, kPrefillRows / (512 / D)), dim3(256), 0,
+                       a.st, a.plan + a.merges_word, a.Hkv, a.G, a.part_o, a.part_lse, a.out, a.o_ts, a.o_hs, a.sinks);
 }
 
 // Visible extent of every query token under the packed mask: 1 + the last kv position whose bit
@@ -1637,14 +1929,14 @@ __global__ __launch_bounds__(256) void attn_pack_mask_kernel(const uint8_t* __re
   packed[gw] = bits;
 }
 
-extern "C" int pie_hip_attention_prefill(
+static int attention_prefill_impl(
     const pie_bf16* q, int64_t q_tok_stride, int64_t q_head_stride, const pie_bf16* k_cache,
     const pie_bf16* v_cache, int64_t page_stride, int64_t slot_stride, int64_t head_stride,
     int64_t num_pages, const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_indices,
     const int32_t* kv_last_page_len, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim,
     int64_t page_size, float sm_scale, int32_t mode, int64_t window_left, const float* sinks,
     const uint32_t* packed_mask, const int32_t* mask_extent, const int32_t* plan, int64_t num_items,
-    int64_t mask_offsets_word, pie_bf16* out,
+    int64_t mask_offsets_word, const int64_t* split, void* scratch, int64_t scratch_bytes, pie_bf16* out,
     int64_t o_tok_stride, int64_t o_head_stride, void* stream) {
   PagedKV kv;
   int rc = paged_kv_desc(&kv, k_cache, v_cache, page_stride, slot_stride, head_stride, num_pages,
@@ -1664,27 +1956,86 @@ extern "C" int pie_hip_attention_prefill(
   PIE_REQUIRE(aligned16(q) && aligned16(out) && q_tok_stride % 8 == 0 && q_head_stride % 8 == 0 &&
                   o_tok_stride % 8 == 0 && o_head_stride % 8 == 0,
               "attention_prefill: q/out pointers and strides must be 16-byte aligned");
+  bool cut = split && split[1] > 0;
+  if (cut)
+    PIE_REQUIRE(split[0] > 0 && split[2] > split[0] && split[3] > 0 && split[1] * num_kv_heads < (1ll << 31) &&
+                    scratch && aligned16(scratch) && split[4] > 0 && scratch_bytes >= split[4],
+                "attention_prefill: a split plan needs %lld bytes of 16-byte-aligned scratch, got %lld",
+                (long long)split[4], (long long)scratch_bytes);
   if (num_items == 0) return PIE_HIP_OK;
-  const int G = (int)(num_qo_heads / num_kv_heads);
-  const float sl2 = sm_scale * 1.4426950408889634f;
-  const int64_t* woff = mode == 2 ? reinterpret_cast<const int64_t*>(plan + mask_offsets_word) : nullptr;
-  const int Wl = window_left < 0 ? -1 : (int)std::min<int64_t>(window_left, 1 << 30);
-  const dim3 grid((unsigned)num_items, (unsigned)num_kv_heads);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  // the head-dim-128 kernel counts its work in the plan's header words
+  // The head-dim-128 kernel counts its work in the plan's header words, so runs of one plan must not
+  // overlap. The other head dims' runs may: one that overlaps another stream's (or is captured,
+  // when that cannot be seen) leaves the scratch alone and runs the plan's uncut items.
   const bool counters = head_dim == 128;
-  if (counters && (rc = inflight_check(plan, stream, "attention_prefill")) != PIE_HIP_OK) return rc;
+  if (counters) {
+    if ((rc = inflight_check(plan, stream, "attention_prefill")) != PIE_HIP_OK) return rc;
+  } else if (cut) {
+    cut = inflight_free(plan, stream);
+  }
+  PrefillLaunch a{};
+  a.st = static_cast<hipStream_t>(stream);
+  a.q = q; a.q_ts = q_tok_stride; a.q_hs = q_head_stride;
+  a.kv = kv;
+  a.qo_indptr = qo_indptr;
+  a.G = (int)(num_qo_heads / num_kv_heads); a.Hkv = (int)num_kv_heads;
+  a.sl2 = sm_scale * 1.4426950408889634f;
+  a.plan = plan;
+  a.items_word = cut ? (int)split[0] : kPlanHeader;
+  a.n_items = (int)(cut ? split[1] : num_items);
+  a.mode = mode;
+  a.window_left = window_left < 0 ? -1 : (int)std::min<int64_t>(window_left, 1 << 30);
+  a.packed = packed_mask;
+  a.woff = mode == 2 ? reinterpret_cast<const int64_t*>(plan + mask_offsets_word) : nullptr;
+  a.extent = mask_extent;
+  a.out = out; a.o_ts = o_tok_stride; a.o_hs = o_head_stride;
+  a.sinks = sinks;
+  if (cut) {
+    a.merges_word = (int)split[2];
+    a.n_merges = (int)split[3];
+    a.part_o = static_cast<float*>(scratch);
+    a.part_lse = a.part_o + split[4] / 4 / (head_dim + 1) * head_dim;
+  }
   switch (head_dim) {
-    case 64: launch_prefill<64>(st, grid, q, q_tok_stride, q_head_stride, kv, qo_indptr, G, sl2, plan,
-                                mode, Wl, packed_mask, woff, mask_extent, out, o_tok_stride, o_head_stride, sinks); break;
-    case 128: launch_prefill<128>(st, grid, q, q_tok_stride, q_head_stride, kv, qo_indptr, G, sl2, plan,
-                                  mode, Wl, packed_mask, woff, mask_extent, out, o_tok_stride, o_head_stride, sinks); break;
-    default: launch_prefill<256>(st, grid, q, q_tok_stride, q_head_stride, kv, qo_indptr, G, sl2, plan,
-                                 mode, Wl, packed_mask, woff, mask_extent, out, o_tok_stride, o_head_stride, sinks); break;
+    case 64: launch_prefill<64>(a); break;
+    case 128: launch_prefill<128>(a); break;
+    default: launch_prefill<256>(a); break;
   }
   rc = check_launch("attention_prefill");
-  if (rc == PIE_HIP_OK && counters) inflight_mark(plan, stream);
+  if (rc == PIE_HIP_OK && (counters || cut)) inflight_mark(plan, stream);
   return rc;
+}
+
+extern "C" int pie_hip_attention_prefill(
+    const pie_bf16* q, int64_t q_tok_stride, int64_t q_head_stride, const pie_bf16* k_cache,
+    const pie_bf16* v_cache, int64_t page_stride, int64_t slot_stride, int64_t head_stride,
+    int64_t num_pages, const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_indices,
+    const int32_t* kv_last_page_len, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim,
+    int64_t page_size, float sm_scale, int32_t mode, int64_t window_left, const float* sinks,
+    const uint32_t* packed_mask, const int32_t* mask_extent, const int32_t* plan, int64_t num_items,
+    int64_t mask_offsets_word, pie_bf16* out,
+    int64_t o_tok_stride, int64_t o_head_stride, void* stream) {
+  return attention_prefill_impl(q, q_tok_stride, q_head_stride, k_cache, v_cache, page_stride, slot_stride,
+                                head_stride, num_pages, qo_indptr, kv_indptr, kv_indices, kv_last_page_len,
+                                num_qo_heads, num_kv_heads, head_dim, page_size, sm_scale, mode, window_left, sinks,
+                                packed_mask, mask_extent, plan, num_items, mask_offsets_word, nullptr, nullptr, 0,
+                                out, o_tok_stride, o_head_stride, stream);
+}
+
+extern "C" int pie_hip_attention_prefill_split(
+    const pie_bf16* q, int64_t q_tok_stride, int64_t q_head_stride, const pie_bf16* k_cache,
+    const pie_bf16* v_cache, int64_t page_stride, int64_t slot_stride, int64_t head_stride,
+    int64_t num_pages, const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_indices,
+    const int32_t* kv_last_page_len, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim,
+    int64_t page_size, float sm_scale, int32_t mode, int64_t window_left, const float* sinks,
+    const uint32_t* packed_mask, const int32_t* mask_extent, const int32_t* plan, int64_t num_items,
+    int64_t mask_offsets_word, const int64_t* split, void* scratch, int64_t scratch_bytes, pie_bf16* out,
+    int64_t o_tok_stride, int64_t o_head_stride, void* stream) {
+  PIE_REQUIRE(split, "attention_prefill_split: null split");
+  return attention_prefill_impl(q, q_tok_stride, q_head_stride, k_cache, v_cache, page_stride, slot_stride,
+                                head_stride, num_pages, qo_indptr, kv_indptr, kv_indices, kv_last_page_len,
+                                num_qo_heads, num_kv_heads, head_dim, page_size, sm_scale, mode, window_left, sinks,
+                                packed_mask, mask_extent, plan, num_items, mask_offsets_word, split, scratch,
+                                scratch_bytes, out, o_tok_stride, o_head_stride, stream);
 }
 
 extern "C" int pie_hip_attention_pack_mask(const uint8_t* custom_mask, const int32_t* plan,

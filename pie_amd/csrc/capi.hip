@@ -70,6 +70,14 @@ int inflight_check(const void* key, void* stream, const char* what) {
   return PIE_HIP_OK;
 }
 
+bool inflight_free(const void* key, void* stream) {
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (capturing(st)) return false;
+  std::lock_guard<std::mutex> lk(g_inflight_mu);
+  auto it = g_inflight.find(key);
+  return it == g_inflight.end() || it->second.stream == st || hipEventQuery(it->second.done) != hipErrorNotReady;
+}
+
 void inflight_mark(const void* key, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (capturing(st)) return;

@@ -24,6 +24,9 @@ int num_cus();  // compute units of the current device (cached per device)
 // launch just made. Launches recorded under stream capture are neither checked nor recorded:
 // they run at replay, which the host does not see.
 int inflight_check(const void* key, void* stream, const char* what);
+// Whether an eager launch on `stream` may use `key`: false under capture, and while the last
+// marked launch that used it is still running on another stream.
+bool inflight_free(const void* key, void* stream);
 void inflight_mark(const void* key, void* stream);
 
 // ---------------------------------------------------------------- grouped launch (host)

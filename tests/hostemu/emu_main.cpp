@@ -538,7 +538,8 @@ static void case_group(int64_t B, int64_t H, int64_t I, int64_t V, bool gelu) {
 // query tokens; mode 0 full, 1 causal, 2 a random custom mask.
 static void case_attn_prefill(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t P, int cmax, int qmax,
                               int mode, bool causal_mask = false, int64_t window = -1,
-                              bool with_sinks = false) {
+                              bool with_sinks = false, int cut_cus = 0, int cmin = 0) {
+  if (cut_cus) printf("cut over kv for %d CUs: ", cut_cus);
   Buf<float> sk(Hq);
   fill_sinks(sk);
   const float* sinks_ptr = with_sinks ? sk.p : nullptr;
@@ -546,7 +547,7 @@ static void case_attn_prefill(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int
   printf("attn_prefill B=%lld Hq=%lld Hkv=%lld D=%lld P=%lld ctx<=%d qo<=%d mode=%d window=%lld\n", (long long)B,
          (long long)Hq, (long long)Hkv, (long long)D, (long long)P, cmax, qmax, mode, (long long)window);
   std::vector<int32_t> qo(B + 1, 0), indptr(B + 1, 0), last(B), kvl(B);
-  std::uniform_int_distribution<int> dc(0, cmax), dq(0, qmax);
+  std::uniform_int_distribution<int> dc(cmin, cmax), dq(cut_cus ? 1 : 0, qmax);
   for (int64_t b = 0; b < B; ++b) {
     const int n = dq(rng);
     kvl[b] = dc(rng) + n;
@@ -585,27 +586,42 @@ static void case_attn_prefill(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int
   const int64_t cap = 16 + 8 * (T * Hq / 32 + 2 * B + 2) + 4 * B + 8 + (T * Hq / 32 + 2 * B + 2) * Hkv + 4096;
   Buf<int32_t> plan(cap);
   int64_t words = 0, items = 0, mb = 0, mw = 0;
-  rc_ok(pie_hip_attention_prefill_plan(qi.p, ip.p, ll.p, B, P, Hq, Hkv, D, mode, plan.p, cap, &words, &items, &mb,
-                                       &mw),
-        "prefill_plan");
+  int64_t split[5] = {0, 0, 0, 0, 0};
+  if (cut_cus)
+    rc_ok(pie_hip_attention_prefill_split_plan(qi.p, ip.p, ll.p, B, P, Hq, Hkv, D, mode, window, cut_cus, 1ll << 30,
+                                               plan.p, cap, &words, &items, &mb, &mw, split),
+          "prefill_split_plan");
+  else
+    rc_ok(pie_hip_attention_prefill_plan(qi.p, ip.p, ll.p, B, P, Hq, Hkv, D, mode, plan.p, cap, &words, &items, &mb,
+                                         &mw),
+          "prefill_plan");
+  if (cut_cus && !split[1]) { printf("  nothing was cut\n"); ++failures; }
+  Buf<float> scratch(std::max<int64_t>(split[4] / 4, 4));
   if (mode == 2 && mb != mbytes) { printf("  mask bytes %lld != %lld\n", (long long)mb, (long long)mbytes); ++failures; }
   Buf<uint32_t> packed(std::max<int64_t>(mw, 1));
   Buf<int32_t> extent(std::max<int64_t>(T, 1));
   if (mode == 2)
     rc_ok(pie_hip_attention_pack_mask(mask.p, plan.p, qi.p, ip.p, ll.p, B, P, mw, T, packed.p, extent.p, nullptr),
           "pack_mask");
-  rc_ok(pie_hip_attention_prefill(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page_elems, Hkv * D, D, pages,
-                                  qi.p, ip.p, idx.p, ll.p, Hq, Hkv, D, P, 1.f / sqrtf((float)D), mode, window,
-                                  sinks_ptr,
-                                  mode == 2 ? packed.p : nullptr, mode == 2 ? extent.p : nullptr, plan.p, items,
-                                  plan[4], out.p, Hq * D, D,
-                                  nullptr),
-        "attention_prefill");
+  const uint32_t* pk = mode == 2 ? packed.p : nullptr;
+  const int32_t* ex = mode == 2 ? extent.p : nullptr;
+  const float scale = 1.f / sqrtf((float)D);
+  if (cut_cus)
+    rc_ok(pie_hip_attention_prefill_split(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page_elems, Hkv * D, D,
+                                          pages, qi.p, ip.p, idx.p, ll.p, Hq, Hkv, D, P, scale, mode, window,
+                                          sinks_ptr, pk, ex, plan.p, items, plan[4], split, scratch.p, split[4],
+                                          out.p, Hq * D, D, nullptr),
+          "attention_prefill_split");
+  else
+    rc_ok(pie_hip_attention_prefill(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page_elems, Hkv * D, D, pages,
+                                    qi.p, ip.p, idx.p, ll.p, Hq, Hkv, D, P, scale, mode, window, sinks_ptr, pk, ex,
+                                    plan.p, items, plan[4], out.p, Hq * D, D, nullptr),
+          "attention_prefill");
   oracle_attention(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page_elems, Hkv * D, D, qi.p, ip.p, idx.p,
                    ll.p, mode == 2 ? mask.p : nullptr, mode == 2 ? moff.data() : nullptr, mode == 1, window, B, Hq,
                    Hkv, D, P, 1.0 / sqrt((double)D), want.p, Hq * D,
                    D, nullptr, sinks_ptr);
-  printf("  T=%lld items=%lld\n", (long long)T, (long long)items);
+  printf("  T=%lld items=%lld cut=%lld\n", (long long)T, (long long)items, (long long)split[1]);
   check_close("prefill attention", out.p, want.p, T * Hq * D);
   float worst = 0.f;
   for (int64_t i = 0; i < T * Hq * D; ++i) {
@@ -829,6 +845,14 @@ int main(int argc, char** argv) {
     case_attn_prefill(2, 8, 2, 128, 8, 100, 90, 2, false, 40);    // custom mask + sliding window
     case_attn_prefill(3, 8, 2, 128, 16, 60, 70, 1, false, -1, true);  // causal + sinks (32-row kernel)
     case_attn_prefill(2, 4, 2, 64, 16, 30, 40, 1, false, 20, true);   // D = 64 + window + sinks
+    case_attn_prefill(2, 8, 4, 256, 8, 40, 70, 2);      // D = 256, custom mask, several items per request
+    case_attn_prefill(2, 4, 2, 256, 3, 30, 20, 0);      // D = 256, a tile's rows on several pages
+    case_attn_prefill(2, 8, 2, 64, 16, 100, 90, 2, false, 40);  // D = 64, custom mask + sliding window
+    // items cut over their kv range, and the merge: few query tokens over long contexts
+    case_attn_prefill(2, 8, 2, 128, 16, 1500, 20, 1, false, -1, true, 64, 900);
+    case_attn_prefill(2, 4, 2, 128, 16, 1400, 9, 2, false, -1, false, 64, 900);
+    case_attn_prefill(2, 8, 2, 64, 8, 1300, 17, 1, false, 850, true, 64, 1000);
+    case_attn_prefill(1, 4, 2, 256, 16, 1100, 40, 0, false, -1, false, 64, 800);
   }
   if (all || c == "group") {
     case_group(5, 4096, 1536, 40, false);  // 8 norm vectors per lane pair (NJ = 2)

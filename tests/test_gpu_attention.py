@@ -385,6 +385,76 @@ def test_prefill_repeated_runs_and_graph_replays(dev, custom):
     assert_bf16_close(N(first), want, what="first run vs oracle")
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,P", [(64, 16, 2, 16), (128, 8, 2, 16), (128, 12, 4, 5), (256, 4, 2, 8)])
+@pytest.mark.parametrize("mode", ["causal", "full", "custom", "window"])
+def test_prefill_items_cut_over_kv(dev, D, Hq, Hkv, P, mode):
+    """A few query tokens over long contexts: the plan cuts the items over their kv range (pieces of
+    the partial results merged afterwards; rows beside, at and past a 128-row item, contexts of one
+    to many pieces) and the output matches the oracle; the workspace holds NaN before, so a partial
+    that is read without having been written shows."""
+    print(f"prefill cut D={D} Hq={Hq} Hkv={Hkv} P={P} mode={mode}", flush=True)
+    a = wl.attn_batch([3000, 1, 259, 1700, 5000], [9, 3, 40, 1, 17], Hq=Hq, Hkv=Hkv, D=D, page_size=P, seed=D + P)
+    pb = a["batch"]
+    window = 2100 if mode == "window" else -1
+    custom = None
+    if mode == "custom":
+        n = int((pb.lens.to(torch.int64) * pb.seq_lens.to(torch.int64)).sum())
+        custom = torch.rand(n, generator=torch.Generator().manual_seed(5)) < 0.5
+    ws = torch.full((WS_BYTES // 4,), float("nan"), device=dev)
+    w = attention.BatchPrefillWithPagedKVCacheWrapper(ws, "NHD")
+    w.plan(pb.qo_indptr.to(dev), pb.kv_indptr.to(dev), pb.kv_indices.to(dev), pb.kv_last_page_len.to(dev), Hq, Hkv,
+           D, P, custom_mask=None if custom is None else custom.to(dev), causal=mode in ("causal", "window"),
+           window_left=window)
+    assert w._plan["split"][1] > w._plan["items"]
+    got = w.run(a["q"].to(dev), a["cache"].to(dev))
+    torch.cuda.synchronize()
+    want = _want(a, custom=None if custom is None else custom.numpy(), window_left=window,
+                 causal=mode in ("causal", "window"))
+    assert_bf16_close(N(got), want, what=mode)
+    _tight(got, want, mode)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_prefill_cut_plan_captured_and_on_two_streams(dev, D):
+    """A cut plan's partial results are shared by its runs. Head dims 64 and 256: a captured run,
+    and one made while another stream's run is in flight, take the uncut items, so both give the
+    eager result up to rounding; head dim 128 replays the cut run and refuses the overlap."""
+    a = wl.attn_batch([6000, 9000], [20, 7], Hq=8, Hkv=2, D=D, page_size=16, seed=77)
+    pb = a["batch"]
+    w = attention.BatchPrefillWithPagedKVCacheWrapper(_workspace(dev), "NHD")
+    w.plan(pb.qo_indptr.to(dev), pb.kv_indptr.to(dev), pb.kv_indices.to(dev), pb.kv_last_page_len.to(dev), 8, 2, D,
+           16, causal=True)
+    assert w._plan["split"][1] > 0
+    q, cache = a["q"].to(dev), a["cache"].to(dev)
+    want = _want(a)
+    out = torch.empty_like(q)
+    w.run(q, cache, out=out)
+    torch.cuda.synchronize()
+    _tight(out, want, "eager")
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(g, stream=s):
+            w.run(q, cache, out=out)
+    torch.cuda.current_stream().wait_stream(s)
+    for i in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _tight(out, want, f"replay {i}")
+    if D != 128:
+        s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+        outs = [torch.empty_like(q) for _ in range(6)]
+        torch.cuda.synchronize()
+        for i, o in enumerate(outs):
+            with torch.cuda.stream((s1, s2)[i % 2]):
+                w.run(q, cache, out=o)
+        torch.cuda.synchronize()
+        for o in outs:
+            _tight(o, want, "two streams")
+
+
 def test_prefill_plan_in_use_on_another_stream_is_refused(dev):
     """The head-dim-128 kernel counts its work in the device plan, so two runs sharing a plan
     must not overlap: an eager run while the plan is still in use on another stream is refused
