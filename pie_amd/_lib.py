@@ -107,7 +107,24 @@ def load() -> C.CDLL:
         raise ImportError(f"pie_amd: {LIB_PATH} has ABI {lib.pie_hip_abi_version()}, "
                           f"expected {ABI_VERSION}; rebuild it")
     _lib = lib
+    _bind_fast(lib)
     return lib
+
+
+# The native call path of the small ops (csrc/host/fast.cpp), bound to the loaded library; None
+# until load() and where the module is not built. Its functions return None for a call that the
+# Python wrappers' general path has to handle.
+fast = None
+
+
+def _bind_fast(lib: C.CDLL) -> None:
+    global fast
+    try:
+        from . import _fast
+    except ImportError:
+        return
+    _fast.bind({n: C.cast(getattr(lib, n), C.c_void_p).value for n in SIGNATURES})
+    fast = _fast
 
 
 _fns: dict = {}

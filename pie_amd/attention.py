@@ -143,6 +143,11 @@ class BatchDecodeWithPagedKVCacheWrapper:
             raise NotImplementedError(f"{name}: lse output")
         if q_scale not in (None, 1.0) or k_scale not in (None, 1.0) or v_scale not in (None, 1.0):
             raise NotImplementedError(f"{name}: quantisation scales")
+        if _lib.fast is not None:
+            r = _lib.fast.attention_decode(p, q, paged_kv_cache, self._kv_layout, self._workspace, out,
+                                           _sinks)
+            if r is not None:
+                return r
         _check(name, _BF16, q=q)
         _check(name, torch.int32, indptr=p["indptr"], indices=p["indices"],
                last_page_len=p["last_page_len"])
@@ -294,6 +299,11 @@ class BatchPrefillWithPagedKVCacheWrapper:
             raise NotImplementedError(f"{name}: lse output")
         if q_scale not in (None, 1.0) or k_scale not in (None, 1.0) or v_scale not in (None, 1.0):
             raise NotImplementedError(f"{name}: quantisation scales")
+        if _lib.fast is not None:
+            r = _lib.fast.attention_prefill(p, q, paged_kv_cache, self._kv_layout, C.addressof(p["split"]),
+                                            out, _sinks)
+            if r is not None:
+                return r
         _check(name, _BF16, q=q)
         _check(name, torch.int32, qo_indptr=p["qo_indptr"], indptr=p["indptr"],
                indices=p["indices"], last_page_len=p["last_page_len"])

@@ -21,6 +21,9 @@ LIB = PKG / "libpie_hip.so"
 # measurement probes (plain kernels with a hot-path kernel's access pattern; bench.py --op ceiling)
 PROBE_SRC = PKG / "probe" / "probe.hip"
 PROBE_LIB = PKG / "libpie_probe.so"
+# the native call path of the small ops (a CPython module on torch's C++ API, host code only)
+FAST_SRC = CSRC / "host" / "fast.cpp"
+FAST_LIB = PKG / "_fast.so"
 ARCH = "gfx950"
 
 # Packed fp32 VALU ops are disabled: hipcc would otherwise form v_pk_{add,mul,fma}_f32 from
@@ -58,6 +61,11 @@ def build(verbose: bool = False, out: Path | None = None, defines: tuple[str, ..
     lib = Path(out) if out else LIB
     build_dir = BUILD if not defines else BUILD / ("v_" + "_".join(defines).replace("=", ""))
     build_dir.mkdir(parents=True, exist_ok=True)
+    fast = None
+    if not defines and out is None:
+        pool = cf.ThreadPoolExecutor(max_workers=1)
+        fast = pool.submit(build_fast, verbose)  # beside the kernels
+        pool.shutdown(wait=False)
     srcs = sorted(CSRC.glob("*.hip"))
     if not srcs:
         raise RuntimeError(f"no kernel sources under {CSRC}")
@@ -72,9 +80,35 @@ def build(verbose: bool = False, out: Path | None = None, defines: tuple[str, ..
     os.replace(tmp, lib)
     if verbose:
         print(f"built {lib}")
-    if not defines and out is None:
+    if fast is not None:
         build_probe(verbose)
+        fast.result()
     return lib
+
+
+def build_fast(verbose: bool = False) -> Path:
+    """The native call path, against the installed torch's headers and libraries."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).parent
+    rocm = Path(_hipcc()).resolve().parents[1]
+    tmp = FAST_LIB.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           *[f"-I{p}" for p in (root / "include", root / "include/torch/csrc/api/include",
+                                rocm / "include", sysconfig.get_paths()["include"])],
+           str(FAST_SRC), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-o", str(tmp)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for {FAST_SRC.name}:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, FAST_LIB)
+    if verbose:
+        print(f"built {FAST_LIB}")
+    return FAST_LIB
 
 
 def build_probe(verbose: bool = False) -> Path:

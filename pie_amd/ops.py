@@ -188,8 +188,11 @@ def _rows(name: str, x: torch.Tensor, cols: int) -> torch.Tensor:
     return x.reshape(-1, cols).contiguous()
 
 
+_EPS = float(torch.finfo(torch.float32).eps)
+
+
 def _eps(eps: Optional[float]) -> float:
-    return float(torch.finfo(torch.float32).eps if eps is None else eps)
+    return _EPS if eps is None else float(eps)
 
 
 # ----------------------------------------------------------------------------- RMSNorm
@@ -212,6 +215,10 @@ def gemma_rms_norm(input: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6,
 
 
 def _rmsnorm(name, input, weight, eps, out, gemma):
+    if _lib.fast is not None:
+        r = _lib.fast.rmsnorm(input, weight, eps, out, gemma)
+        if r is not None:
+            return r
     _check(name, _BF16, input=input, weight=weight)
     H = input.shape[-1]
     if weight.shape != (H,):
@@ -310,6 +317,11 @@ def add_rms_norm(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tens
     normed       = rms_norm(new_residual)  -- the next layer's fun.rms_norm (llama3.py:555/:618)
     Pass residual_out=residual to update the residual stream in place.
     """
+    if _lib.fast is not None and _group_keep is None:
+        r = _lib.fast.add_rms_norm(input, residual, weight, _EPS if eps is None else eps, out,
+                                   residual_out, _gemma)
+        if r is not None:
+            return r
     _check("add_rms_norm", _BF16, input=input, residual=residual, weight=weight)
     if input.shape != residual.shape:
         raise ValueError(f"add_rms_norm: input {tuple(input.shape)} != residual {tuple(residual.shape)}")
@@ -359,6 +371,10 @@ def gelu_tanh_and_mul(input: torch.Tensor, out: Optional[torch.Tensor] = None) -
 
 
 def _act_and_mul(name, sym, input, out):
+    if _lib.fast is not None and _group_keep is None:
+        r = _lib.fast.act_and_mul(input, out, sym == "pie_hip_gelu_tanh_and_mul")
+        if r is not None:
+            return r
     _check(name, _BF16, input=input)
     if input.shape[-1] % 2:
         raise ValueError(f"{name}: last dim {input.shape[-1]} must be even")
@@ -385,6 +401,10 @@ def embedding(input: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Ten
     The kernel writes a zero row for an id outside [0, V) (it cannot raise without a host
     sync); check_ids=True validates on the host first and raises IndexError as torch does.
     """
+    if _lib.fast is not None and _group_keep is None and scale is None and not check_ids:
+        r = _lib.fast.embedding(input, weight, out)
+        if r is not None:
+            return r
     _check("embedding", _BF16, weight=weight)
     _check("embedding", torch.int32, input=input)
     if weight.dim() != 2 or weight.stride(1) != 1:
@@ -630,6 +650,14 @@ def qk_rms_norm_rope_append(q, k, v, q_weight, k_weight, eps, pos_ids, batch_ind
     append_paged_kv_cache(k, v, batch_indices, positions, paged_kv_cache, ...).
     Returns the normalised, rotated (q, k) (new contiguous tensors unless q_out/k_out given);
     bit-identical to the three calls."""
+    if _lib.fast is not None and _group_keep is None and isinstance(q, torch.Tensor) and q.dim() == 3 \
+            and 0 < q.shape[2] <= 512 and q.shape[2] % 2 == 0:
+        r = _lib.fast.qk_rms_norm_rope_append(
+            q, k, v, q_weight, k_weight, _EPS if eps is None else eps, pos_ids, batch_indices, positions,
+            paged_kv_cache, kv_indices, kv_indptr, kv_last_page_len, kv_layout,
+            C.addressof(rope_inv_freq(q.shape[2], rope_scale, rope_theta)), q_out, k_out)
+        if r is not None:
+            return r
     T, Hq, Hkv, D, rd = _rope_shapes("qk_rms_norm_rope_append", q, k, pos_ids, None)
     _check("qk_rms_norm_rope_append", _BF16, q_weight=q_weight, k_weight=k_weight)
     if q_weight.shape != (D,) or k_weight.shape != (D,):
