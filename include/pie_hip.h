@@ -479,6 +479,18 @@ int pie_hip_sample(const float* probs, int64_t prob_stride, int64_t prob_rows, i
                    int32_t top_k_scalar, const float* top_p, float top_p_scalar,
                    const float* min_p, float min_p_scalar, const double* uniforms, uint64_t seed,
                    uint64_t offset, int32_t* out, void* stream);
+/*
+ * The same draw for few rows, each row's work spread over several work groups (identical results).
+ * workspace: pie_hip_sample_workspace(batch, vocab, mode) bytes, 16-byte aligned, used until the launch
+ * has run (0: the one-launch form is used anyway, and a NULL workspace always selects it).
+ */
+int64_t pie_hip_sample_workspace(int64_t batch, int64_t vocab, int32_t mode);
+int pie_hip_sample_sliced(const float* probs, int64_t prob_stride, int64_t prob_rows, int64_t vocab,
+                   int64_t batch, const int32_t* row_indices, int32_t mode, const int32_t* top_k,
+                   int32_t top_k_scalar, const float* top_p, float top_p_scalar,
+                   const float* min_p, float min_p_scalar, const double* uniforms, uint64_t seed,
+                   uint64_t offset, int32_t* out, void* workspace,
+                          int64_t workspace_bytes, void* stream);
 
 /*
  * safe_scaled_softmax of pie/src/pie_worker/model/common.py:38-59, :68-188 (the Triton kernel Pie
@@ -489,6 +501,16 @@ int pie_hip_sample(const float* probs, int64_t prob_stride, int64_t prob_rows, i
 int pie_hip_scaled_softmax(const void* logits, int32_t is_bf16, int64_t stride, int64_t batch,
                            int64_t vocab, const float* temperatures, float greedy_threshold,
                            void* out, int64_t out_stride, void* stream);
+/*
+ * The same result for few rows, each row's work spread over several work groups (sums in another
+ * order). In place (out == logits) as above. workspace: pie_hip_scaled_softmax_workspace(batch,
+ * vocab, is_bf16) bytes, 16-byte aligned (0, or a NULL workspace: the one-launch form).
+ */
+int64_t pie_hip_scaled_softmax_workspace(int64_t batch, int64_t vocab, int32_t is_bf16);
+int pie_hip_scaled_softmax_sliced(const void* logits, int32_t is_bf16, int64_t stride, int64_t batch,
+                           int64_t vocab, const float* temperatures, float greedy_threshold,
+                           void* out, int64_t out_stride, void* workspace,
+                                  int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

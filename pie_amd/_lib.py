@@ -17,7 +17,7 @@ HEADER = _PKG.parent / "include" / "pie_hip.h"
 i64, i32, f32, vp = C.c_int64, C.c_int, C.c_float, C.c_void_p
 u64 = C.c_uint64
 
-# name -> argtypes (restype is int for all but pie_hip_last_error)
+# name -> argtypes (restype is int for all but pie_hip_last_error and RETURNS_I64)
 SIGNATURES: dict[str, list] = {
     "pie_hip_abi_version": [],
     "pie_hip_rmsnorm": [vp, i64, vp, vp, i64, i64, i64, f32, vp],
@@ -62,7 +62,12 @@ SIGNATURES: dict[str, list] = {
                                         i64, i64, i64, f32, i32, i64, vp, vp, vp, vp, i64, i64, vp, vp,
                                         i64, vp, i64, i64, vp],
     "pie_hip_sample": [vp, i64, i64, i64, i64, vp, i32, vp, i32, vp, f32, vp, f32, vp, u64, u64, vp, vp],
+    "pie_hip_sample_workspace": [i64, i64, i32],
+    "pie_hip_sample_sliced": [vp, i64, i64, i64, i64, vp, i32, vp, i32, vp, f32, vp, f32, vp, u64, u64, vp,
+                              vp, i64, vp],
     "pie_hip_scaled_softmax": [vp, i32, i64, i64, i64, vp, f32, vp, i64, vp],
+    "pie_hip_scaled_softmax_workspace": [i64, i64, i32],
+    "pie_hip_scaled_softmax_sliced": [vp, i32, i64, i64, i64, vp, f32, vp, i64, vp, i64, vp],
     "pie_hip_group_begin": [],
     "pie_hip_group_end": [vp],
     "pie_hip_group_save": [vp, vp],
@@ -70,6 +75,7 @@ SIGNATURES: dict[str, list] = {
     "pie_hip_get_seq_lens": [vp, vp, i64, i64, vp, vp],
     "pie_hip_get_batch_indices_positions": [vp, vp, i64, i64, vp, vp, vp],
 }
+RETURNS_I64 = {"pie_hip_sample_workspace", "pie_hip_scaled_softmax_workspace"}
 ABI_VERSION = 3
 
 _lib: C.CDLL | None = None
@@ -101,7 +107,7 @@ def load() -> C.CDLL:
     lib.pie_hip_group_free.argtypes = [C.c_void_p]
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)
-        fn.restype = C.c_int
+        fn.restype = C.c_int64 if name in RETURNS_I64 else C.c_int
         fn.argtypes = argtypes
     if lib.pie_hip_abi_version() != ABI_VERSION:
         raise ImportError(f"pie_amd: {LIB_PATH} has ABI {lib.pie_hip_abi_version()}, "

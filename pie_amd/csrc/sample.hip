@@ -28,6 +28,8 @@
 // pass sums chunks of the row so that only the chunk holding the target is scanned.
 #include <math.h>
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace pie {
@@ -1275,10 +1277,249 @@ __device__ __forceinline__ void hist_pass(const float* p, int V, bool vec, HistS
   *row_tot = block_sum_u64(m, sh);
 }
 
+// Few rows leave most of the chip idle at one work group per row (9 rows of 128,256: top_p 69.5 us on
+// 9 CUs). Such top_p launches run sliced: kernel 1 builds the mass histogram of each of S slices of a
+// row (10 us), kernel 2 merges a row's histograms in every slice's work group, picks the bin that
+// holds the threshold and copies the slice's elements from that bin up (or the bin's alone) into the
+// row's list, at the slice's place in vocabulary order, which the histograms give (17 us); kernel 3 is
+// sample_kernel starting from that list (16 us, bound by the search in the bin and the draw in one
+// work group). Plain sampling needs each slice's mass (kernel 1) and a scan of the slice that holds
+// the target. Masses and counts are integers, so the kept set and the draw are those of the
+// one-launch path bit for bit; a row whose list would not fit runs that path in kernel 3.
+constexpr int kMaxSlices = 16;
+struct SliceHead {   // one per (row, slice)
+  uint64_t mass;     // of the slice
+  uint32_t npos;     // its count of p > 0
+  uint32_t lo, hi;   // its non-empty bins lie in [lo, hi] (lo > hi: none)
+  uint32_t over;     // kernel 2: some wave's list overflowed
+};
+struct RowHead {     // one per row
+  uint64_t tot, above;        // the row's mass; the mass in bins above `bin`
+  uint32_t kind;              // 0 no list; 1 every key of the bins from `bin` up; 2 the bin's keys
+  uint32_t bin, n, npos;      // list length; the row's count of p > 0
+};
+struct SliceArgs {
+  int32_t S, per;  // slices per row and elements per slice (a multiple of 4)
+  SliceHead* slices;
+  RowHead* rows;
+  uint32_t* cnt;   // [row][slice][kBins]
+  uint64_t* mass;
+  float* val;      // [row][kCands]
+  uint32_t* idx;
+};
+
+// The row and slice of work group x; false when the row index is outside probs (kernel 3 answers it).
+__device__ __forceinline__ bool slice_of(const SampleArgs& a, const SliceArgs& sl, int& r, int& s, const float*& p,
+                                         int& i0, int& n) {
+  r = blockIdx.x / sl.S;
+  s = blockIdx.x - r * sl.S;
+  const int src = a.rows ? a.rows[r] : r;
+  if (src < 0 || src >= a.nrows) return false;
+  i0 = min(a.V, s * sl.per);
+  n = min(a.V, i0 + sl.per) - i0;
+  p = a.probs + (int64_t)src * a.stride + i0;
+  return true;
+}
+
+__global__ __launch_bounds__(kSampThreads) void sample_hist_kernel(SampleArgs a, SliceArgs sl) {
+  __shared__ SampleShared sh;
+  __shared__ HistShared hs;
+  __shared__ uint32_t range[2];
+  int r, s, i0, n;
+  const float* p;
+  if (!slice_of(a, sl, r, s, p, i0, n)) return;
+  SliceHead& head = sl.slices[blockIdx.x];
+  if (a.mode == 0) {  // plain sampling: the slice's mass alone
+    uint64_t m = 0;
+    for_row(p, n, a.vec != 0, [&](int, float x) { m += prob_mass(x); });
+    m = block_sum_u64(m, sh);
+    if (threadIdx.x == 0) head.mass = m;
+    return;
+  }
+  if (threadIdx.x == 0) { range[0] = kBins; range[1] = 0u; }
+  int64_t npos;
+  uint64_t tot;
+  hist_pass(p, n, a.vec != 0, hs, sh, &npos, &tot);
+  static_assert(kBins == 2 * kSampThreads, "two bins per thread");
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int b = threadIdx.x + h * kSampThreads;
+    if (hs.cnt[b]) {
+      atomicMin(&range[0], (uint32_t)b);
+      atomicMax(&range[1], (uint32_t)b);
+    }
+  }
+  __syncthreads();
+  const uint32_t lo = range[0], hi = range[1];
+  uint32_t* cnt = sl.cnt + (int64_t)blockIdx.x * kBins;
+  uint64_t* mass = sl.mass + (int64_t)blockIdx.x * kBins;
+  for (uint32_t b = lo + threadIdx.x; b <= hi; b += kSampThreads) {
+    cnt[b] = hs.cnt[b];
+    mass[b] = hs.mass[b];
+  }
+  if (threadIdx.x == 0) {
+    head.mass = tot;
+    head.npos = (uint32_t)npos;
+    head.lo = lo;
+    head.hi = hi;
+  }
+}
+
+__global__ __launch_bounds__(kSampThreads) void sample_gather_kernel(SampleArgs a, SliceArgs sl) {
+  __shared__ SampleShared sh;
+  __shared__ HistShared hs;
+  __shared__ CandShared cs;
+  int r, s, i0, n;
+  const float* p;
+  if (!slice_of(a, sl, r, s, p, i0, n)) return;
+  const int S = sl.S;
+  const RowParams rp = row_params(a, r);
+  // every slice's head and bins are loaded at once: one round trip each, not one per slice
+  __shared__ SliceHead heads[kMaxSlices];
+  if ((int)threadIdx.x < S) heads[threadIdx.x] = sl.slices[(int64_t)r * S + threadIdx.x];
+  __syncthreads();
+  uint32_t lo = kBins, hi = 0u, npos = 0;
+  uint64_t tot = 0;
+  for (int i = 0; i < S; ++i) {
+    lo = min(lo, heads[i].lo);
+    hi = max(hi, heads[i].hi);
+    npos += heads[i].npos;
+    tot += heads[i].mass;
+  }
+  const uint32_t* cnt = sl.cnt + (int64_t)r * S * kBins;
+  const uint64_t* mass = sl.mass + (int64_t)r * S * kBins;
+  for (int b = threadIdx.x; b < kBins; b += kSampThreads) {
+    uint32_t c = 0;
+    uint64_t m = 0;
+    if ((uint32_t)b >= lo && (uint32_t)b <= hi) {
+      uint32_t cv[kMaxSlices];
+      uint64_t mv[kMaxSlices];
+#pragma unroll
+      for (int i = 0; i < kMaxSlices; ++i) {  // (bins outside a slice's range hold nothing: not counted)
+        cv[i] = cnt[min(i, S - 1) * kBins + b];
+        mv[i] = mass[min(i, S - 1) * kBins + b];
+      }
+#pragma unroll
+      for (int i = 0; i < kMaxSlices; ++i)
+        if (i < S && (uint32_t)b >= heads[i].lo && (uint32_t)b <= heads[i].hi) {
+          c += cv[i];
+          m += mv[i];
+        }
+    }
+    hs.cnt[b] = c;
+    hs.mass[b] = m;
+  }
+  if (threadIdx.x == 0) { hs.bin = 0xffffffffu; hs.n_ge = 0; hs.n_bin = 0; hs.above = 0; }
+  __syncthreads();
+  select_bin((double)rp.tp * (double)tot, hs);
+  __syncthreads();
+  const uint32_t bin = hs.bin;
+  const uint32_t kind = bin == 0xffffffffu               ? 0u
+                        : hs.n_ge <= (uint32_t)kCands  ? 1u
+                        : hs.n_bin <= (uint32_t)kCands ? 2u
+                                                       : 0u;
+  if (s == 0 && threadIdx.x == 0)
+    sl.rows[r] = RowHead{tot, hs.above, kind, bin, kind == 1u ? hs.n_ge : hs.n_bin, npos};
+  if (kind == 0u) return;
+  // this slice's place in the row's list: the elements that the slices before it put there
+  uint32_t before = 0;
+  const uint32_t b0 = max(bin, lo), b1 = kind == 1u ? hi : bin;
+  const int span = b1 >= b0 ? (int)(b1 - b0 + 1) : 0;
+  for (int j = threadIdx.x; j < s * span; j += kSampThreads) {
+    const int i = j / span;
+    const uint32_t b = b0 + (uint32_t)(j - i * span);
+    if (b >= heads[i].lo && b <= heads[i].hi) before += cnt[i * kBins + b];
+  }
+  const int base = (int)block_sum_u64(before, sh);
+  __syncthreads();
+  int total = 0;
+  const ListPred pred = kind == 1u ? ListPred{0, max(1u, bin << kBinShift), 0u, 0.0} : ListPred{2, 0u, bin, 0.0};
+  const bool ok = gather_list(p, n, a.vec != 0, pred, cs, &total, nullptr);
+  __syncthreads();
+  if (threadIdx.x == 0) sl.slices[blockIdx.x].over = ok ? 0u : 1u;
+  if (!ok) return;
+  float* val = sl.val + (int64_t)r * kCands + base;
+  uint32_t* idx = sl.idx + (int64_t)r * kCands + base;
+  for (int j = threadIdx.x; j < min(total, kCands - base); j += kSampThreads) {
+    val[j] = cs.val[j];
+    idx[j] = cs.idx[j] + (uint32_t)i0;
+  }
+}
+
+// Plain sampling's kernel 2: the slice that holds the target, scanned in index order.
+__global__ __launch_bounds__(kSampThreads) void sample_plain_draw_kernel(SampleArgs a, SliceArgs sl) {
+  __shared__ SampleShared sh;
+  const int r = blockIdx.x;
+  const int src = a.rows ? a.rows[r] : r;
+  if (src < 0 || src >= a.nrows) {  // a row index outside probs: no draw
+    if (threadIdx.x == 0) a.out[r] = -1;
+    return;
+  }
+  const float* p = a.probs + (int64_t)src * a.stride;
+  const RowParams rp = row_params(a, r);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __shared__ uint64_t heads[kMaxSlices];
+  if ((int)threadIdx.x < sl.S) heads[threadIdx.x] = sl.slices[(int64_t)r * sl.S + threadIdx.x].mass;
+  __syncthreads();
+  uint64_t tot = 0, run = 0;
+  for (int i = 0; i < sl.S; ++i) tot += heads[i];
+  const double target = rp.u * (double)tot;
+  int pick = -1;  // the first slice whose inclusive prefix exceeds the target, or the last with mass
+  uint64_t excl_pick = 0;
+  for (int i = 0; i < sl.S; ++i) {
+    const uint64_t m = heads[i];
+    if (m) { pick = i; excl_pick = run; }
+    run += m;
+    if (m && (double)run > target) break;
+  }
+  if (pick < 0) {  // nothing to draw from
+    if (threadIdx.x == 0) a.out[r] = -1;
+    return;
+  }
+  if (threadIdx.x == 0) { sh.pick = -1; sh.u32b = 0u; }
+  const int i0 = pick * sl.per, i1 = min(a.V, i0 + sl.per);
+  uint64_t base = excl_pick;
+  int last = -1;
+  for (int at = i0; at < i1; at += 4 * kSampThreads) {
+    const int i = at + 4 * threadIdx.x;
+    uint64_t m[4], mine = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      m[e] = i + e < i1 ? prob_mass(p[i + e]) : 0ull;
+      mine += m[e];
+      if (m[e]) last = i + e;
+    }
+    const uint64_t incl = wave_incl_scan_u64(mine);
+    __syncthreads();
+    if (lane == 63) sh.wsum[w] = incl;
+    __syncthreads();
+    uint64_t excl = base + incl - mine;
+    uint64_t tile = 0;
+    for (int j = 0; j < kSampWaves; ++j) {
+      if (j < w) excl += sh.wsum[j];
+      tile += sh.wsum[j];
+    }
+    if (mine && (double)(excl + mine) > target && !((double)excl > target)) {
+      uint64_t c = excl;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        c += m[e];
+        if (m[e] && (double)c > target) { sh.pick = i + e; break; }
+      }
+    }
+    __syncthreads();
+    if (sh.pick >= 0) break;
+    base += tile;
+  }
+  if (sh.pick < 0 && last >= 0) atomicMax((unsigned*)&sh.u32b, (unsigned)(last + 1));
+  __syncthreads();
+  if (threadIdx.x == 0) a.out[r] = sh.pick >= 0 ? sh.pick : (int)sh.u32b - 1;
+}
+
 // kTopP: the top_p instantiation (mode 1 only, the histogram path); the other serves modes 0, 2-4.
-// Two kernels, so each gets the registers its own paths need.
-template <bool kTopP>
-__global__ __launch_bounds__(kSampThreads) void sample_kernel(SampleArgs a) {
+// Two kernels, so each gets the registers its own paths need. kSliced: kernel 3 of a sliced top_p.
+template <bool kTopP, bool kSliced>
+__global__ __launch_bounds__(kSampThreads) void sample_kernel(SampleArgs a, SliceArgs sl) {
   prefetch_kernarg<(int)sizeof(SampleArgs)>(a);
   __shared__ SampleShared sh;
   __shared__ CandShared cs;
@@ -1315,8 +1556,45 @@ __global__ __launch_bounds__(kSampThreads) void sample_kernel(SampleArgs a) {
   };
   bool listed = false;
   uint32_t lo_given = 0u;
+  bool from_slices = false;  // the list of kernel 2
+  RowHead rh{};
+  if constexpr (kSliced) {
+    rh = sl.rows[r];
+    const uint32_t over = sl.slices[(int64_t)r * sl.S + min(lane, sl.S - 1)].over;
+    from_slices = rh.kind != 0u && __builtin_amdgcn_ballot_w64(over != 0u) == 0;
+    if (from_slices) {
+      const float* lv = sl.val + (int64_t)r * kCands;
+      const uint32_t* li = sl.idx + (int64_t)r * kCands;
+      for (int i = threadIdx.x; i < (int)rh.n; i += kSampThreads) {
+        cs.val[i] = lv[i];
+        cs.idx[i] = li[i];
+      }
+      __syncthreads();
+      sp = cs.val;
+      sidx = cs.idx;
+      sV = (int)rh.n;
+      svec = true;
+      npos = (int64_t)rh.npos;
+      row_tot = rh.tot;
+      listed = true;
+    }
+  }
   if constexpr (kTopP) {
     __shared__ HistShared hs;
+    if (from_slices) {
+      listed = rh.kind == 1u;
+      if (!listed || sV > kSampThreads) {  // (a short list's threshold comes from its sort)
+        const double thr_in = (double)rp.tp * (double)row_tot - (double)rh.above;
+        lo_given = max(1u, radix_threshold(cs.val, sV, true, 1u, true, 0u, thr_in, sh, rh.bin << kBinShift,
+                                           ~((1u << kBinShift) - 1u), kBinShift - 8));
+      }
+      if (!listed) {  // the draw runs over the row
+        sp = p;
+        sidx = nullptr;
+        sV = V;
+        svec = vec;
+      }
+    } else {
     // top_p: the histogram pass (with the row's count of p > 0 and its mass), then one gather
     hist_pass(p, V, vec, hs, sh, &npos, &row_tot);
     const double thr = (double)rp.tp * (double)row_tot;
@@ -1349,6 +1627,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_kernel(SampleArgs a) {
         sV = V;
         svec = vec;
       }
+    }
     }
     __syncthreads();
   }
@@ -1763,15 +2042,158 @@ __global__ __launch_bounds__(kSampThreads) void scaled_softmax_resident_kernel(
                             : __builtin_amdgcn_exp2f((xt - M) * c) * inv);
 }
 
+// safe_scaled_softmax of few rows, S work groups per row (slices, as in the sampler): kernel 1
+// leaves each slice's maximum, its first index and the sum relative to it; kernel 2 combines a row's
+// slices and writes (5.1 and 6.9 us for 9 rows of 151,936 bf16 logits, 18.6 in one work group per row).
+struct SoftPart {
+  float m, s;
+  int32_t am, pad;
+};
+template <bool BF16>
+__global__ __launch_bounds__(kSampThreads) void scaled_softmax_part_kernel(const void* __restrict__ logits,
+                                                                           int64_t stride, int V, int S, int per,
+                                                                           const float* __restrict__ temps,
+                                                                           float greedy, int vec, int first_masked,
+                                                                           SoftPart* __restrict__ parts) {
+  using IO = RowIO<BF16>;
+  constexpr int E = IO::E;
+  __shared__ float red_max[kSampWaves], red_sum[kSampWaves], red[kSampWaves];
+  const int r = blockIdx.x / S, i0 = min(V, (int)(blockIdx.x - r * S) * per), n = min(V, i0 + per) - i0;
+  const char* row = reinterpret_cast<const char*>(logits) + ((int64_t)r * stride + i0) * (BF16 ? 2 : 4);
+  const float T = temps[r];
+  const bool greedy_row = T < greedy;
+  const float c = greedy_row ? 1.f : 1.4426950408889634f / T;
+  float mx = -INFINITY, s = 0.f;
+  int am = 0x7fffffff;
+  auto visit = [&](float x, int i) {
+    if (x > mx) {
+      s = s * __builtin_amdgcn_exp2f((mx - x) * c);
+      mx = x;
+      am = i;
+    }
+    // (a row of masked logits: its first entry, where the register-resident kernel gives that)
+    if (first_masked && x == -INFINITY && mx == -INFINITY) am = min(am, i);
+    s += x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((x - mx) * c);
+  };
+  const int nv = vec ? n / E : 0;
+  int v = threadIdx.x;
+  for (; v + kSampThreads < nv; v += 2 * kSampThreads) {  // two 16-byte loads in flight
+    float x[2][E];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) IO::load(row, (int64_t)(v + k * kSampThreads) * E, x[k]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int e = 0; e < E; ++e) visit(x[k][e], i0 + (v + k * kSampThreads) * E + e);
+  }
+  for (; v < nv; v += kSampThreads) {
+    float x[E];
+    IO::load(row, (int64_t)v * E, x);
+#pragma unroll
+    for (int e = 0; e < E; ++e) visit(x[e], i0 + v * E + e);
+  }
+  for (int i = nv * E + threadIdx.x; i < n; i += kSampThreads) visit(IO::get(row, i), i0 + i);
+  const float M = block_reduce_once<true>(mx, red_max);
+  s = mx == -INFINITY ? s : s * __builtin_amdgcn_exp2f((mx - M) * c);  // (s is 0 there, or NaN from a NaN)
+  const float sum = block_reduce_once<false>(s, red_sum);
+  const int A = block_min_i(mx == M ? am : 0x7fffffff, red);
+  if (threadIdx.x == 0) parts[blockIdx.x] = SoftPart{M, sum, A, 0};
+}
+
+template <bool BF16>
+__global__ __launch_bounds__(kSampThreads) void scaled_softmax_write_kernel(const void* __restrict__ logits,
+                                                                            int64_t stride, int V, int S, int per,
+                                                                            const float* __restrict__ temps,
+                                                                            float greedy, int vec,
+                                                                            const SoftPart* __restrict__ parts,
+                                                                            void* __restrict__ out,
+                                                                            int64_t out_stride) {
+  using IO = RowIO<BF16>;
+  constexpr int E = IO::E;
+  const int r = blockIdx.x / S, i0 = min(V, (int)(blockIdx.x - r * S) * per), n = min(V, i0 + per) - i0;
+  const char* row = reinterpret_cast<const char*>(logits) + ((int64_t)r * stride + i0) * (BF16 ? 2 : 4);
+  char* orow = reinterpret_cast<char*>(out) + ((int64_t)r * out_stride + i0) * (BF16 ? 2 : 4);
+  const float T = temps[r];
+  const bool greedy_row = T < greedy;
+  const float c = greedy_row ? 1.f : 1.4426950408889634f / T;
+  float M = -INFINITY, sum = 0.f;
+  int A = 0x7fffffff;
+  for (int i = 0; i < S; ++i) {
+    const SoftPart q = parts[r * S + i];
+    if (q.m > M || (q.m == M && q.am < A)) { M = q.m; A = q.am; }
+  }
+  for (int i = 0; i < S; ++i) {
+    const SoftPart q = parts[r * S + i];
+    sum += q.m == -INFINITY ? q.s : q.s * __builtin_amdgcn_exp2f((q.m - M) * c);
+  }
+  const float inv = 1.f / sum;
+  const int nv = vec ? n / E : 0;
+  for (int v = threadIdx.x; v < nv; v += kSampThreads) {
+    float x[E];
+    if (greedy_row) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = i0 + v * E + e == A ? 1.f : 0.f;
+    } else {
+      IO::load(row, (int64_t)v * E, x);
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[e] = __builtin_amdgcn_exp2f((x[e] - M) * c) * inv;
+    }
+    IO::store(orow, (int64_t)v * E, x);
+  }
+  for (int i = nv * E + threadIdx.x; i < n; i += kSampThreads)
+    IO::put(orow, i, greedy_row ? (i0 + i == A ? 1.f : 0.f) : __builtin_amdgcn_exp2f((IO::get(row, i) - M) * c) * inv);
+}
+
 }  // namespace pie
 
 using namespace pie;
 
-extern "C" int pie_hip_sample(const float* probs, int64_t prob_stride, int64_t prob_rows, int64_t vocab,
-                              int64_t batch, const int32_t* row_indices, int32_t mode, const int32_t* top_k,
-                              int32_t top_k_scalar, const float* top_p, float top_p_scalar,
-                              const float* min_p, float min_p_scalar, const double* uniforms,
-                              uint64_t seed, uint64_t offset, int32_t* out, void* stream) {
+// Slices per row of a launch (1: the one-launch path): enough work groups to fill the chip once. Rows
+// per launch and sizes where slices measured faster on [B, 128256]: top_p 69.5 -> 41.7 us at 9 rows,
+// 71 -> 53 at 64 (32,000 entries: 34 -> 37, so long rows only); plain 20.9 -> 12.0 at 9 rows, 15.6 at
+// 32, 27 against 22 at 64; top_k, top_k_top_p and min_p read the row once and lose (21 -> 29).
+constexpr int64_t kSliceGroups = 256, kSliceMinV = 65536;
+static int64_t row_slices(int64_t batch) { return std::min<int64_t>(kMaxSlices, kSliceGroups / batch); }
+static int64_t sample_slices(int64_t batch, int64_t vocab, int64_t mode) {
+  const int64_t most = mode == 1 ? 64 : mode == 0 ? 32 : 0;
+  return batch <= 0 || batch > most || vocab < kSliceMinV ? 1 : row_slices(batch);
+}
+// Workspace: [slice heads | row heads | counts | masses | list values | list indices]
+static int64_t sample_layout(int64_t batch, int64_t S, void* ws, SliceArgs* sl) {
+  int64_t at = 0;
+  const auto take = [&](int64_t bytes) {
+    char* p = static_cast<char*>(ws) + at;
+    at += (bytes + 255) / 256 * 256;
+    return p;
+  };
+  char* slices = take(batch * S * (int64_t)sizeof(SliceHead));
+  char* rows = take(batch * (int64_t)sizeof(RowHead));
+  char* cnt = take(batch * S * kBins * 4);
+  char* mass = take(batch * S * kBins * 8);
+  char* val = take(batch * kCands * 4);
+  char* idx = take(batch * kCands * 4);
+  if (sl) {
+    sl->slices = reinterpret_cast<SliceHead*>(slices);
+    sl->rows = reinterpret_cast<RowHead*>(rows);
+    sl->cnt = reinterpret_cast<uint32_t*>(cnt);
+    sl->mass = reinterpret_cast<uint64_t*>(mass);
+    sl->val = reinterpret_cast<float*>(val);
+    sl->idx = reinterpret_cast<uint32_t*>(idx);
+  }
+  return at;
+}
+
+extern "C" int64_t pie_hip_sample_workspace(int64_t batch, int64_t vocab, int32_t mode) {
+  const int64_t S = sample_slices(batch, vocab, mode);
+  return S > 1 ? sample_layout(batch, S, nullptr, nullptr) : 0;
+}
+
+static int sample_impl(const float* probs, int64_t prob_stride, int64_t prob_rows, int64_t vocab,
+                       int64_t batch, const int32_t* row_indices, int32_t mode, const int32_t* top_k,
+                       int32_t top_k_scalar, const float* top_p, float top_p_scalar,
+                       const float* min_p, float min_p_scalar, const double* uniforms,
+                       uint64_t seed, uint64_t offset, int32_t* out, void* workspace, int64_t workspace_bytes,
+                       void* stream) {
   if (batch == 0) return PIE_HIP_OK;  // an empty batch (whose tensors may have null data)
   PIE_REQUIRE(probs && out, "sample: null probs or out");
   PIE_REQUIRE(vocab > 0 && vocab < (1ll << 28) && batch >= 0 && batch < (1ll << 31) &&
@@ -1784,14 +2206,64 @@ extern "C" int pie_hip_sample(const float* probs, int64_t prob_stride, int64_t p
   SampleArgs a{probs, prob_stride, (int32_t)vocab, (int32_t)batch, row_indices, (int32_t)prob_rows, mode, top_k,
                top_k_scalar, top_p, top_p_scalar, min_p, min_p_scalar, uniforms, seed, offset, out,
                (prob_stride % 4 == 0 && aligned16(probs)) ? 1 : 0};
-  hipLaunchKernelGGL(mode == 1 ? sample_kernel<true> : sample_kernel<false>, dim3((unsigned)batch), dim3(kSampThreads), 0,
-                     static_cast<hipStream_t>(stream), a);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const dim3 rows((unsigned)batch), block(kSampThreads);
+  SliceArgs sl{};
+  const int64_t S = sample_slices(batch, vocab, mode);
+  if (S > 1 && workspace && aligned16(workspace) && workspace_bytes >= sample_layout(batch, S, nullptr, nullptr)) {
+    sl.S = (int32_t)S;
+    sl.per = (int32_t)(((vocab + 3) / 4 + S - 1) / S * 4);
+    sample_layout(batch, S, workspace, &sl);
+    const dim3 slices((unsigned)(batch * S));
+    hipLaunchKernelGGL(sample_hist_kernel, slices, block, 0, st, a, sl);
+    if (mode == 1) {
+      hipLaunchKernelGGL(sample_gather_kernel, slices, block, 0, st, a, sl);
+      hipLaunchKernelGGL((sample_kernel<true, true>), rows, block, 0, st, a, sl);
+    } else {
+      hipLaunchKernelGGL(sample_plain_draw_kernel, rows, block, 0, st, a, sl);
+    }
+  } else {
+    hipLaunchKernelGGL((mode == 1 ? sample_kernel<true, false> : sample_kernel<false, false>), rows, block, 0, st, a, sl);
+  }
   return check_launch("sample");
 }
 
-extern "C" int pie_hip_scaled_softmax(const void* logits, int32_t is_bf16, int64_t stride, int64_t batch,
-                                      int64_t vocab, const float* temperatures, float greedy_threshold,
-                                      void* out, int64_t out_stride, void* stream) {
+extern "C" int pie_hip_sample(const float* probs, int64_t prob_stride, int64_t prob_rows, int64_t vocab,
+                              int64_t batch, const int32_t* row_indices, int32_t mode, const int32_t* top_k,
+                              int32_t top_k_scalar, const float* top_p, float top_p_scalar,
+                              const float* min_p, float min_p_scalar, const double* uniforms,
+                              uint64_t seed, uint64_t offset, int32_t* out, void* stream) {
+  return sample_impl(probs, prob_stride, prob_rows, vocab, batch, row_indices, mode, top_k, top_k_scalar, top_p,
+                     top_p_scalar, min_p, min_p_scalar, uniforms, seed, offset, out, nullptr, 0, stream);
+}
+
+extern "C" int pie_hip_sample_sliced(const float* probs, int64_t prob_stride, int64_t prob_rows, int64_t vocab,
+                                     int64_t batch, const int32_t* row_indices, int32_t mode, const int32_t* top_k,
+                                     int32_t top_k_scalar, const float* top_p, float top_p_scalar,
+                                     const float* min_p, float min_p_scalar, const double* uniforms,
+                                     uint64_t seed, uint64_t offset, int32_t* out, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  return sample_impl(probs, prob_stride, prob_rows, vocab, batch, row_indices, mode, top_k, top_k_scalar, top_p,
+                     top_p_scalar, min_p, min_p_scalar, uniforms, seed, offset, out, workspace, workspace_bytes,
+                     stream);
+}
+
+// Slices per row (1: one work group per row): for at most 64 rows of more than 16 16-byte vectors per
+// thread, whose exponentials one work group does not keep in registers. Measured for 9 rows: fp32
+// [9, 128256] 26.9 -> 11.5 us (33.6 -> 19.6 at 64 rows), bf16 [9, 151936] 18.6 -> 12.0; rows within 16
+// vectors gain nothing (bf16 [9, 128256] 12.7 -> 11.3 with a second launch; [64, 128256] 13.0 -> 14.5).
+static int64_t softmax_slices(int64_t batch, int64_t vocab, bool is_bf16) {
+  return batch <= 0 || batch > 64 || vocab <= 16 * kSampThreads * (is_bf16 ? 8 : 4) ? 1 : row_slices(batch);
+}
+
+extern "C" int64_t pie_hip_scaled_softmax_workspace(int64_t batch, int64_t vocab, int32_t is_bf16) {
+  const int64_t S = softmax_slices(batch, vocab, is_bf16 != 0);
+  return S > 1 ? batch * S * (int64_t)sizeof(SoftPart) : 0;
+}
+
+static int scaled_softmax_impl(const void* logits, int32_t is_bf16, int64_t stride, int64_t batch, int64_t vocab,
+                               const float* temperatures, float greedy_threshold, void* out, int64_t out_stride,
+                               void* workspace, int64_t workspace_bytes, void* stream) {
   if (batch == 0) return PIE_HIP_OK;  // an empty batch (whose tensors may have null data)
   PIE_REQUIRE(logits && out && temperatures, "scaled_softmax: null pointer");
   PIE_REQUIRE(vocab > 0 && vocab < (1ll << 31) && batch >= 0 && batch < (1ll << 31) && stride >= vocab &&
@@ -1805,12 +2277,32 @@ extern "C" int pie_hip_scaled_softmax(const void* logits, int32_t is_bf16, int64
   // (65,536 entries: at 20 the fp32 kernel's registers spill)
   const int64_t per_thread = (vocab / e + kSampThreads - 1) / kSampThreads;
   const dim3 grid((unsigned)batch), block(kSampThreads);
+  const bool resident = vec && vocab >= e && per_thread <= (is_bf16 ? 20 : 16);
+  const int64_t S = softmax_slices(batch, vocab, is_bf16 != 0);
+  if (S > 1 && workspace && aligned16(workspace) &&
+      workspace_bytes >= pie_hip_scaled_softmax_workspace(batch, vocab, is_bf16)) {
+    const int per = (int)(((vocab + 7) / 8 + S - 1) / S * 8);  // slices start on whole vectors
+    SoftPart* parts = static_cast<SoftPart*>(workspace);
+    const dim3 slices((unsigned)(batch * S));
+#define PIE_SOFTMAX_SLICED(BF)                                                                               \
+  hipLaunchKernelGGL(scaled_softmax_part_kernel<BF>, slices, block, 0, st, logits, stride, (int)vocab, (int)S, per, \
+                     temperatures, greedy_threshold, vec, resident ? 1 : 0, parts);                          \
+  hipLaunchKernelGGL(scaled_softmax_write_kernel<BF>, slices, block, 0, st, logits, stride, (int)vocab, (int)S,  \
+                     per, temperatures, greedy_threshold, vec, parts, out, out_stride)
+    if (is_bf16) {
+      PIE_SOFTMAX_SLICED(true);
+    } else {
+      PIE_SOFTMAX_SLICED(false);
+    }
+#undef PIE_SOFTMAX_SLICED
+    return check_launch("scaled_softmax");
+  }
 #define PIE_SOFTMAX_RESIDENT(BF, NV)                                                                      \
   hipLaunchKernelGGL((scaled_softmax_resident_kernel<BF, NV>), grid, block, 0, st, logits, stride, (int)vocab, \
                      temperatures, greedy_threshold, out, out_stride)
   // (rows shorter than one 16-byte vector take the streaming kernel: the resident one reads
   // whole vectors)
-  if (vec && vocab >= e && per_thread <= (is_bf16 ? 20 : 16)) {
+  if (resident) {
     if (is_bf16) {
       if (per_thread <= 8) PIE_SOFTMAX_RESIDENT(true, 8);
       else if (per_thread <= 16) PIE_SOFTMAX_RESIDENT(true, 16);
@@ -1828,4 +2320,19 @@ extern "C" int pie_hip_scaled_softmax(const void* logits, int32_t is_bf16, int64
   }
 #undef PIE_SOFTMAX_RESIDENT
   return check_launch("scaled_softmax");
+}
+
+extern "C" int pie_hip_scaled_softmax(const void* logits, int32_t is_bf16, int64_t stride, int64_t batch,
+                                      int64_t vocab, const float* temperatures, float greedy_threshold,
+                                      void* out, int64_t out_stride, void* stream) {
+  return scaled_softmax_impl(logits, is_bf16, stride, batch, vocab, temperatures, greedy_threshold, out, out_stride,
+                             nullptr, 0, stream);
+}
+
+extern "C" int pie_hip_scaled_softmax_sliced(const void* logits, int32_t is_bf16, int64_t stride, int64_t batch,
+                                             int64_t vocab, const float* temperatures, float greedy_threshold,
+                                             void* out, int64_t out_stride, void* workspace,
+                                             int64_t workspace_bytes, void* stream) {
+  return scaled_softmax_impl(logits, is_bf16, stride, batch, vocab, temperatures, greedy_threshold, out, out_stride,
+                             workspace, workspace_bytes, stream);
 }

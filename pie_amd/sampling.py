@@ -7,8 +7,9 @@ pie/src/flashinfer_metal/sampling.py:19-79 (whose top-k keeps the batch's larges
 row and whose top-p drops the token that crosses p; these follow flashinfer: per-row k, and the
 crossing token stays).
 
-Each call is one kernel launch (``pie_hip_sample``): one work group per row, exact thresholds by
-radix select, an inverse-CDF draw in index order. Randomness: Philox4x32-10 keyed by ``seed`` and
+Each call is one kernel launch, one work group per row (``pie_hip_sample_sliced``: for few long rows
+of top_p and plain sampling two or three launches, several work groups per row, same draws): exact
+thresholds by radix select, an inverse-CDF draw in index order. Randomness: Philox4x32-10 keyed by ``seed`` and
 counted by ``offset``; when neither is given, a per-process seed (from torch's default generator)
 and an offset that advances by one per call, so successive calls draw independent numbers and a
 fixed (seed, offset) reproduces a draw exactly. ``generator=`` (a torch.Generator) supplies the
@@ -92,10 +93,13 @@ def _sample(name, mode, probs, indices, top_k=0, top_p=1.0, min_p=0.0, generator
     s, o = _seed_offset(generator, seed, offset)
     out = torch.empty(B, dtype=torch.int32, device=dev)
     ptr = lambda t: t.data_ptr() if t is not None else None
-    _lib.call("pie_hip_sample", probs.data_ptr(), probs.stride(0), probs.shape[0], probs.shape[1], B,
+    # few rows: scratch that spreads each row over several work groups
+    need = _lib.load().pie_hip_sample_workspace(B, probs.shape[1], _MODES[mode])
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    _lib.call("pie_hip_sample_sliced", probs.data_ptr(), probs.stride(0), probs.shape[0], probs.shape[1], B,
               ptr(rows),
               _MODES[mode], ptr(tk), int(tks), ptr(tp), float(tps), ptr(mp), float(mps), ptr(u),
-              C.c_uint64(s), C.c_uint64(o), out.data_ptr(), _stream(probs))
+              C.c_uint64(s), C.c_uint64(o), out.data_ptr(), ptr(ws), need, _stream(probs))
     return out
 
 
@@ -171,7 +175,11 @@ def safe_scaled_softmax(logits: torch.Tensor, temperatures: torch.Tensor,
         out = torch.empty_like(logits)
     elif out.shape != logits.shape or out.dtype != logits.dtype or out.stride(1) != 1:
         raise ValueError(f"{name}: out must match logits")
-    _lib.call("pie_hip_scaled_softmax", logits.data_ptr(), 1 if logits.dtype == torch.bfloat16 else 0,
-              logits.stride(0), B, V, t.data_ptr(), float(greedy_threshold), out.data_ptr(),
-              out.stride(0), _stream(logits))
+    bf16 = 1 if logits.dtype == torch.bfloat16 else 0
+    # few long rows: scratch that spreads each row over several work groups
+    need = _lib.load().pie_hip_scaled_softmax_workspace(B, V, bf16)
+    ws = torch.empty(need, dtype=torch.uint8, device=logits.device) if need else None
+    _lib.call("pie_hip_scaled_softmax_sliced", logits.data_ptr(), bf16, logits.stride(0), B, V,
+              t.data_ptr(), float(greedy_threshold), out.data_ptr(), out.stride(0),
+              None if ws is None else ws.data_ptr(), need, _stream(logits))
     return out

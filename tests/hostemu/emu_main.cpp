@@ -677,6 +677,15 @@ static void case_sample(int64_t B, int64_t V, int mode, bool row_map, bool peake
   for (int64_t r = 0; r < B; ++r) memcpy(mapped.p + r * V, probs.p + (int64_t)rows[r] * V, V * 4);
   oracle_sample(mapped.p, B, V, V, mode, topk.p, topp.p, minp.p, u.p, want.p, nullptr);
   check_equal("sample", out.p, want.p, B);
+  const int64_t wb = pie_hip_sample_workspace(B, V, mode);
+  if (wb) {  // few long rows: several work groups per row
+    Buf<char> ws(wb);
+    memset(ws.p, 0xab, wb);
+    for (int64_t r = 0; r < B; ++r) out[r] = -7;
+    rc_ok(pie_hip_sample_sliced(padded.p, S, B, V, B, row_map ? rows.p : nullptr, mode, topk.p, 0, topp.p, 0.f, minp.p,
+                                0.f, u.p, 0, 0, out.p, ws.p, wb, nullptr), "sample_sliced");
+    check_equal("sample sliced", out.p, want.p, B);
+  }
 }
 
 // masked: rows carry -inf logits (padding / banned tokens): row 1 its first 3/4, row 2 every
@@ -704,6 +713,20 @@ static void case_softmax(int64_t B, int64_t V, bool bf16, bool masked = false) {
     if (!(fabs(g - want[i]) <= 1e-2 * fabs(want[i]) + 1e-7)) ++bad;
   }
   printf("  %-40s %s (%zu / %lld outside 1e-2 rel + 1e-7 abs)\n", "scaled_softmax", bad ? "FAIL" : "ok", bad,
+         (long long)(B * V));
+  failures += bad != 0;
+  const int64_t wb = pie_hip_scaled_softmax_workspace(B, V, bf16);
+  if (!wb) return;
+  Buf<char> ws(wb);
+  memset(ws.p, 0xab, wb);
+  if (bf16) rc_ok(pie_hip_scaled_softmax_sliced(xb.p, 1, V, B, V, temps.p, 1e-5f, ob.p, V, ws.p, wb, nullptr), "sliced");
+  else rc_ok(pie_hip_scaled_softmax_sliced(x.p, 0, V, B, V, temps.p, 1e-5f, out.p, V, ws.p, wb, nullptr), "sliced");
+  bad = 0;
+  for (int64_t i = 0; i < B * V; ++i) {
+    const double g = bf16 ? bf2f(ob[i]) : out[i];
+    if (!(fabs(g - want[i]) <= 1e-2 * fabs(want[i]) + 1e-7)) ++bad;
+  }
+  printf("  %-40s %s (%zu / %lld outside 1e-2 rel + 1e-7 abs)\n", "scaled_softmax sliced", bad ? "FAIL" : "ok", bad,
          (long long)(B * V));
   failures += bad != 0;
 }
@@ -828,6 +851,9 @@ int main(int argc, char** argv) {
     case_softmax(4, 1000, false, true);   // -inf logits, register-resident kernel
     case_softmax(4, 4096, true, true);
     case_softmax(4, 70003, false, true);  // -inf logits, streaming kernel
+    case_softmax(4, 140001, true, true);  // sliced rows of bf16 logits, not 16-byte aligned
+    case_sample(3, 70001, 0, true);       // plain sampling over slices
+    case_sample(2, 66000, 0, false, true, 3, 65000);  // most slices empty
   }
   if (all || c == "prefill") {
     case_attn_prefill(3, 8, 2, 128, 16, 40, 45, 1);   // causal, chunked prefill over cached context

@@ -6,12 +6,14 @@ kept-set distribution (chi-square over 40k draws with a fixed seed) and stay ins
 at full vocabulary size (Llama-3 128256, Qwen3 151936)."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from pie_amd import sampling
+from pie_amd import _lib, sampling
 from tests._util import assert_bf16_close
 
 pytestmark = pytest.mark.gpu
@@ -337,3 +339,77 @@ def test_sample_one_read_and_fallbacks(dev, mode, case):
                                top_p=prm["top_p"].numpy(), min_p=prm["min_p"].numpy())
     assert kept[np.arange(B), got].all()
     assert (got == want).all(), f"{got} vs {want}"
+
+
+def _one_launch(probs, mode, **kw):
+    """The draw by the one-launch entry point (no workspace)."""
+    B, V = probs.shape
+    out = torch.empty(B, dtype=torch.int32, device=probs.device)
+    p = lambda t: t.data_ptr() if t is not None else None
+    _lib.call("pie_hip_sample", probs.data_ptr(), probs.stride(0), B, V, B, None, mode, p(kw.get("top_k")), 0,
+              p(kw.get("top_p")), 0.0, p(kw.get("min_p")), 0.0, None, C.c_uint64(11), C.c_uint64(5), out.data_ptr(),
+              torch.cuda.current_stream().cuda_stream)
+    return out
+
+
+@pytest.mark.parametrize("B,V", [(1, 65536), (2, 70003), (9, 151936), (16, 100277), (33, 128256), (64, 65539)])
+@pytest.mark.parametrize("kind", ["peaked", "flat", "ties", "sparse"])
+def test_sliced_draws_equal_the_one_launch(dev, B, V, kind):
+    """Few long rows of top_p and plain sampling run over several work groups per row: the same
+    tokens as one work group per row (the other samplers keep it), rows of few and of all tokens kept, ties, and mostly zero rows."""
+    print(f"sliced draws B={B} V={V} {kind}", flush=True)
+    assert _lib.load().pie_hip_sample_workspace(B, V, 1) > 0
+    assert (_lib.load().pie_hip_sample_workspace(B, V, 0) > 0) == (B <= 32)
+    g = torch.Generator(device=dev).manual_seed(B + V)
+    x = torch.randn((B, V), generator=g, device=dev) * {"peaked": 4.0, "flat": 0.01, "ties": 1.0, "sparse": 2.0}[kind]
+    if kind == "ties":
+        x = x.round()
+    if kind == "sparse":
+        x[:, 7:-9] = -float("inf")
+        x[0] = -float("inf")
+        x[0, V // 2] = 0.0
+    probs = torch.softmax(x, -1)
+    if kind == "sparse" and B > 1:
+        probs[1] = 0.0  # nothing to draw
+    u = lambda: torch.rand(B, generator=g, device=dev)
+    tk = (1 + 300 * u()).int()
+    tk[-1] = 0
+    kw = dict(seed=11, offset=5)
+    tp, mp = u(), 0.5 * u()
+    for got, want in (
+            (sampling.sampling_from_probs(probs, **kw), _one_launch(probs, 0)),
+            (sampling.top_p_sampling_from_probs(probs, tp, **kw), _one_launch(probs, 1, top_p=tp)),
+            (sampling.top_k_sampling_from_probs(probs, tk, **kw), _one_launch(probs, 2, top_k=tk)),
+            (sampling.min_p_sampling_from_probs(probs, mp, **kw), _one_launch(probs, 3, min_p=mp)),
+            (sampling.top_k_top_p_sampling_from_probs(probs, tk, tp, **kw),
+             _one_launch(probs, 4, top_k=tk, top_p=tp))):
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,V", [(1, 131080), (5, 140003), (9, 151936), (64, 131073)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sliced_softmax(dev, B, V, dtype):
+    """softmax over several work groups per row against float64, with masked logits, a greedy row
+    whose maximum is tied across slices, and a row with a NaN."""
+    print(f"sliced softmax B={B} V={V} {dtype}", flush=True)
+    assert _lib.load().pie_hip_scaled_softmax_workspace(B, V, int(dtype == torch.bfloat16)) > 0
+    g = torch.Generator(device=dev).manual_seed(V + B)
+    x = (torch.randn((B, V), generator=g, device=dev) * 3).to(dtype)
+    x[:, ::3] = -float("inf")
+    temps = 0.5 + torch.rand(B, generator=g, device=dev)
+    temps[0] = 0.0
+    x[0, V - 2] = x[0, V // 2 + 1] = 100.0
+    if B > 4:
+        x[4, V // 3] = float("nan")
+    got = sampling.safe_scaled_softmax(x, temps)
+    one = torch.zeros(V, device=dev)
+    one[V // 2 + 1] = 1
+    assert torch.equal(got[0].float(), one)
+    for r in range(1, B):
+        if r == 4:
+            assert bool(got[r].isnan().all())
+            continue
+        want = torch.softmax(x[r].double() / temps[r].double(), -1)
+        err = (got[r].double() - want).abs() / (want + 1e-30)
+        # fp32 sums and exponentials (2^-20 with the argument's rounding), then one bf16 rounding
+        assert float(err[want > 1e-30].max()) <= (2.0**-8 if dtype == torch.bfloat16 else 1e-5)
