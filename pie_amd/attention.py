@@ -112,8 +112,10 @@ class BatchDecodeWithPagedKVCacheWrapper:
                 max_kv = int(((np_ - 1).clamp(min=0) * page_size + last_page_len.to(torch.int64)).max())
         splits = C.c_int64(0)
         dev = self._workspace.device
-        _lib.call("pie_hip_attention_decode_plan", batch, num_kv_heads, max_kv,
-                  _num_cus(dev) if dev.type == "cuda" else 0, C.byref(splits))
+        cus = _num_cus(dev) if dev.type == "cuda" else 0
+        if head_dim == 256:  # one work group fits a CU, where the rule counts on two
+            cus = max(cus // 2, 1) if cus else 128
+        _lib.call("pie_hip_attention_decode_plan", batch, num_kv_heads, max_kv, cus, C.byref(splits))
         s = splits.value
         need = batch * s * num_qo_heads * (head_dim + 1) * 4 if s > 1 else 0
         ws_bytes = self._workspace.numel() * self._workspace.element_size()

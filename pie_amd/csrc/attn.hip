@@ -1466,19 +1466,26 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
 
 using namespace pie;
 
-// Host: how many splits per request. Aims at ~4 work groups per CU over all (request, kv head,
-// split) triples when the launch takes requests longest first (batches of at most kRankMax), at
-// ~16 otherwise (smaller pieces even out the tail that request order leaves); when the longest
-// context is known (max_kv_len >= 0) no split is shorter than kMinChunk tokens. The result
-// depends on the batch only, so one plan serves a captured graph.
+// Host: how many splits per request, for per = batch * kv heads work groups a split. A work group
+// costs ~4 us before and after its tokens (ranking, page table, first loads, merge), so where per
+// fills at most half the CUs a launch aims at the ~2 work groups per CU that run at once, and at more,
+// which evens out requests of different lengths, as per grows: 3 per CU below one per CU, 4 from
+// there (batches of at most kRankMax, longest requests first; larger batches ~16: request order
+// leaves a longer tail). Measured (us, cache cold, Llama-8B heads): 8 x 500-4,000 tokens 8 splits
+// 24.0, 16 27.1; 3 x 16-32k 21 splits 80.7, 43 84.9; 24 x 128-4,096 4 splits 53.2, 6 55.1, 2 58.7;
+// 32 x 128-4,096 4 splits 73.4, 1 76.7. When the longest context is known (max_kv_len >= 0) no split
+// is shorter than kMinChunk tokens. The result depends on the batch only, so one plan serves a
+// captured graph.
 extern "C" int pie_hip_attention_decode_plan(int64_t batch, int64_t num_kv_heads, int64_t max_kv_len,
                                              int64_t num_cus, int64_t* splits) {
   PIE_REQUIRE(splits && batch >= 0 && num_kv_heads > 0, "decode_plan: bad batch %lld / num_kv_heads %lld",
               (long long)batch, (long long)num_kv_heads);
   const int64_t cus = num_cus > 0 ? num_cus : 256;
   const int64_t per = std::max<int64_t>(1, batch * num_kv_heads);
-  const int64_t groups = (batch <= kRankMax ? 4 : 16) * cus;
-  int64_t s = (groups + per - 1) / per;
+  int64_t s = batch > kRankMax ? (16 * cus + per - 1) / per
+              : per >= cus     ? (4 * cus + per - 1) / per
+              : 2 * per > cus  ? 3 * cus / per
+                               : 2 * cus / per;
   if (max_kv_len >= 0) s = std::min<int64_t>(s, std::max<int64_t>(1, (max_kv_len + kMinChunk - 1) / kMinChunk));
   *splits = std::max<int64_t>(1, std::min<int64_t>(s, 64));
   return PIE_HIP_OK;
