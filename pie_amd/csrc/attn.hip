@@ -325,8 +325,9 @@ constexpr int kRankMax = 256;  // one request per thread of the work group
 __device__ __forceinline__ int request_of_rank(const PagedKV& kv, int B, int window_left, int r,
                                                int32_t* lens, int32_t* pick, int& kv_len, int& page0) {
   const int i = threadIdx.x;
-  int kl = 0, li = -1;  // padding: below every length
+  int kl = 0, li = -1, p0 = 0;  // padding: below every length
   if (i < B) {
+    p0 = kv.indptr[i];
     kl = kv_length(kv, i);
     li = window_left >= 0 ? min(kl, window_left + 1) : kl;
   }
@@ -342,12 +343,12 @@ __device__ __forceinline__ int request_of_rank(const PagedKV& kv, int B, int win
         before += le > li || (le == li && k + e < i);
       }
     }
-    if (before == r) { pick[0] = i; pick[1] = kl; }
+    if (before == r) { pick[0] = i; pick[1] = kl; pick[2] = p0; }
   }
   __syncthreads();
   const int b = uniform(pick[0]);
   kv_len = uniform(pick[1]);
-  page0 = kv.indptr[b];
+  page0 = uniform(pick[2]);  // (not loaded again: a round trip before the page table's)
   return b;
 }
 
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   constexpr int kSmem = (4 * kVtile * 2 > 4 * 16 * (D + 2) * 4) ? 4 * kVtile * 2 : 4 * 16 * (D + 2) * 4;
   static_assert(kSmem >= kRankMax * 4, "the ranked lengths fit in the V tiles' LDS");
   __shared__ __attribute__((aligned(16))) char smem[kSmem];
-  __shared__ int32_t rank_pick[2];
+  __shared__ int32_t rank_pick[3];
 
   const int Hkv = Hq / G;
   const int per = splits * Hkv;
@@ -512,7 +513,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 // before the first is used, and meet in LDS. Partial s of the lane's row is
 // po[s * o_stride .. +8) (fp32, normalised) with log2-sum-exp pl[s * l_stride]. Every thread of the
 // work group calls it; wave 0 gets the row's weighted sum (acc), weight sum (L) and maximum (M,
-// -inf if no partial saw anything).
+// -inf if no partial saw anything) of partials [0, ns); there is memory for room >= max(ns, 1).
 // Bound: load latency. The partials are read in ns / 32 rounds of independent loads, and only the
 // splits that hold tokens: 3.0 us for one request of 1,000 tokens planned at 64 splits (32 heads,
 // 8 splits hold tokens) and 5.3 us for three of 16-32k tokens at 43; one wave reading every split
@@ -521,7 +522,7 @@ constexpr int kMergeBatch = 8;
 template <int D>
 __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int64_t o_stride,
                                                const float* __restrict__ pl, int64_t l_stride, int ns,
-                                               float (&acc)[8], float& L, float& M) {
+                                               int room, float (&acc)[8], float& L, float& M) {
   constexpr int CH = D / 8;
   __shared__ float sm[4][64][10];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -529,12 +530,15 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
   L = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-  for (int s0 = w; s0 < ns; s0 += 4 * kMergeBatch) {
+  // The first round's loads do not wait for ns (which may itself be in flight): partials [ns, room)
+  // are memory, but hold nothing, and count as zero.
+  for (int s0 = w; s0 == w || s0 < ns; s0 += 4 * kMergeBatch) {
+    const int top = (s0 == w ? room : ns) - 1;
     float4 a[kMergeBatch], b[kMergeBatch];
     float ls[kMergeBatch];
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
-      const int s = min(s0 + 4 * k, ns - 1);
+      const int s = min(s0 + 4 * k, top);
       ls[k] = pl[s * l_stride];
       a[k] = *reinterpret_cast<const float4*>(po + s * o_stride);
       b[k] = *reinterpret_cast<const float4*>(po + s * o_stride + 4);
@@ -542,7 +546,10 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
     float mx = M;
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
-      if (s0 + 4 * k >= ns) ls[k] = -INFINITY;
+      if (s0 + 4 * k >= ns) {
+        ls[k] = -INFINITY;
+        a[k] = b[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
       mx = fmaxf(mx, ls[k]);
     }
     if (mx == -INFINITY) continue;
@@ -606,7 +613,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(PagedKV kv, int window_
   const int ns = split_count(len, splits);
   const int64_t first = (int64_t)b * splits * Hq + hl;
   float acc[8], L, M;
-  merge_partials<D>(part_o + first * D + 8 * c, (int64_t)Hq * D, part_lse + first, Hq, ns, acc, L, M);
+  merge_partials<D>(part_o + first * D + 8 * c, (int64_t)Hq * D, part_lse + first, Hq, ns, splits, acc, L, M);
   if (threadIdx.x >= 64 || hq >= Hq) return;
   if (M != -INFINITY) L += sink_mass(sinks, hq, M);
   const float inv = L > 0.f ? 1.f / L : 0.f;
@@ -1452,7 +1459,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
   const int64_t first = ((int64_t)slot * n_kv_heads + kvh) * kPrefillRows + (R - row0);
   const int64_t step = (int64_t)n_kv_heads * kPrefillRows;
   float acc[8], L, M;
-  merge_partials<D>(part_o + first * D + 8 * c, step * D, part_lse + first, step, pieces, acc, L, M);
+  merge_partials<D>(part_o + first * D + 8 * c, step * D, part_lse + first, step, pieces, pieces, acc, L, M);
   if (threadIdx.x >= 64 || row0 + rl0 + lane / CH >= rows) return;
   const int tok = R / G, hq = kvh * G + (R - tok * G);
   if (M != -INFINITY) L += sink_mass(sinks, hq, M);
