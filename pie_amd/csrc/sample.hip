@@ -2162,7 +2162,7 @@ static int64_t sample_slices(int64_t batch, int64_t vocab, int64_t mode) {
 static int64_t sample_layout(int64_t batch, int64_t S, void* ws, SliceArgs* sl) {
   int64_t at = 0;
   const auto take = [&](int64_t bytes) {
-    char* p = static_cast<char*>(ws) + at;
+    char* p = ws ? static_cast<char*>(ws) + at : nullptr;  // null: only the size is asked for
     at += (bytes + 255) / 256 * 256;
     return p;
   };
