@@ -677,14 +677,16 @@ static void case_sample(int64_t B, int64_t V, int mode, bool row_map, bool peake
   for (int64_t r = 0; r < B; ++r) memcpy(mapped.p + r * V, probs.p + (int64_t)rows[r] * V, V * 4);
   oracle_sample(mapped.p, B, V, V, mode, topk.p, topp.p, minp.p, u.p, want.p, nullptr);
   check_equal("sample", out.p, want.p, B);
-  const int64_t wb = pie_hip_sample_workspace(B, V, mode);
-  if (wb) {  // few long rows: several work groups per row
+  // few long rows: several work groups per row (64 of 1024 lanes each, slow here: one or two rows, row 1 with ties)
+  const int64_t nb = B > 2 ? 2 : 1, r0 = B == 2 ? 1 : 0;
+  const int64_t wb = pie_hip_sample_workspace(nb, V, mode);
+  if (wb) {
     Buf<char> ws(wb);
     memset(ws.p, 0xab, wb);
     for (int64_t r = 0; r < B; ++r) out[r] = -7;
-    rc_ok(pie_hip_sample_sliced(padded.p, S, B, V, B, row_map ? rows.p : nullptr, mode, topk.p, 0, topp.p, 0.f, minp.p,
-                                0.f, u.p, 0, 0, out.p, ws.p, wb, nullptr), "sample_sliced");
-    check_equal("sample sliced", out.p, want.p, B);
+    rc_ok(pie_hip_sample_sliced(padded.p, S, B, V, nb, rows.p + r0, mode, topk.p + r0, 0, topp.p + r0, 0.f,
+                                minp.p + r0, 0.f, u.p + r0, 0, 0, out.p, ws.p, wb, nullptr), "sample_sliced");
+    check_equal("sample sliced", out.p, want.p + r0, nb);
   }
 }
 
@@ -716,7 +718,7 @@ static void case_softmax(int64_t B, int64_t V, bool bf16, bool masked = false) {
          (long long)(B * V));
   failures += bad != 0;
   const int64_t wb = pie_hip_scaled_softmax_workspace(B, V, bf16);
-  if (!wb) return;
+  if (!wb || !masked) return;  // slow here: the rows with -inf logits
   Buf<char> ws(wb);
   memset(ws.p, 0xab, wb);
   if (bf16) rc_ok(pie_hip_scaled_softmax_sliced(xb.p, 1, V, B, V, temps.p, 1e-5f, ob.p, V, ws.p, wb, nullptr), "sliced");
@@ -876,8 +878,8 @@ int main(int argc, char** argv) {
     case_attn_prefill(2, 8, 2, 64, 16, 100, 90, 2, false, 40);  // D = 64, custom mask + sliding window
     // items cut over their kv range, and the merge: few query tokens over long contexts
     case_attn_prefill(2, 8, 2, 128, 16, 1500, 20, 1, false, -1, true, 64, 900);
-    case_attn_prefill(2, 4, 2, 128, 16, 1400, 9, 2, false, -1, false, 64, 900);
-    case_attn_prefill(2, 8, 2, 64, 8, 1300, 17, 1, false, 850, true, 64, 1000);
+    case_attn_prefill(1, 4, 2, 128, 16, 1400, 9, 2, false, -1, false, 64, 900);
+    case_attn_prefill(1, 8, 2, 64, 8, 1300, 17, 1, false, 850, true, 64, 1000);
     case_attn_prefill(1, 4, 2, 256, 16, 1100, 40, 0, false, -1, false, 64, 800);
   }
   if (all || c == "group") {
