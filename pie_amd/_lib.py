@@ -119,7 +119,7 @@ def load() -> C.CDLL:
 
 # The native call path of the small ops (csrc/host/fast.cpp), bound to the loaded library; None
 # until load() and where the module is not built. Its functions return None for a call that the
-# Python wrappers' general path has to handle.
+# Python wrappers' general path has to handle, and raise an error of the launch itself.
 fast = None
 
 
@@ -129,8 +129,12 @@ def _bind_fast(lib: C.CDLL) -> None:
         from . import _fast
     except ImportError:
         return
-    _fast.bind({n: C.cast(getattr(lib, n), C.c_void_p).value for n in SIGNATURES})
+    _fast.bind(_addresses(lib), _check_rc)
     fast = _fast
+
+
+def _addresses(lib: C.CDLL) -> dict:
+    return {n: C.cast(getattr(lib, n), C.c_void_p).value for n in SIGNATURES}
 
 
 _fns: dict = {}
@@ -142,6 +146,12 @@ def call(name: str, *args) -> None:
     if fn is None:
         fn = _fns[name] = getattr(load(), name)
     rc = fn(*args)
+    if rc != 0:
+        _check_rc(name, rc)
+
+
+def _check_rc(name: str, rc: int) -> None:
+    """Raise the library's error of a call that returned ``rc`` on this thread."""
     if rc != 0:
         msg = load().pie_hip_last_error().decode(errors="replace")
         if rc == 1:

@@ -7,9 +7,11 @@
 // costs little more than its output allocations and launches.
 //
 // Every function handles the plain case and returns None for anything else (another type or tensor
-// subclass, a transform's or mode's tensor, a dtype, shape, stride or device it does not serve, an
-// error from the library): the Python wrapper then takes its general path, which accepts, converts
-// or refuses the call as it always has. Nothing is kept between calls.
+// subclass, a transform's or mode's tensor, a dtype, shape, stride or device it does not serve, a
+// call the library refuses before any launch): the Python wrapper then takes its general path, which
+// accepts, converts or refuses the call as it always has. An error of the launch itself is raised
+// here: it is found after the kernel was handed to the runtime, so the op must not be issued again.
+// Nothing is kept between calls.
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -128,6 +130,22 @@ int launch(F&& f) {
   return rc;
 }
 
+// The binding's check(entry point name, return code), which raises the library's error (bind()).
+PyObject* on_error = nullptr;
+
+// Makes the call; hands it to the general path where the library refused it before any launch, and
+// raises any other error.
+#define LAUNCH(name, ...)                                                    \
+  do {                                                                       \
+    const int rc = launch([&] { return __VA_ARGS__; });                      \
+    if (rc == PIE_HIP_EINVAL || rc == PIE_HIP_EBUSY) NOT_SERVED;             \
+    if (rc != PIE_HIP_OK) {                                                  \
+      Py_XDECREF(PyObject_CallFunction(on_error, "si", name, rc));           \
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, name);      \
+      return nullptr;                                                        \
+    }                                                                        \
+  } while (0)
+
 // rmsnorm(input, weight, eps, out, gemma)
 PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -142,10 +160,12 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   SERVE(output(a[3], *x, x->sizes(), out));
   const Rows yr = rows(out, H);
   SERVE(yr.ok);
-  const auto fn = a[4] == Py_True ? lib.pie_hip_gemma_rmsnorm : lib.pie_hip_rmsnorm;
+  const bool gemma = a[4] == Py_True;
+  const auto fn = gemma ? lib.pie_hip_gemma_rmsnorm : lib.pie_hip_rmsnorm;
   void* st = stream_of(*x);
   const uint16_t* wp = ptr<uint16_t>(*w);
-  SERVE(launch([&] { return fn(xr.p, xr.stride, wp, yr.p, yr.stride, xr.n, H, (float)eps, st); }) == 0);
+  LAUNCH(gemma ? "pie_hip_gemma_rmsnorm" : "pie_hip_rmsnorm",
+         fn(xr.p, xr.stride, wp, yr.p, yr.stride, xr.n, H, (float)eps, st));
   return give(a[3], out);
   END_HANDLE_TH_ERRORS
 }
@@ -165,12 +185,12 @@ PyObject* add_rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   SERVE(output(a[4], *x, x->sizes(), out) && output(a[5], *x, x->sizes(), sum));
   const Rows yr = rows(out, H), sr = rows(sum, H);
   SERVE(yr.ok && sr.ok);
-  const auto fn = a[6] == Py_True ? lib.pie_hip_gemma_fused_add_rmsnorm : lib.pie_hip_fused_add_rmsnorm;
+  const bool gemma = a[6] == Py_True;
+  const auto fn = gemma ? lib.pie_hip_gemma_fused_add_rmsnorm : lib.pie_hip_fused_add_rmsnorm;
   void* st = stream_of(*x);
   const uint16_t* wp = ptr<uint16_t>(*w);
-  SERVE(launch([&] {
-          return fn(xr.p, xr.stride, rr.p, rr.stride, sr.p, sr.stride, yr.p, yr.stride, wp, xr.n, H, (float)eps, st);
-        }) == 0);
+  LAUNCH(gemma ? "pie_hip_gemma_fused_add_rmsnorm" : "pie_hip_fused_add_rmsnorm",
+         fn(xr.p, xr.stride, rr.p, rr.stride, sr.p, sr.stride, yr.p, yr.stride, wp, xr.n, H, (float)eps, st));
   PyObject* pair = PyTuple_New(2);
   if (!pair) return nullptr;
   PyTuple_SET_ITEM(pair, 0, give(a[4], out));
@@ -194,9 +214,10 @@ PyObject* act_and_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   SERVE(output(a[1], *x, sizes, out));
   const Rows yr = rows(out, I);
   SERVE(yr.ok);
-  const auto fn = a[2] == Py_True ? lib.pie_hip_gelu_tanh_and_mul : lib.pie_hip_silu_and_mul;
+  const bool gelu = a[2] == Py_True;
+  const auto fn = gelu ? lib.pie_hip_gelu_tanh_and_mul : lib.pie_hip_silu_and_mul;
   void* st = stream_of(*x);
-  SERVE(launch([&] { return fn(xr.p, xr.stride, yr.p, yr.stride, xr.n, I, st); }) == 0);
+  LAUNCH(gelu ? "pie_hip_gelu_tanh_and_mul" : "pie_hip_silu_and_mul", fn(xr.p, xr.stride, yr.p, yr.stride, xr.n, I, st));
   return give(a[1], out);
   END_HANDLE_TH_ERRORS
 }
@@ -218,9 +239,7 @@ PyObject* embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* st = stream_of(*w);
   const int32_t* ip = ptr<int32_t>(*ids);
   const uint16_t* wp = ptr<uint16_t>(*w);
-  SERVE(launch([&] {
-          return lib.pie_hip_embedding(ip, T, wp, w->size(0), H, w->stride(0), yr.p, yr.stride, st);
-        }) == 0);
+  LAUNCH("pie_hip_embedding", lib.pie_hip_embedding(ip, T, wp, w->size(0), H, w->stride(0), yr.p, yr.stride, st));
   return give(a[2], out);
   END_HANDLE_TH_ERRORS
 }
@@ -287,12 +306,11 @@ PyObject* qk_rms_norm_rope_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
            *kop = ptr<uint16_t>(ko), *qwp = ptr<uint16_t>(*qw), *kwp = ptr<uint16_t>(*kw);
   const int32_t *pp = ptr<int32_t>(*pos), *bp = ptr<int32_t>(*bi), *sp = ptr<int32_t>(*ps), *kip = ptr<int32_t>(*ki),
                 *kpi = ptr<int32_t>(*kp);
-  SERVE(launch([&] {
-          return lib.pie_hip_qk_rmsnorm_rope_append(
-              qp, q->stride(0), q->stride(1), kpp, k->stride(0), k->stride(1), vp, v->stride(0), v->stride(1), qop,
-              qo.stride(0), qo.stride(1), kop, ko.stride(0), ko.stride(1), qwp, kwp, (float)eps, pp, T, Hq, Hkv, D,
-              inv, bp, sp, kip, kpi, kp->numel() - 1, c.k, c.v, c.pages, c.page, c.slot, c.head, c.page_size, st);
-        }) == 0);
+  LAUNCH("pie_hip_qk_rmsnorm_rope_append",
+         lib.pie_hip_qk_rmsnorm_rope_append(
+             qp, q->stride(0), q->stride(1), kpp, k->stride(0), k->stride(1), vp, v->stride(0), v->stride(1), qop,
+             qo.stride(0), qo.stride(1), kop, ko.stride(0), ko.stride(1), qwp, kwp, (float)eps, pp, T, Hq, Hkv, D,
+             inv, bp, sp, kip, kpi, kp->numel() - 1, c.k, c.v, c.pages, c.page, c.slot, c.head, c.page_size, st));
   PyObject* pair = PyTuple_New(2);
   if (!pair) return nullptr;
   PyTuple_SET_ITEM(pair, 0, give(a[15], qo));
@@ -354,11 +372,10 @@ PyObject* attention_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t wn = ws.numel() * (int64_t)ws.element_size();
   uint16_t *qp = ptr<uint16_t>(*q), *op = ptr<uint16_t>(out);
   const int32_t *ipp = ptr<int32_t>(*ip), *ixp = ptr<int32_t>(*ix), *llp = ptr<int32_t>(*ll);
-  SERVE(launch([&] {
-          return lib.pie_hip_attention_decode(qp, q->stride(0), q->stride(1), c.k, c.v, c.page, c.slot, c.head, c.pages,
-                                              ipp, ixp, llp, B, Hq, Hkv, D, P, (float)scale, window, sinks, splits, wp,
-                                              wn, op, out.stride(0), out.stride(1), st);
-        }) == 0);
+  LAUNCH("pie_hip_attention_decode",
+         lib.pie_hip_attention_decode(qp, q->stride(0), q->stride(1), c.k, c.v, c.page, c.slot, c.head, c.pages, ipp,
+                                      ixp, llp, B, Hq, Hkv, D, P, (float)scale, window, sinks, splits, wp, wn, op,
+                                      out.stride(0), out.stride(1), st));
   return give(a[5], out);
   END_HANDLE_TH_ERRORS
 }
@@ -404,22 +421,23 @@ PyObject* attention_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 *plp = ptr<int32_t>(*plan), *exp = extent ? ptr<int32_t>(*extent) : nullptr;
   const uint32_t* pkp = packed ? ptr<uint32_t>(*packed) : nullptr;
   const int64_t scn = scratch->numel();
-  SERVE(launch([&] {
-          return lib.pie_hip_attention_prefill_split(qp, q->stride(0), q->stride(1), c.k, c.v, c.page, c.slot, c.head,
-                                                     c.pages, qip, ipp, ixp, llp, Hq, Hkv, D, P, (float)scale,
-                                                     (int32_t)mode, window, sinks, pkp, exp, plp, items, woff, split,
-                                                     scp, scn, op, out.stride(0), out.stride(1), st);
-        }) == 0);
+  LAUNCH("pie_hip_attention_prefill_split",
+         lib.pie_hip_attention_prefill_split(qp, q->stride(0), q->stride(1), c.k, c.v, c.page, c.slot, c.head, c.pages,
+                                             qip, ipp, ixp, llp, Hq, Hkv, D, P, (float)scale, (int32_t)mode, window,
+                                             sinks, pkp, exp, plp, items, woff, split, scp, scn, op, out.stride(0),
+                                             out.stride(1), st));
   return give(a[5], out);
   END_HANDLE_TH_ERRORS
 }
 
-// bind({entry point name: address}): the loaded library's functions
-PyObject* bind(PyObject*, PyObject* d) {
-  if (!PyDict_CheckExact(d)) {
-    PyErr_SetString(PyExc_TypeError, "bind: a dict of entry point addresses");
+// bind({entry point name: address}, check): the loaded library's functions, and check(name, code)
+// raising the library's error of a call that returned code
+PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 2 || !PyDict_CheckExact(a[0]) || !PyCallable_Check(a[1])) {
+    PyErr_SetString(PyExc_TypeError, "bind: a dict of entry point addresses and the error check");
     return nullptr;
   }
+  PyObject* d = a[0];
   Lib next;
 #define X(name)                                                              \
   {                                                                          \
@@ -434,11 +452,13 @@ PyObject* bind(PyObject*, PyObject* d) {
   PIE_ENTRY_POINTS(X)
 #undef X
   lib = next;
+  Py_INCREF(a[1]);
+  Py_XSETREF(on_error, a[1]);
   Py_RETURN_NONE;
 }
 
 #define FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {{"bind", bind, METH_O, nullptr},
+PyMethodDef methods[] = {FAST(bind),
                          FAST(rmsnorm),
                          FAST(add_rms_norm),
                          FAST(act_and_mul),

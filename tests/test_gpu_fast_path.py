@@ -3,6 +3,9 @@ takes (ranks, row strides, given outputs, single rows, odd sizes) and forms it h
 layouts, modes): same bits, same objects for given outputs, same exceptions."""
 from __future__ import annotations
 
+import contextlib
+import ctypes as C
+
 import pytest
 import torch
 
@@ -129,3 +132,80 @@ def test_modes_and_subclasses_take_the_general_path(dev):
     assert _lib.fast.rmsnorm(x.as_subclass(Sub), w, 1e-5, None, False) is None
     assert _lib.fast.rmsnorm(x, w, "1e-5", None, False) is None
     assert _lib.fast.rmsnorm(x) is None
+
+
+_ENTRY_POINTS = ("pie_hip_rmsnorm", "pie_hip_gemma_rmsnorm", "pie_hip_fused_add_rmsnorm",
+                 "pie_hip_gemma_fused_add_rmsnorm", "pie_hip_silu_and_mul", "pie_hip_gelu_tanh_and_mul",
+                 "pie_hip_embedding", "pie_hip_qk_rmsnorm_rope_append", "pie_hip_attention_decode",
+                 "pie_hip_attention_prefill_split")
+
+
+@contextlib.contextmanager
+def _native_entry_points_return(rc, calls):
+    """The native path's entry points replaced by stubs that record their name and return rc."""
+    addr = _lib._addresses(_lib.load())
+    stubs = {}
+    for n in _ENTRY_POINTS:
+        def stub(*args, n=n):
+            calls.append(n)
+            return rc
+        stubs[n] = C.CFUNCTYPE(C.c_int, *_lib.SIGNATURES[n])(stub)
+    try:
+        _lib.fast.bind({**addr, **{n: C.cast(f, C.c_void_p).value for n, f in stubs.items()}}, _lib._check_rc)
+        yield
+    finally:
+        _lib.fast.bind(addr, _lib._check_rc)
+
+
+def _one_call_each(dev):
+    """(entry point, call) of every op the native path serves; the in-place ones among them."""
+    x, r, w = _x(dev, 4, 256), _x(dev, 4, 256, seed=1), _x(dev, 256, seed=2)
+    a = wl.attn_batch([40, 0, 700], [1, 1, 1], Hq=8, Hkv=2, D=128, page_size=16, seed=9)
+    pb, cache = a["batch"], a["cache"].to(dev)
+    t = {n: getattr(pb, n).to(dev) for n in ("qo_indptr", "kv_indptr", "kv_indices", "kv_last_page_len",
+                                             "positions", "batch_indices")}
+    q, k, v = wl.split_qkv(_x(dev, 3, 12 * 128), 8, 2, 128)
+    qw, kw = _x(dev, 128, seed=1), _x(dev, 128, seed=2)
+    ws = lambda: torch.zeros(32 << 20, dtype=torch.uint8, device=dev)
+    d = attention.BatchDecodeWithPagedKVCacheWrapper(ws(), "NHD")
+    d.plan(t["kv_indptr"], t["kv_indices"], t["kv_last_page_len"], 8, 2, 128, 16)
+    p = attention.BatchPrefillWithPagedKVCacheWrapper(ws(), "NHD")
+    p.plan(t["qo_indptr"], t["kv_indptr"], t["kv_indices"], t["kv_last_page_len"], 8, 2, 128, 16, causal=True)
+    qc = q.contiguous()
+    return [
+        ("pie_hip_rmsnorm", lambda: ops.rmsnorm(x, w)),
+        ("pie_hip_gemma_rmsnorm", lambda: ops.gemma_rms_norm(x, w)),
+        ("pie_hip_fused_add_rmsnorm", lambda: ops.fused_add_rmsnorm(x, r, w)),
+        ("pie_hip_gemma_fused_add_rmsnorm", lambda: ops.gemma_add_rms_norm(x, r, w, residual_out=r)),
+        ("pie_hip_silu_and_mul", lambda: ops.silu_and_mul(x)),
+        ("pie_hip_gelu_tanh_and_mul", lambda: ops.gelu_tanh_and_mul(x)),
+        ("pie_hip_embedding", lambda: ops.embedding(t["positions"], x)),
+        ("pie_hip_qk_rmsnorm_rope_append", lambda: ops.qk_rms_norm_rope_append(
+            q, k, v, qw, kw, 1e-6, t["positions"], t["batch_indices"], t["positions"], cache, t["kv_indices"],
+            t["kv_indptr"], t["kv_last_page_len"], q_out=q, k_out=k)),
+        ("pie_hip_attention_decode", lambda: d.run(qc, cache)),
+        ("pie_hip_attention_prefill_split", lambda: p.run(qc, cache)),
+    ]
+
+
+def test_a_rejected_launch_raises_and_is_not_repeated(dev):
+    """PIE_HIP_ELAUNCH comes after the kernel was handed to the runtime (the error may be an older
+    one of the thread): the native path raises it, as the general path does, and runs the op once."""
+    for name, call in _one_call_each(dev):
+        calls = []
+        with _native_entry_points_return(2, calls):
+            with pytest.raises(_lib.PieHipError, match=f"{name} failed"):
+                call()
+        assert calls == [name]
+
+
+@pytest.mark.parametrize("rc", [1, 3])
+def test_a_refusal_before_any_launch_takes_the_general_path(dev, rc):
+    """Invalid arguments and busy state are returned before any launch: the general path then runs,
+    or refuses, the call."""
+    for name, call in _one_call_each(dev):
+        calls = []
+        with _native_entry_points_return(rc, calls):
+            call()
+        assert calls == [name]
+    torch.cuda.synchronize()
