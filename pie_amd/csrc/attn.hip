@@ -1647,19 +1647,17 @@ extern "C" int pie_hip_attention_decode_noalloc(
               "or pie_hip_attention_decode with a workspace)",
               what, (long long)need, (long long)kDecodeScratchBytes);
   void* ws = nullptr;
+  InflightClaim claim;
   if (need > 0) {
-    int rc = decode_scratch(&ws);
+    const int rc = decode_scratch(&ws);
     if (rc) return rc;
-    rc = inflight_check(ws, stream, what);
-    if (rc) return rc;
+    if (claim.take(ws, stream) == InflightClaim::kBusy) return inflight_busy(what);
   }
-  const int rc = attention_decode_impl(q, q_tok_stride, q_head_stride, k_cache, v_cache, page_stride,
+  return attention_decode_impl(q, q_tok_stride, q_head_stride, k_cache, v_cache, page_stride,
                                slot_stride, head_stride, num_pages, kv_indptr, kv_indices,
                                kv_last_page_len, batch, num_qo_heads, num_kv_heads, head_dim,
                                page_size, sm_scale, window_left, sinks, splits, ws, kDecodeScratchBytes,
                                out, o_tok_stride, o_head_stride, stream, what);
-  if (rc == PIE_HIP_OK && need > 0) inflight_mark(ws, stream);
-  return rc;
 }
 
 // Host: the prefill work list. Reads host copies of qo_indptr, kv_indptr and kv_last_page_len
@@ -1969,12 +1967,14 @@ static int attention_prefill_impl(
   if (num_items == 0) return PIE_HIP_OK;
   // The head-dim-128 kernel counts its work in the plan's header words, so runs of one plan must not
   // overlap. The other head dims' runs may: one that overlaps another stream's (or is captured,
-  // when that cannot be seen) leaves the scratch alone and runs the plan's uncut items.
+  // when that cannot be seen) leaves the scratch alone and runs the plan's uncut items. So does, at
+  // any head dim, one whose launches would fall between those of another thread's run on its stream.
   const bool counters = head_dim == 128;
-  if (counters) {
-    if ((rc = inflight_check(plan, stream, "attention_prefill")) != PIE_HIP_OK) return rc;
-  } else if (cut) {
-    cut = inflight_free(plan, stream);
+  InflightClaim claim;
+  if (counters || cut) {
+    const InflightClaim::State got = claim.take(plan, stream);
+    if (counters && got == InflightClaim::kBusy) return inflight_busy("attention_prefill");
+    cut = cut && (got == InflightClaim::kOwn || (counters && got == InflightClaim::kCapture));
   }
   PrefillLaunch a{};
   a.st = static_cast<hipStream_t>(stream);
@@ -2004,9 +2004,7 @@ static int attention_prefill_impl(
     case 128: launch_prefill<128>(a); break;
     default: launch_prefill<256>(a); break;
   }
-  rc = check_launch("attention_prefill");
-  if (rc == PIE_HIP_OK && (counters || cut)) inflight_mark(plan, stream);
-  return rc;
+  return check_launch("attention_prefill");
 }
 
 extern "C" int pie_hip_attention_prefill(

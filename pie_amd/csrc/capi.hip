@@ -45,6 +45,7 @@ namespace {
 struct Inflight {
   hipStream_t stream;
   hipEvent_t done;
+  int launching;  // runs between take() and the claim's end, all on `stream`
 };
 std::mutex g_inflight_mu;
 std::unordered_map<const void*, Inflight> g_inflight;
@@ -55,41 +56,40 @@ bool capturing(hipStream_t st) {
 }
 }  // namespace
 
-int inflight_check(const void* key, void* stream, const char* what) {
+InflightClaim::State InflightClaim::take(const void* key, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (capturing(st)) return PIE_HIP_OK;
-  std::lock_guard<std::mutex> lk(g_inflight_mu);
-  auto it = g_inflight.find(key);
-  if (it == g_inflight.end() || it->second.stream == st) return PIE_HIP_OK;
-  if (hipEventQuery(it->second.done) == hipErrorNotReady)
-    return set_error(PIE_HIP_EBUSY,
-                     "%s: a launch on another stream still uses the same device state (the "
-                     "static scratch or the prefill plan); synchronise first, or give each stream "
-                     "its own",
-                     what);
-  return PIE_HIP_OK;
-}
-
-bool inflight_free(const void* key, void* stream) {
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (capturing(st)) return false;
-  std::lock_guard<std::mutex> lk(g_inflight_mu);
-  auto it = g_inflight.find(key);
-  return it == g_inflight.end() || it->second.stream == st || hipEventQuery(it->second.done) != hipErrorNotReady;
-}
-
-void inflight_mark(const void* key, void* stream) {
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (capturing(st)) return;
+  if (capturing(st)) return kCapture;
   std::lock_guard<std::mutex> lk(g_inflight_mu);
   auto it = g_inflight.find(key);
   if (it == g_inflight.end()) {
     hipEvent_t ev = nullptr;
-    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return;
-    it = g_inflight.emplace(key, Inflight{st, ev}).first;
+    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return kUntracked;
+    it = g_inflight.emplace(key, Inflight{st, ev, 0}).first;
   }
-  it->second.stream = st;
-  (void)hipEventRecord(it->second.done, st);
+  Inflight& f = it->second;
+  if (f.stream != st && (f.launching > 0 || hipEventQuery(f.done) == hipErrorNotReady)) return kBusy;
+  f.stream = st;
+  key_ = key;
+  stream_ = stream;
+  return f.launching++ > 0 ? kShared : kOwn;
+}
+
+InflightClaim::~InflightClaim() {
+  if (!key_) return;
+  hipStream_t st = static_cast<hipStream_t>(stream_);
+  std::lock_guard<std::mutex> lk(g_inflight_mu);
+  Inflight& f = g_inflight.find(key_)->second;
+  // (an event that cannot be recorded would answer for an earlier run: wait for this one instead)
+  if (hipEventRecord(f.done, st) != hipSuccess) (void)hipStreamSynchronize(st);
+  --f.launching;
+}
+
+int inflight_busy(const char* what) {
+  return set_error(PIE_HIP_EBUSY,
+                   "%s: a launch on another stream still uses the same device state (the "
+                   "static scratch or the prefill plan); synchronise first, or give each stream "
+                   "its own",
+                   what);
 }
 
 }  // namespace pie

@@ -17,17 +17,33 @@ int set_error(int code, const char* fmt, ...);
 int check_launch(const char* what);
 int num_cus();  // compute units of the current device (cached per device)
 
-// Device state that overlapping launches would race on (the allocation-free decode's static
-// scratch, a prefill plan's work counters), keyed by its address. inflight_check refuses a
-// launch (PIE_HIP_EBUSY) while the last launch that used `key` is still running on another
-// stream; launches on the same stream are ordered by it and pass. inflight_mark records the
-// launch just made. Launches recorded under stream capture are neither checked nor recorded:
-// they run at replay, which the host does not see.
-int inflight_check(const void* key, void* stream, const char* what);
-// Whether an eager launch on `stream` may use `key`: false under capture, and while the last
-// marked launch that used it is still running on another stream.
-bool inflight_free(const void* key, void* stream);
-void inflight_mark(const void* key, void* stream);
+// A claim on device state that overlapping runs would race on (the allocation-free decode's static
+// scratch, a prefill plan's work counters and the partial results of its cut items), keyed by its
+// address. take() tests and reserves in one step, before the run's launches; the destructor, after
+// them, gives the reservation back and records the stream, so a run on another stream is busy until
+// the recorded one has finished.
+class InflightClaim {
+ public:
+  enum State {
+    kOwn,       // this run alone
+    kShared,    // another thread is making its launches on the same stream: stream order serves state
+                // that one kernel uses, not state handed from one kernel to the next
+    kBusy,      // another stream's run is being made or still running; nothing is claimed
+    kCapture,   // the stream is being captured: the run happens at replay, which the host does not see
+    kUntracked  // no event to be had: nothing is known or recorded
+  };
+  State take(const void* key, void* stream);
+  ~InflightClaim();
+  InflightClaim() = default;
+  InflightClaim(const InflightClaim&) = delete;
+  InflightClaim& operator=(const InflightClaim&) = delete;
+
+ private:
+  const void* key_ = nullptr;
+  void* stream_ = nullptr;
+};
+// The error of a run that kBusy refuses.
+int inflight_busy(const char* what);
 
 // ---------------------------------------------------------------- grouped launch (host)
 // Between pie_hip_group_begin and pie_hip_group_end (group.hip) the groupable entry points

@@ -3,7 +3,7 @@
 // the results with the CPU oracle (oracle/oracle.c). TEST INFRASTRUCTURE.
 //
 //   emu_main <case>    case = norm | qk | silu | embed | rope | fused | decode | index | qkfused |
-//                      variants | fastdiv | attn | prefill | sample | group | all | big
+//                      variants | fastdiv | attn | prefill | cut | sample | group | all | big
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -632,6 +632,71 @@ static void case_attn_prefill(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int
   failures += !(worst <= 1.f);
 }
 
+// One request of `qo` query tokens over `kv` cached tokens, causal, with a plan whose items are cut.
+struct CutPrefill {
+  const int64_t Hq = 2, Hkv = 1, P = 16, D, kv, qo;
+  Buf<int32_t> qi{2}, ip{2}, ll{1}, idx, plan;
+  Buf<uint16_t> cache;
+  int64_t words = 0, items = 0, mb = 0, mw = 0, split[5] = {0, 0, 0, 0, 0};
+  CutPrefill(int64_t D_, int64_t kv_ = 790, int64_t qo_ = 3)
+      : D(D_), kv(kv_), qo(qo_), idx(pages()), plan(4096), cache(pages() * 2 * P * Hkv * D) {
+    qi[0] = ip[0] = 0;
+    qi[1] = (int32_t)qo;
+    ip[1] = (int32_t)pages();
+    ll[0] = (int32_t)(kv - (pages() - 1) * P);
+    for (int64_t i = 0; i < pages(); ++i) idx[i] = (int32_t)(pages() - 1 - i);
+    fill_normal(cache);
+    rc_ok(pie_hip_attention_prefill_split_plan(qi.p, ip.p, ll.p, 1, P, Hq, Hkv, D, 1, -1, 64, 1ll << 30, plan.p, 4096,
+                                               &words, &items, &mb, &mw, split),
+          "prefill_split_plan");
+    if (!split[1]) { printf("  nothing was cut\n"); ++failures; }
+  }
+  int64_t pages() const { return (kv + P - 1) / P; }
+  int64_t page() const { return 2 * P * Hkv * D; }
+  int run(const Buf<uint16_t>& q, Buf<uint16_t>& out, Buf<float>& scratch, const int64_t* sp, void* stream) {
+    return pie_hip_attention_prefill_split(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page(), Hkv * D, D, pages(),
+                                           qi.p, ip.p, idx.p, ll.p, Hq, Hkv, D, P, 1.f / sqrtf((float)D), 1, -1,
+                                           nullptr, nullptr, nullptr, plan.p, items, plan[4], sp, scratch.p,
+                                           (int64_t)scratch.n * 4, out.p, Hq * D, D, stream);
+  }
+  void check(const char* what, const Buf<uint16_t>& q, const Buf<uint16_t>& out) {
+    Buf<uint16_t> want(qo * Hq * D);
+    oracle_attention(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page(), Hkv * D, D, qi.p, ip.p, idx.p, ll.p,
+                     nullptr, nullptr, 1, -1, 1, Hq, Hkv, D, P, 1.0 / sqrt((double)D), want.p, Hq * D, D, nullptr,
+                     nullptr);
+    check_close(what, out.p, want.p, qo * Hq * D);
+  }
+};
+
+// Two host threads running one cut plan: the second run is made while the first is between its
+// launches (before its `at`-th), on its stream or another. The partial results are one run's
+// alone: the other takes the uncut items (head dim 128, whose plan also counts work, refuses another
+// stream's run), and both outputs are right.
+static void case_prefill_two_threads(int64_t D, int at, bool same_stream) {
+  printf("prefill, two threads on one cut plan: D=%lld launch %d %s stream\n", (long long)D, at,
+         same_stream ? "same" : "other");
+  CutPrefill c(D);
+  const size_t n = c.qo * c.Hq * D;
+  Buf<uint16_t> q1(n), q2(n), o1(n), o2(n);
+  Buf<float> scratch(c.split[4] / 4);
+  fill_normal(q1);
+  fill_normal(q2);
+  void *s1 = (void*)16, *s2 = same_stream ? s1 : (void*)32;
+  int launches = 0, rc2 = -1;
+  emu::on_launch = [&] {
+    if (++launches == at) rc2 = c.run(q2, o2, scratch, c.split, s2);
+  };
+  rc_ok(c.run(q1, o1, scratch, c.split, s1), "first run");
+  emu::on_launch = nullptr;
+  c.check("first run", q1, o1);
+  if (D == 128 && !same_stream) {
+    if (rc2 != PIE_HIP_EBUSY) { printf("  the overlapping run returned %d\n", rc2); ++failures; }
+  } else {
+    rc_ok(rc2, "second run");
+    c.check("second run", q2, o2);
+  }
+}
+
 // ---------------------------------------------------------------------------- sampling
 // Probabilities are multiples of 2^-30 (exact in the kernel's 2^-40 fixed point and in float64),
 // so kept sets and draws must match the oracle exactly; ties are forced in some rows.
@@ -881,6 +946,12 @@ int main(int argc, char** argv) {
     case_attn_prefill(1, 4, 2, 128, 16, 1400, 9, 2, false, -1, false, 64, 900);
     case_attn_prefill(1, 8, 2, 64, 8, 1300, 17, 1, false, 850, true, 64, 1000);
     case_attn_prefill(1, 4, 2, 256, 16, 1100, 40, 0, false, -1, false, 64, 800);
+  }
+  if (all || c == "cut") {
+    case_prefill_two_threads(64, 2, false);
+    case_prefill_two_threads(64, 2, true);
+    case_prefill_two_threads(128, 2, true);
+    case_prefill_two_threads(128, 2, false);
   }
   if (all || c == "group") {
     case_group(5, 4096, 1536, 40, false);  // 8 norm vectors per lane pair (NJ = 2)

@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <thread>
 #include <vector>
@@ -53,6 +54,7 @@ inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = (hipEvent_t)1; return hipSuccess; }
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 inline hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
   const char* e = getenv("EMU_CUS");
   *v = e ? atoi(e) : 1;  // few "CUs" so grid caps engage and grid-stride loops iterate
@@ -247,8 +249,17 @@ inline void global_load_lds(G src, L lds_base, unsigned size, int offset, int) {
   memcpy((char*)(void*)lds_base + offset + (size_t)ctx->lane * size, (const void*)src, size);
 }
 
+// Called before each launch (not those it makes itself): what another host thread may do there.
+inline std::function<void()> on_launch;
+
 template <typename K, typename... A>
 void launch(K kernel, dim3 grid, dim3 block, A... args) {
+  if (on_launch) {
+    const auto f = std::move(on_launch);
+    on_launch = nullptr;
+    f();
+    on_launch = f;
+  }
   const unsigned nt = block.x * block.y * block.z;
   if (nt % 64 != 0) { fprintf(stderr, "emu: block size %u not a multiple of 64\n", nt); abort(); }
   for (unsigned b = 0; b < grid.x * grid.y * grid.z; ++b) {

@@ -455,6 +455,38 @@ def test_prefill_cut_plan_captured_and_on_two_streams(dev, D):
             _tight(o, want, "two streams")
 
 
+@pytest.mark.parametrize("D", [64, 256])
+def test_prefill_run_beside_another_streams_takes_the_uncut_items(dev, D):
+    """While a cut plan's run is queued on one stream, a run on another leaves its partial results
+    alone: bit for bit the uncut items' output, and the queued run's is the cut items'."""
+    a = wl.attn_batch([6000, 9000], [20, 7], Hq=8, Hkv=2, D=D, page_size=16, seed=77)
+    pb = a["batch"]
+    w = attention.BatchPrefillWithPagedKVCacheWrapper(_workspace(dev), "NHD")
+    w.plan(pb.qo_indptr.to(dev), pb.kv_indptr.to(dev), pb.kv_indices.to(dev), pb.kv_last_page_len.to(dev), 8, 2, D,
+           16, causal=True)
+    q, cache, split = a["q"].to(dev), a["cache"].to(dev), w._plan["split"]
+    cut = w.run(q, cache)
+    n, split[1] = split[1], 0
+    uncut = w.run(q, cache)
+    split[1] = n
+    torch.cuda.synchronize()
+    assert n > 0 and not torch.equal(cut, uncut)
+    big = torch.ones((8192, 8192), dtype=torch.bfloat16, device=dev)
+    s1, s2, done = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.Event()
+    o1, o2 = torch.empty_like(q), torch.empty_like(q)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s1):
+        for _ in range(20):  # ~16 ms before the run on s1
+            torch.mm(big, big)
+        w.run(q, cache, out=o1)
+        done.record()
+    with torch.cuda.stream(s2):
+        w.run(q, cache, out=o2)
+    assert not done.query()
+    torch.cuda.synchronize()
+    assert torch.equal(o1, cut) and torch.equal(o2, uncut)
+
+
 def test_prefill_plan_in_use_on_another_stream_is_refused(dev):
     """The head-dim-128 kernel counts its work in the device plan, so two runs sharing a plan
     must not overlap: an eager run while the plan is still in use on another stream is refused
