@@ -1902,6 +1902,10 @@ __global__ __launch_bounds__(256) void attn_mask_kernel(const uint8_t* __restric
     if (qo_indptr[mid] <= j) lo = mid; else hi = mid - 1;
   }
   const int b = lo, q0 = qo_indptr[b], i = j - q0, qo_len = qo_indptr[b + 1] - q0;
+  if (i < 0 || i >= qo_len) {  // a token outside the batch (qo_indptr may start past 0): no mask row
+    if (threadIdx.x == 0) extent[j] = 0;
+    return;
+  }
   const int kv_len = kv_length(kv, b), nw = (kv_len + 31) / 32;
   const uint8_t* src = mask + reinterpret_cast<const int64_t*>(plan + plan[3])[b] + (int64_t)i * kv_len;
   uint32_t* dst = packed + reinterpret_cast<const int64_t*>(plan + plan[4])[b] + (int64_t)i * nw;

@@ -3,7 +3,7 @@
 // the results with the CPU oracle (oracle/oracle.c). TEST INFRASTRUCTURE.
 //
 //   emu_main <case>    case = norm | qk | silu | embed | rope | fused | decode | index | qkfused |
-//                      variants | fastdiv | attn | prefill | cut | sample | group | all | big
+//                      variants | fastdiv | attn | prefill | first | cut | sample | group | all | big
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -632,6 +632,44 @@ static void case_attn_prefill(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int
   failures += !(worst <= 1.f);
 }
 
+// A batch whose query tokens start past 0 (qo_indptr[0] > 0) and hold an empty request, under a custom
+// mask: the mask rows of its own tokens alone are packed, and the output of the others is left alone.
+static void case_prefill_first_token() {
+  printf("prefill, custom mask, qo_indptr from 3\n");
+  const int64_t B = 3, Hq = 2, Hkv = 1, D = 64, P = 16, T = 8, pages = 5, page = 2 * P * Hkv * D;
+  const int32_t qv[] = {3, 5, 5, 8}, iv[] = {0, 3, 4, 5}, lv[] = {8, 16, 7}, kv[] = {40, 16, 7};
+  Buf<int32_t> qi(B + 1), ip(B + 1), ll(B), idx(pages), plan(256), extent(T);
+  for (int b = 0; b <= B; ++b) { qi[b] = qv[b]; ip[b] = iv[b]; }
+  for (int b = 0; b < B; ++b) ll[b] = lv[b];
+  for (int i = 0; i < pages; ++i) idx[i] = pages - 1 - i;
+  int64_t moff[B] = {0, 2 * 40, 2 * 40}, words, items, mb, mw;
+  Buf<uint8_t> mask(2 * 40 + 3 * 7);
+  for (size_t i = 0; i < mask.n; ++i) mask[i] = i % 3 != 1;
+  rc_ok(pie_hip_attention_prefill_plan(qi.p, ip.p, ll.p, B, P, Hq, Hkv, D, 2, plan.p, 256, &words, &items, &mb, &mw),
+        "prefill_plan");
+  if (mb != (int64_t)mask.n) { printf("  mask bytes %lld\n", (long long)mb); ++failures; }
+  Buf<uint32_t> packed(mw), want_packed(mw);
+  for (size_t i = 0; i < want_packed.n; ++i) want_packed[i] = 0;
+  for (int b = 0, w0 = 0; b < B; w0 += (qv[b + 1] - qv[b]) * ((kv[b] + 31) / 32), ++b)
+    for (int i = 0; i < qv[b + 1] - qv[b]; ++i)
+      for (int t = 0; t < kv[b]; ++t)
+        want_packed[w0 + i * ((kv[b] + 31) / 32) + t / 32] |= (uint32_t)mask[moff[b] + i * kv[b] + t] << (t % 32);
+  rc_ok(pie_hip_attention_pack_mask(mask.p, plan.p, qi.p, ip.p, ll.p, B, P, mw, T, packed.p, extent.p, nullptr),
+        "pack_mask");
+  check_equal("packed mask", packed.p, want_packed.p, mw);
+  Buf<uint16_t> cache(pages * page), q(T * Hq * D), out(T * Hq * D), want(T * Hq * D);
+  fill_normal(cache);
+  fill_normal(q);
+  for (size_t i = 0; i < out.n; ++i) out[i] = want[i] = 0x4242;
+  rc_ok(pie_hip_attention_prefill(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page, Hkv * D, D, pages, qi.p, ip.p,
+                                  idx.p, ll.p, Hq, Hkv, D, P, 0.125f, 2, -1, nullptr, packed.p, extent.p, plan.p, items,
+                                  plan[4], out.p, Hq * D, D, nullptr),
+        "attention_prefill");
+  oracle_attention(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page, Hkv * D, D, qi.p, ip.p, idx.p, ll.p, mask.p,
+                   moff, 0, -1, B, Hq, Hkv, D, P, 0.125, want.p, Hq * D, D, nullptr, nullptr);
+  check_close("prefill from token 3", out.p, want.p, T * Hq * D);
+}
+
 // One request of `qo` query tokens over `kv` cached tokens, causal, with a plan whose items are cut.
 struct CutPrefill {
   const int64_t Hq = 2, Hkv = 1, P = 16, D, kv, qo;
@@ -947,6 +985,7 @@ int main(int argc, char** argv) {
     case_attn_prefill(1, 8, 2, 64, 8, 1300, 17, 1, false, 850, true, 64, 1000);
     case_attn_prefill(1, 4, 2, 256, 16, 1100, 40, 0, false, -1, false, 64, 800);
   }
+  if (all || c == "first") case_prefill_first_token();
   if (all || c == "cut") {
     case_prefill_two_threads(64, 2, false);
     case_prefill_two_threads(64, 2, true);

@@ -455,6 +455,27 @@ def test_prefill_cut_plan_captured_and_on_two_streams(dev, D):
             _tight(o, want, "two streams")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("custom", [False, True])
+def test_prefill_of_tokens_past_the_first(dev, D, custom):
+    """qo_indptr that starts past 0: the batch is rows 5.. of q, the rows before them are left alone."""
+    a = wl.attn_batch([40, 0, 700], [7, 0, 20], Hq=8, Hkv=2, D=D, page_size=16, seed=79)
+    pb = a["batch"]
+    mask = None
+    if custom:
+        n = int((pb.lens.to(torch.int64) * pb.seq_lens.to(torch.int64)).sum())
+        mask = torch.rand(n, generator=torch.Generator().manual_seed(5)) < 0.5
+    w = attention.BatchPrefillWithPagedKVCacheWrapper(_workspace(dev), "NHD")
+    w.plan((pb.qo_indptr + 5).to(dev), pb.kv_indptr.to(dev), pb.kv_indices.to(dev), pb.kv_last_page_len.to(dev), 8, 2,
+           D, 16, custom_mask=None if mask is None else mask.to(dev), causal=mask is None)
+    q = torch.cat([a["q"][:5], a["q"]]).to(dev)
+    out = torch.full_like(q, 3.0)
+    w.run(q, a["cache"].to(dev), out=out)
+    torch.cuda.synchronize()
+    assert bool((out[:5] == 3.0).all())
+    _tight(out[5:], _want(a, custom=None if mask is None else mask.numpy(), causal=mask is None), "tokens from 5")
+
+
 @pytest.mark.parametrize("D", [64, 256])
 def test_prefill_run_beside_another_streams_takes_the_uncut_items(dev, D):
     """While a cut plan's run is queued on one stream, a run on another leaves its partial results
