@@ -430,7 +430,8 @@ int pie_hip_attention_prefill(const pie_bf16* q, int64_t q_tok_stride, int64_t q
  * longest items cut, where that pays and plan_capacity (8 words more per piece) and the workspace
  * hold it: split[5] = {word of the cut items, their number (0: no cut), word of the merge list,
  * its entries, scratch bytes}. pie_hip_attention_prefill_split takes pie_hip_attention_prefill's
- * arguments, that array and 16-byte-aligned scratch. Runs of one plan share its scratch: for
+ * arguments, that array and 16-byte-aligned scratch; a cut plan runs at its own head_dim and
+ * num_kv_heads only (PIE_HIP_EINVAL otherwise). Runs of one plan share its scratch: for
  * head_dim 128 overlapping runs are refused as above; for 64 and 256 a run that is captured, or made
  * while another stream's run uses the scratch, runs the uncut items; so does, at any head_dim, one
  * made while another thread makes a run of the plan on the same stream.

@@ -1442,15 +1442,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill32_kernel(
 }
 
 // Combines the pieces of split items: work group x takes (merge entry, kv head) x and 512 / D of
-// its 128 rows.
+// its 128 rows. (A plan that attn_prefill_kernel could not use has no pieces: its NaN stays.)
 template <int D>
 __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
-    const int32_t* __restrict__ merges, int n_kv_heads, int G, const float* __restrict__ part_o,
+    const int32_t* __restrict__ plan, int merges_word, int n_kv_heads, int G, const float* __restrict__ part_o,
     const float* __restrict__ part_lse, uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs,
     const float* __restrict__ sinks) {
   constexpr int CH = D / 8;
+  if (plan[2] != plan_rows_word(D)) return;
   const int e = blockIdx.x / n_kv_heads, kvh = blockIdx.x - e * n_kv_heads;
-  const int32_t* m = merges + kPlanMergeWords * e;
+  const int32_t* m = plan + merges_word + kPlanMergeWords * e;
   const int row0 = m[0], q0 = m[1], rows = m[2] * G, slot = m[3], pieces = m[4];
   const int lane = threadIdx.x & 63, c = lane % CH;
   const int rl0 = blockIdx.y * (64 / CH);
@@ -1678,6 +1679,11 @@ struct PrefillSplit {
 // kSplitMinGain tokens: less than that the merge launch costs more than the cut saves.
 constexpr int64_t kSplitMinChunk = 256, kSplitMinGain = 512;
 
+// Bytes of the partial results of `pieces` pieces: kPrefillRows rows of D outputs and a log-sum-exp each.
+static int64_t prefill_scratch_bytes(int64_t pieces, int64_t num_kv_heads, int64_t head_dim) {
+  return pieces * num_kv_heads * kPrefillRows * (head_dim + 1) * 4;
+}
+
 static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr, const int32_t* kv_last_page_len,
                              int64_t batch, int64_t page_size, int64_t num_qo_heads, int64_t num_kv_heads,
                              int64_t head_dim, int32_t mode, int32_t* plan, int64_t plan_capacity,
@@ -1754,7 +1760,7 @@ static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr,
         if (n > 1) { pieces += n; ++cut; } else ++whole;
       }
       const int64_t all = words + kPlanItemWords * (pieces + whole) + kPlanMergeWords * cut;
-      const int64_t scratch = pieces * num_kv_heads * kPrefillRows * (head_dim + 1) * 4;
+      const int64_t scratch = prefill_scratch_bytes(pieces, num_kv_heads, head_dim);
       const int64_t masks = mode == 2 ? (wtotal * 4 + 15) / 16 * 16 + qo_indptr[batch] * 4ll : 0;
       if (all <= plan_capacity && (all * 4 + 15) / 16 * 16 + (masks + 15) / 16 * 16 + scratch <= split->workspace_bytes &&
           (pieces + whole) * num_kv_heads < (1ll << 31)) {
@@ -1878,7 +1884,7 @@ static void launch_prefill(const PrefillLaunch& a) {
                      a.extent, a.out, a.o_ts, a.o_hs, a.sinks, a.part_o, a.part_lse);
   if (a.n_merges)
     hipLaunchKernelGGL(attn_prefill_merge_kernel<D>, dim3(a.n_merges * a.Hkv, kPrefillRows / (512 / D)), dim3(256), 0,
-                       a.st, a.plan + a.merges_word, a.Hkv, a.G, a.part_o, a.part_lse, a.out, a.o_ts, a.o_hs, a.sinks);
+                       a.st, a.plan, a.merges_word, a.Hkv, a.G, a.part_o, a.part_lse, a.out, a.o_ts, a.o_hs, a.sinks);
 }
 
 // Packs the custom mask and finds every query token's visible extent: one work group per query token
@@ -1963,11 +1969,16 @@ static int attention_prefill_impl(
                   o_tok_stride % 8 == 0 && o_head_stride % 8 == 0,
               "attention_prefill: q/out pointers and strides must be 16-byte aligned");
   bool cut = split && split[1] > 0;
-  if (cut)
+  if (cut) {
     PIE_REQUIRE(split[0] > 0 && split[2] > split[0] && split[3] > 0 && split[1] * num_kv_heads < (1ll << 31) &&
                     scratch && aligned16(scratch) && split[4] > 0 && scratch_bytes >= split[4],
                 "attention_prefill: a split plan needs %lld bytes of 16-byte-aligned scratch, got %lld",
                 (long long)split[4], (long long)scratch_bytes);
+    // the pieces: the cut list without the items that stayed whole
+    PIE_REQUIRE(split[4] == prefill_scratch_bytes(split[1] - (num_items - split[3]), num_kv_heads, head_dim),
+                "attention_prefill: the split plan is for another head_dim or num_kv_heads than %lld, %lld",
+                (long long)head_dim, (long long)num_kv_heads);
+  }
   if (num_items == 0) return PIE_HIP_OK;
   // The head-dim-128 kernel counts its work in the plan's header words, so runs of one plan must not
   // overlap. The other head dims' runs may: one that overlaps another stream's (or is captured,

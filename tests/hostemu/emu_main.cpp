@@ -3,7 +3,7 @@
 // the results with the CPU oracle (oracle/oracle.c). TEST INFRASTRUCTURE.
 //
 //   emu_main <case>    case = norm | qk | silu | embed | rope | fused | decode | index | qkfused |
-//                      variants | fastdiv | attn | prefill | first | cut | sample | group | all | big
+//                      variants | fastdiv | attn | prefill | first | cut | mismatch | sample | group | all | big
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -735,6 +735,36 @@ static void case_prefill_two_threads(int64_t D, int at, bool same_stream) {
   }
 }
 
+// A cut plan belongs to its head dim and kv heads: a run at others is refused before it can write past
+// the scratch; and where the device plan is not the one the split array came with, the merge leaves the
+// NaN of the attention kernel in place.
+static void case_prefill_cut_plan_mismatch() {
+  printf("prefill, cut plans run at another head dim\n");
+  for (int64_t D : {64, 256})
+    for (int64_t D2 : {64, 128, 256}) {
+      if (D2 == D) continue;
+      CutPrefill c(D), c2(D2);
+      Buf<uint16_t> q(c.qo * c.Hq * D2), out(c.qo * c.Hq * D2);
+      Buf<float> scratch(c.split[4] / 4);
+      fill_normal(q);
+      memcpy(c2.plan.p, c.plan.p, c.words * 4);
+      const int rc = c2.run(q, out, scratch, c.split, nullptr);
+      if (rc != PIE_HIP_EINVAL) { printf("  plan for %lld run at %lld returned %d\n", (long long)D, (long long)D2, rc); ++failures; }
+    }
+  CutPrefill c(64), other(256);
+  const size_t n = c.qo * c.Hq * 64;
+  Buf<uint16_t> q(n), out(n);
+  Buf<float> scratch(c.split[4] / 4);
+  fill_normal(q);
+  for (size_t i = 0; i < n; ++i) out[i] = 0;
+  for (size_t i = 0; i < scratch.n; ++i) scratch[i] = 1.f;
+  memcpy(c.plan.p, other.plan.p, other.words * 4);
+  rc_ok(c.run(q, out, scratch, c.split, nullptr), "prefill_split");
+  size_t bad = 0;
+  for (size_t i = 0; i < n; ++i) bad += out[i] != 0x7fc0;
+  if (bad) { printf("  %zu of %zu outputs are not NaN\n", bad, n); ++failures; }
+}
+
 // ---------------------------------------------------------------------------- sampling
 // Probabilities are multiples of 2^-30 (exact in the kernel's 2^-40 fixed point and in float64),
 // so kept sets and draws must match the oracle exactly; ties are forced in some rows.
@@ -986,6 +1016,7 @@ int main(int argc, char** argv) {
     case_attn_prefill(1, 4, 2, 256, 16, 1100, 40, 0, false, -1, false, 64, 800);
   }
   if (all || c == "first") case_prefill_first_token();
+  if (all || c == "mismatch") case_prefill_cut_plan_mismatch();
   if (all || c == "cut") {
     case_prefill_two_threads(64, 2, false);
     case_prefill_two_threads(64, 2, true);
