@@ -512,8 +512,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 // the four waves of the work group take every fourth partial, kMergeBatch of them loaded at once
 // before the first is used, and meet in LDS. Partial s of the lane's row is
 // po[s * o_stride .. +8) (fp32, normalised) with log2-sum-exp pl[s * l_stride]. Every thread of the
-// work group calls it; wave 0 gets the row's weighted sum (acc), weight sum (L) and maximum (M,
-// -inf if no partial saw anything) of partials [0, ns); there is memory for room >= max(ns, 1).
+// work group calls it; wave 0 gets the row's weighted sum (acc, NaN if a partial is), weight sum (L)
+// and maximum (M, -inf if no partial saw anything) of partials [0, ns); there is memory for room >= max(ns, 1).
 // Bound: load latency. The partials are read in ns / 32 rounds of independent loads, and only the
 // splits that hold tokens: 3.0 us for one request of 1,000 tokens planned at 64 splits (32 heads,
 // 8 splits hold tokens) and 5.3 us for three of 16-32k tokens at 43; one wave reading every split
@@ -552,14 +552,15 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
       }
       mx = fmaxf(mx, ls[k]);
     }
-    if (mx == -INFINITY) continue;
-    const float f0 = fast_exp2(M - mx);
+    // with nothing seen yet every weight is 0; a NaN among the partials still has to reach the sum
+    const float ref = mx == -INFINITY ? 0.f : mx;
+    const float f0 = fast_exp2(M - ref);
     L *= f0;
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] *= f0;
 #pragma unroll
     for (int k = 0; k < kMergeBatch; ++k) {
-      const float f = fast_exp2(ls[k] - mx);
+      const float f = fast_exp2(ls[k] - ref);
       L += f;
       const float v[8] = {a[k].x, a[k].y, a[k].z, a[k].w, b[k].x, b[k].y, b[k].z, b[k].w};
 #pragma unroll
@@ -579,20 +580,19 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
     float mx = M;
 #pragma unroll
     for (int ww = 1; ww < 4; ++ww) mx = fmaxf(mx, sm[ww][lane][9]);
-    if (mx != -INFINITY) {
-      const float f0 = fast_exp2(M - mx);
-      L *= f0;
+    const float ref = mx == -INFINITY ? 0.f : mx;
+    const float f0 = fast_exp2(M - ref);
+    L *= f0;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] *= f0;
+    for (int e = 0; e < 8; ++e) acc[e] *= f0;
 #pragma unroll
-      for (int ww = 1; ww < 4; ++ww) {
-        const float f = fast_exp2(sm[ww][lane][9] - mx);
-        L = fmaf(sm[ww][lane][8], f, L);
+    for (int ww = 1; ww < 4; ++ww) {
+      const float f = fast_exp2(sm[ww][lane][9] - ref);
+      L = fmaf(sm[ww][lane][8], f, L);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] = fmaf(sm[ww][lane][e], f, acc[e]);
-      }
-      M = mx;
+      for (int e = 0; e < 8; ++e) acc[e] = fmaf(sm[ww][lane][e], f, acc[e]);
     }
+    M = mx;
   }
 }
 

@@ -508,6 +508,40 @@ def test_prefill_run_beside_another_streams_takes_the_uncut_items(dev, D):
     assert torch.equal(o1, cut) and torch.equal(o2, uncut)
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_nan_reaches_the_output_through_the_merge(dev, D):
+    """A NaN key makes every row that sees it NaN, and a NaN query of a prefill its own row, also where
+    the context is worked on in splits or pieces of which one, or every one, holds nothing else."""
+    ctx = [2500, 600]
+    a = wl.attn_batch(ctx, [1, 1], Hq=4, Hkv=2, D=D, page_size=16, seed=D)
+    pb, q, cache = a["batch"], a["q"].to(dev), a["cache"].to(dev)
+    t = [getattr(pb, n).to(dev) for n in ("kv_indptr", "kv_indices", "kv_last_page_len")]
+    w = attention.BatchDecodeWithPagedKVCacheWrapper(_workspace(dev), "NHD")
+    w.plan(*t, 4, 2, D, 16)
+    for splits in (1, 2, 4, 20):
+        w._plan["splits"] = splits
+        for pos in (0, 1000, 2500):
+            bad = cache.clone()
+            bad[int(pb.kv_indices[pos // 16]), 0, pos % 16, 0] = float("nan")
+            got = w.run(q, bad).float().isnan()
+            assert got[0, :2].all() and not got[0, 2:].any() and not got[1].any(), f"key {pos}, {splits} splits"
+    a = wl.attn_batch(ctx, [5, 3], Hq=4, Hkv=2, D=D, page_size=16, seed=D + 1)
+    pb, q, cache = a["batch"], a["q"].to(dev), a["cache"].to(dev)
+    w = attention.BatchPrefillWithPagedKVCacheWrapper(_workspace(dev), "NHD")
+    w.plan(pb.qo_indptr.to(dev), pb.kv_indptr.to(dev), pb.kv_indices.to(dev), pb.kv_last_page_len.to(dev), 4, 2, D,
+           16, causal=True)
+    assert w._plan["split"][1] > w._plan["items"]
+    for pos in (0, 1000, 2500):
+        bad = cache.clone()
+        bad[int(pb.kv_indices[pos // 16]), 0, pos % 16, 0] = float("nan")
+        got = w.run(q, bad).float().isnan()
+        assert got[:5, :2].all() and not got[:, 2:].any() and not got[5:].any(), f"prefill, key {pos}"
+    bad = q.clone()
+    bad[2, 3] = float("nan")
+    got = w.run(bad, cache).float().isnan()
+    assert got[2, 3].all() and int(got.sum()) == D, "prefill, query"
+
+
 def test_prefill_plan_in_use_on_another_stream_is_refused(dev):
     """The head-dim-128 kernel counts its work in the device plan, so two runs sharing a plan
     must not overlap: an eager run while the plan is still in use on another stream is refused
