@@ -2063,17 +2063,20 @@ __global__ __launch_bounds__(kSampThreads) void scaled_softmax_part_kernel(const
   const float T = temps[r];
   const bool greedy_row = T < greedy;
   const float c = greedy_row ? 1.f : 1.4426950408889634f / T;
-  float mx = -INFINITY, s = 0.f;
+  // ref: the finite maximum s is relative to. From the lowest float, a masked (-inf) logit adds 0 and
+  // the first finite one scales the empty sum by a finite factor, also at T = inf (c = 0, where -inf
+  // itself gives NaN).
+  float mx = -INFINITY, ref = -3.402823466e38f, s = 0.f;
   int am = 0x7fffffff;
   auto visit = [&](float x, int i) {
     if (x > mx) {
-      s = s * __builtin_amdgcn_exp2f((mx - x) * c);
-      mx = x;
+      s = s * __builtin_amdgcn_exp2f((ref - x) * c);
+      mx = ref = x;
       am = i;
     }
     // (a row of masked logits: its first entry, where the register-resident kernel gives that)
     if (first_masked && x == -INFINITY && mx == -INFINITY) am = min(am, i);
-    s += x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((x - mx) * c);
+    s += __builtin_amdgcn_exp2f((x - ref) * c);
   };
   const int nv = vec ? n / E : 0;
   int v = threadIdx.x;

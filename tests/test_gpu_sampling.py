@@ -413,3 +413,16 @@ def test_sliced_softmax(dev, B, V, dtype):
         err = (got[r].double() - want).abs() / (want + 1e-30)
         # fp32 sums and exponentials (2^-20 with the argument's rounding), then one bf16 rounding
         assert float(err[want > 1e-30].max()) <= (2.0**-8 if dtype == torch.bfloat16 else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sliced_softmax_of_an_infinite_temperature(dev, dtype):
+    """T = inf scales every finite logit to 0 (the uniform distribution) and -inf to NaN, as the
+    division logits / T does."""
+    B, V = 3, 151936
+    assert _lib.load().pie_hip_scaled_softmax_workspace(B, V, int(dtype == torch.bfloat16)) > 0
+    x = torch.randn((B, V), generator=torch.Generator(device=dev).manual_seed(5), device=dev).to(dtype)
+    x[2, V // 2] = -float("inf")
+    got = sampling.safe_scaled_softmax(x, torch.full((B,), float("inf"), device=dev)).float()
+    assert torch.allclose(got[:2], torch.full_like(got[:2], 1 / V), rtol=2.0**-8)
+    assert bool(got[2].isnan().all())
