@@ -260,7 +260,8 @@ class BatchPrefillWithPagedKVCacheWrapper:
         mask_off = nbytes
         ext_off = mask_off + (mwords.value * 4 + 15) // 16 * 16
         need = ext_off + T * 4 if mode == 2 else nbytes
-        scratch_off = (need + 15) // 16 * 16
+        # (on a 16-byte boundary of memory: the workspace itself may start off one)
+        scratch_off = need + -(self._workspace.data_ptr() + need) % 16
         if split[4] and scratch_off + split[4] > ws_bytes:
             split[1] = split[4] = 0
         if need > ws_bytes:

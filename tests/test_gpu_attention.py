@@ -542,6 +542,22 @@ def test_nan_reaches_the_output_through_the_merge(dev, D):
     assert got[2, 3].all() and int(got.sum()) == D, "prefill, query"
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_prefill_in_a_workspace_off_16_byte_alignment(dev, D):
+    """A workspace that starts 4 bytes past a 16-byte boundary serves a batch whose items are cut
+    (their partial results are placed on a boundary of their own) as it serves any other."""
+    a = wl.attn_batch([6000, 90], [20, 7], Hq=8, Hkv=2, D=D, page_size=16, seed=78)
+    pb = a["batch"]
+    ws = torch.zeros(WS_BYTES // 4 + 1, device=dev)[1:]
+    assert ws.data_ptr() % 16 == 4
+    w = attention.BatchPrefillWithPagedKVCacheWrapper(ws, "NHD")
+    w.plan(pb.qo_indptr.to(dev), pb.kv_indptr.to(dev), pb.kv_indices.to(dev), pb.kv_last_page_len.to(dev), 8, 2, D,
+           16, causal=True)
+    got = w.run(a["q"].to(dev), a["cache"].to(dev))
+    torch.cuda.synchronize()
+    _tight(got, _want(a), "unaligned workspace")
+
+
 def test_prefill_plan_in_use_on_another_stream_is_refused(dev):
     """The head-dim-128 kernel counts its work in the device plan, so two runs sharing a plan
     must not overlap: an eager run while the plan is still in use on another stream is refused
