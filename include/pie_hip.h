@@ -431,10 +431,10 @@ int pie_hip_attention_prefill(const pie_bf16* q, int64_t q_tok_stride, int64_t q
  * hold it: split[5] = {word of the cut items, their number (0: no cut), word of the merge list,
  * its entries, scratch bytes}. pie_hip_attention_prefill_split takes pie_hip_attention_prefill's
  * arguments, that array and 16-byte-aligned scratch; a cut plan runs at its own head_dim and
- * num_kv_heads only (PIE_HIP_EINVAL otherwise). Runs of one plan share its scratch: for
- * head_dim 128 overlapping runs are refused as above; for 64 and 256 a run that is captured, or made
- * while another stream's run uses the scratch, runs the uncut items; so does, at any head_dim, one
- * made while another thread makes a run of the plan on the same stream.
+ * num_kv_heads only (PIE_HIP_EINVAL otherwise), and at any mode and window_left. Runs of one plan
+ * share its scratch: for head_dim 128 overlapping runs are refused as above; for 64 and 256 a run
+ * that is captured, or made while another stream's run uses the scratch, runs the uncut items; so
+ * does, at any head_dim, one made while another thread makes a run of the plan on the same stream.
  */
 int pie_hip_attention_prefill_split_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
                                          const int32_t* kv_last_page_len, int64_t batch,

@@ -668,8 +668,12 @@ constexpr int kPlanQueueWord = 8, kPlanDoneWord = 7;
 // words per work item: request b, first packed row, the request's q0 (first query token),
 // qo_len, kv_len and first page-table slot, so the kernels' prologue reads one 32-byte item
 // instead of chasing b through qo_indptr / kv_indptr / kv_last_page_len; then, for an item split
-// over its kv range, the piece's index and 1 + its partial-result slot (0: not split)
+// over its kv range, the piece's index (kLastPiece set in the item's last) and 1 + its
+// partial-result slot (0: not split)
 constexpr int kPlanItemWords = 8;
+// The last piece ends where the item's kv range does, whatever mode and window the run has: pieces
+// planned for a shorter range than the run's are longer at the end, not short of it.
+constexpr int kLastPiece = 1 << 30;
 // words per merge entry of a split plan: first packed row, q0, qo_len, first slot, pieces
 constexpr int kPlanMergeWords = 8;
 
@@ -826,8 +830,8 @@ __global__ __launch_bounds__(256, prefill_groups<D>()) void attn_prefill_kernel(
   int kv_begin = window_left >= 0 ? max(0, kv_len - qo_len + row0 / G - window_left) & ~31 : 0;
   if (slot >= 0) {
     const int chunk = uniform(plan[kPlanChunkWord]);
-    kv_begin += piece * chunk;
-    kv_end = min(kv_end, kv_begin + chunk);
+    kv_begin += (piece & (kLastPiece - 1)) * chunk;
+    if (!(piece & kLastPiece)) kv_end = min(kv_end, kv_begin + chunk);
   }
   const int nw = (kv_len + 31) / 32;
   const uint32_t* mword = mode == 2 ? packed + word_off[b] + (int64_t)max(row_tok, 0) * nw : nullptr;
@@ -1805,7 +1809,7 @@ static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr,
       const int32_t w8[kPlanMergeWords] = {it.row0, it.q0, it.qo, slot, n, 0, 0, 0};
       memcpy(m, w8, sizeof(w8));
       m += kPlanMergeWords;
-      for (int32_t i = 0; i < n; ++i) { put(p, it, i, ++slot); p += kPlanItemWords; }
+      for (int32_t i = 0; i < n; ++i) { put(p, it, i + 1 < n ? i : i | kLastPiece, ++slot); p += kPlanItemWords; }
     }
   }
   return PIE_HIP_OK;

@@ -3,7 +3,7 @@
 // the results with the CPU oracle (oracle/oracle.c). TEST INFRASTRUCTURE.
 //
 //   emu_main <case>    case = norm | qk | silu | embed | rope | fused | decode | index | qkfused |
-//                      variants | fastdiv | attn | prefill | first | cut | mismatch | sample | group | all | big
+//                      variants | fastdiv | attn | prefill | first | range | cut | mismatch | sample | group | all | big
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -676,7 +676,7 @@ struct CutPrefill {
   Buf<int32_t> qi{2}, ip{2}, ll{1}, idx, plan;
   Buf<uint16_t> cache;
   int64_t words = 0, items = 0, mb = 0, mw = 0, split[5] = {0, 0, 0, 0, 0};
-  CutPrefill(int64_t D_, int64_t kv_ = 790, int64_t qo_ = 3)
+  CutPrefill(int64_t D_, int64_t kv_ = 790, int64_t qo_ = 3, int64_t window = -1)
       : D(D_), kv(kv_), qo(qo_), idx(pages()), plan(4096), cache(pages() * 2 * P * Hkv * D) {
     qi[0] = ip[0] = 0;
     qi[1] = (int32_t)qo;
@@ -684,24 +684,25 @@ struct CutPrefill {
     ll[0] = (int32_t)(kv - (pages() - 1) * P);
     for (int64_t i = 0; i < pages(); ++i) idx[i] = (int32_t)(pages() - 1 - i);
     fill_normal(cache);
-    rc_ok(pie_hip_attention_prefill_split_plan(qi.p, ip.p, ll.p, 1, P, Hq, Hkv, D, 1, -1, 64, 1ll << 30, plan.p, 4096,
+    rc_ok(pie_hip_attention_prefill_split_plan(qi.p, ip.p, ll.p, 1, P, Hq, Hkv, D, 1, window, 64, 1ll << 30, plan.p, 4096,
                                                &words, &items, &mb, &mw, split),
           "prefill_split_plan");
     if (!split[1]) { printf("  nothing was cut\n"); ++failures; }
   }
   int64_t pages() const { return (kv + P - 1) / P; }
   int64_t page() const { return 2 * P * Hkv * D; }
-  int run(const Buf<uint16_t>& q, Buf<uint16_t>& out, Buf<float>& scratch, const int64_t* sp, void* stream) {
+  int run(const Buf<uint16_t>& q, Buf<uint16_t>& out, Buf<float>& scratch, const int64_t* sp, void* stream,
+          int mode = 1, int64_t window = -1) {
     return pie_hip_attention_prefill_split(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page(), Hkv * D, D, pages(),
-                                           qi.p, ip.p, idx.p, ll.p, Hq, Hkv, D, P, 1.f / sqrtf((float)D), 1, -1,
+                                           qi.p, ip.p, idx.p, ll.p, Hq, Hkv, D, P, 1.f / sqrtf((float)D), mode, window,
                                            nullptr, nullptr, nullptr, plan.p, items, plan[4], sp, scratch.p,
                                            (int64_t)scratch.n * 4, out.p, Hq * D, D, stream);
   }
-  void check(const char* what, const Buf<uint16_t>& q, const Buf<uint16_t>& out) {
+  void check(const char* what, const Buf<uint16_t>& q, const Buf<uint16_t>& out, int mode = 1, int64_t window = -1) {
     Buf<uint16_t> want(qo * Hq * D);
     oracle_attention(q.p, Hq * D, D, cache.p, cache.p + P * Hkv * D, page(), Hkv * D, D, qi.p, ip.p, idx.p, ll.p,
-                     nullptr, nullptr, 1, -1, 1, Hq, Hkv, D, P, 1.0 / sqrt((double)D), want.p, Hq * D, D, nullptr,
-                     nullptr);
+                     nullptr, nullptr, mode, window, 1, Hq, Hkv, D, P, 1.0 / sqrt((double)D), want.p, Hq * D, D,
+                     nullptr, nullptr);
     check_close(what, out.p, want.p, qo * Hq * D);
   }
 };
@@ -732,6 +733,22 @@ static void case_prefill_two_threads(int64_t D, int at, bool same_stream) {
   } else {
     rc_ok(rc2, "second run");
     c.check("second run", q2, o2);
+  }
+}
+
+// A cut plan's run covers its own kv range whatever mode and window the plan was made for.
+static void case_prefill_cut_plan_other_range(int64_t D) {
+  printf("prefill, cut plans run at another mode or window: D=%lld\n", (long long)D);
+  struct { int64_t kv, qo, planned; int mode; int64_t window; } runs[] = {
+      {1100, 3, 780, 1, -1}, {1250, 300, -1, 0, -1}};
+  for (const auto& r : runs) {
+    CutPrefill c(D, r.kv, r.qo, r.planned);
+    const size_t n = r.qo * c.Hq * D;
+    Buf<uint16_t> q(n), out(n);
+    Buf<float> scratch(c.split[4] / 4);
+    fill_normal(q);
+    rc_ok(c.run(q, out, scratch, c.split, nullptr, r.mode, r.window), "prefill_split");
+    c.check("other range", q, out, r.mode, r.window);
   }
 }
 
@@ -1017,6 +1034,7 @@ int main(int argc, char** argv) {
   }
   if (all || c == "first") case_prefill_first_token();
   if (all || c == "mismatch") case_prefill_cut_plan_mismatch();
+  if (all || c == "range") case_prefill_cut_plan_other_range(64);
   if (all || c == "cut") {
     case_prefill_two_threads(64, 2, false);
     case_prefill_two_threads(64, 2, true);
