@@ -35,9 +35,10 @@ enum {
 /* Message describing the last nonzero return on this thread ("" if none). */
 const char* pie_hip_last_error(void);
 
-/* ABI version; bumped whenever a signature below changes (2: paged attention and sampling;
- * 3: attention sinks). */
-int pie_hip_abi_version(void);
+/* ABI version; bumped whenever a declaration below changes or is added (2: paged attention and
+ * sampling; 3: attention sinks; 4: cut prefill plans, sliced sampling and softmax). */
+#define PIE_HIP_ABI_VERSION 4
+int pie_hip_abi_version(void); /* of the library: PIE_HIP_ABI_VERSION where header and library match */
 
 /*
  * RMSNorm over the last dimension:

@@ -76,7 +76,7 @@ SIGNATURES: dict[str, list] = {
     "pie_hip_get_batch_indices_positions": [vp, vp, i64, i64, vp, vp, vp],
 }
 RETURNS_I64 = {"pie_hip_sample_workspace", "pie_hip_scaled_softmax_workspace"}
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 _lib: C.CDLL | None = None
 
@@ -101,6 +101,10 @@ def load() -> C.CDLL:
             f"pie_amd: kernel library {LIB_PATH} not built; run `python -m pie_amd.build` "
             "(there is no fallback path)")
     lib = C.CDLL(str(LIB_PATH))
+    # before anything else is looked up: another version may lack names or take other arguments
+    if lib.pie_hip_abi_version() != ABI_VERSION:
+        raise ImportError(f"pie_amd: {LIB_PATH} has ABI {lib.pie_hip_abi_version()}, "
+                          f"expected {ABI_VERSION}; rebuild it")
     lib.pie_hip_last_error.restype = C.c_char_p
     lib.pie_hip_last_error.argtypes = []
     lib.pie_hip_group_free.restype = None
@@ -109,9 +113,6 @@ def load() -> C.CDLL:
         fn = getattr(lib, name)
         fn.restype = C.c_int64 if name in RETURNS_I64 else C.c_int
         fn.argtypes = argtypes
-    if lib.pie_hip_abi_version() != ABI_VERSION:
-        raise ImportError(f"pie_amd: {LIB_PATH} has ABI {lib.pie_hip_abi_version()}, "
-                          f"expected {ABI_VERSION}; rebuild it")
     _lib = lib
     _bind_fast(lib)
     return lib

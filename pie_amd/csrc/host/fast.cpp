@@ -28,10 +28,10 @@ namespace {
 
 // The C ABI of the kernel library the Python binding loaded (bind()).
 #define PIE_ENTRY_POINTS(X)                                                                       \
-  X(pie_hip_rmsnorm) X(pie_hip_gemma_rmsnorm) X(pie_hip_fused_add_rmsnorm)                        \
-  X(pie_hip_gemma_fused_add_rmsnorm) X(pie_hip_silu_and_mul) X(pie_hip_gelu_tanh_and_mul)         \
-  X(pie_hip_embedding) X(pie_hip_qk_rmsnorm_rope_append) X(pie_hip_attention_decode)              \
-  X(pie_hip_attention_prefill_split)
+  X(pie_hip_abi_version) X(pie_hip_rmsnorm) X(pie_hip_gemma_rmsnorm)                              \
+  X(pie_hip_fused_add_rmsnorm) X(pie_hip_gemma_fused_add_rmsnorm) X(pie_hip_silu_and_mul)         \
+  X(pie_hip_gelu_tanh_and_mul) X(pie_hip_embedding) X(pie_hip_qk_rmsnorm_rope_append)             \
+  X(pie_hip_attention_decode) X(pie_hip_attention_prefill_split)
 struct Lib {
 #define X(name) decltype(&::name) name = nullptr;
   PIE_ENTRY_POINTS(X)
@@ -431,7 +431,8 @@ PyObject* attention_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // bind({entry point name: address}, check): the loaded library's functions, and check(name, code)
-// raising the library's error of a call that returned code
+// raising the library's error of a call that returned code. The calls below are compiled against one
+// version of the C ABI, so a library of another is refused (ImportError).
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 2 || !PyDict_CheckExact(a[0]) || !PyCallable_Check(a[1])) {
     PyErr_SetString(PyExc_TypeError, "bind: a dict of entry point addresses and the error check");
@@ -451,6 +452,12 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   PIE_ENTRY_POINTS(X)
 #undef X
+  const int version = next.pie_hip_abi_version();
+  if (version != PIE_HIP_ABI_VERSION) {
+    PyErr_Format(PyExc_ImportError, "pie_amd: the native call path is built for ABI %d, the library has %d; rebuild it",
+                 PIE_HIP_ABI_VERSION, version);
+    return nullptr;
+  }
   lib = next;
   Py_INCREF(a[1]);
   Py_XSETREF(on_error, a[1]);

@@ -102,6 +102,26 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         _lib.load()
 
 
+def test_a_library_of_another_abi_is_refused_before_its_names_are_looked_up(monkeypatch, tmp_path):
+    src, old = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text(f"int pie_hip_abi_version(void) {{ return {_lib.ABI_VERSION - 1}; }}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(old)], check=True)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", old)
+    with pytest.raises(ImportError, match="rebuild it"):
+        _lib.load()
+
+
+def test_native_call_path_refuses_a_library_of_another_abi():
+    addr = _lib._addresses(_lib.load())
+    other = C.CFUNCTYPE(C.c_int)(lambda: _lib.ABI_VERSION - 1)
+    try:
+        with pytest.raises(ImportError, match="rebuild it"):
+            _lib.fast.bind({**addr, "pie_hip_abi_version": C.cast(other, C.c_void_p).value}, _lib._check_rc)
+    finally:
+        _lib.fast.bind(addr, _lib._check_rc)
+
+
 def test_integration_installs_flashinfer_namespace():
     import importlib
     import sys
