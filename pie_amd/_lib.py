@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes as C
 import os
 import re
+import warnings
 from pathlib import Path
 
 _PKG = Path(__file__).resolve().parent
@@ -119,8 +120,8 @@ def load() -> C.CDLL:
 
 
 # The native call path of the small ops (csrc/host/fast.cpp), bound to the loaded library; None
-# until load() and where the module is not built. Its functions return None for a call that the
-# Python wrappers' general path has to handle, and raise an error of the launch itself.
+# until load() and where the module cannot be imported (a warning says so). Its functions return None
+# for a call that the Python wrappers' general path has to handle, and raise an error of the launch itself.
 fast = None
 
 
@@ -128,7 +129,9 @@ def _bind_fast(lib: C.CDLL) -> None:
     global fast
     try:
         from . import _fast
-    except ImportError:
+    except ImportError as e:
+        warnings.warn(f"pie_amd: no native call path, small ops take the slower general path: {e}",
+                      RuntimeWarning, stacklevel=3)
         return
     _fast.bind(_addresses(lib), _check_rc)
     fast = _fast

@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import warnings
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -64,7 +65,7 @@ def build(verbose: bool = False, out: Path | None = None, defines: tuple[str, ..
     fast = None
     if not defines and out is None:
         pool = cf.ThreadPoolExecutor(max_workers=1)
-        fast = pool.submit(build_fast, verbose)  # beside the kernels
+        fast = pool.submit(_try_build_fast, verbose)  # beside the kernels
         pool.shutdown(wait=False)
     srcs = sorted(CSRC.glob("*.hip"))
     if not srcs:
@@ -84,6 +85,16 @@ def build(verbose: bool = False, out: Path | None = None, defines: tuple[str, ..
         build_probe(verbose)
         fast.result()
     return lib
+
+
+def _try_build_fast(verbose: bool) -> None:
+    """build_fast, which the kernels and the C ABI do without: a failure leaves no module and warns."""
+    try:
+        build_fast(verbose)
+    except (RuntimeError, ImportError, OSError) as e:
+        FAST_LIB.unlink(missing_ok=True)
+        warnings.warn(f"pie_amd: the native call path was not built, small ops take the slower general path: {e}",
+                      RuntimeWarning, stacklevel=2)
 
 
 def build_fast(verbose: bool = False) -> Path:

@@ -122,6 +122,36 @@ def test_native_call_path_refuses_a_library_of_another_abi():
         _lib.fast.bind(addr, _lib._check_rc)
 
 
+def test_build_goes_on_without_the_native_call_path(monkeypatch, tmp_path):
+    """The library needs neither a host compiler nor torch: where the module does not compile, the
+    build says so and leaves none (not an older one) behind."""
+    from pie_amd import build
+    src, lib, kernels = tmp_path / "fast.cpp", tmp_path / "_fast.so", tmp_path / "lib.so"
+    src.write_text("#error no\n")
+    lib.write_text("older")
+    (tmp_path / "k.hip").write_text("")
+    obj = tmp_path / "k.o"
+    subprocess.run(["gcc", "-c", "-x", "c", "/dev/null", "-o", str(obj)], check=True)
+    for name, value in dict(FAST_SRC=src, FAST_LIB=lib, LIB=kernels, CSRC=tmp_path, BUILD=tmp_path / "b",
+                            _compile=lambda *a: obj, build_probe=lambda *a: None).items():
+        monkeypatch.setattr(build, name, value)
+    with pytest.warns(RuntimeWarning, match="native call path was not built"):
+        assert build.build() == kernels
+    assert kernels.exists() and not lib.exists()
+
+
+def test_a_native_call_path_that_does_not_import_is_reported(monkeypatch):
+    import sys
+    import pie_amd
+    _lib.load()
+    monkeypatch.setattr(_lib, "fast", None)
+    monkeypatch.delattr(pie_amd, "_fast", raising=False)
+    monkeypatch.setitem(sys.modules, "pie_amd._fast", None)  # import raises
+    with pytest.warns(RuntimeWarning, match="no native call path"):
+        _lib._bind_fast(_lib._lib)
+    assert _lib.fast is None
+
+
 def test_integration_installs_flashinfer_namespace():
     import importlib
     import sys
