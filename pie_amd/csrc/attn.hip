@@ -509,8 +509,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 }
 
 // Sums partial results of 64 / (D/8) output rows, one row per group of D/8 lanes, each lane 8 dims;
-// the four waves of the work group take every fourth partial, kMergeBatch of them loaded at once
-// before the first is used, and meet in LDS. Partial s of the lane's row is
+// the four waves of the work group take every fourth partial, KB of them loaded at once before the
+// first is used, and meet in LDS. Partial s of the lane's row is
 // po[s * o_stride .. +8) (fp32, normalised) with log2-sum-exp pl[s * l_stride]. Every thread of the
 // work group calls it; wave 0 gets the row's weighted sum (acc, NaN if a partial is), weight sum (L)
 // and maximum (M, -inf if no partial saw anything) of partials [0, ns); there is memory for room >= max(ns, 1).
@@ -518,8 +518,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 // splits that hold tokens: 3.0 us for one request of 1,000 tokens planned at 64 splits (32 heads,
 // 8 splits hold tokens) and 5.3 us for three of 16-32k tokens at 43; one wave reading every split
 // in turn took 27.9 us at either.
-constexpr int kMergeBatch = 8;
-template <int D>
+template <int D, int KB>
 __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int64_t o_stride,
                                                const float* __restrict__ pl, int64_t l_stride, int ns,
                                                int room, float (&acc)[8], float& L, float& M) {
@@ -532,12 +531,12 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
   // The first round's loads do not wait for ns (which may itself be in flight): partials [ns, room)
   // are memory, but hold nothing, and count as zero.
-  for (int s0 = w; s0 == w || s0 < ns; s0 += 4 * kMergeBatch) {
+  for (int s0 = w; s0 == w || s0 < ns; s0 += 4 * KB) {
     const int top = (s0 == w ? room : ns) - 1;
-    float4 a[kMergeBatch], b[kMergeBatch];
-    float ls[kMergeBatch];
+    float4 a[KB], b[KB];
+    float ls[KB];
 #pragma unroll
-    for (int k = 0; k < kMergeBatch; ++k) {
+    for (int k = 0; k < KB; ++k) {
       const int s = min(s0 + 4 * k, top);
       ls[k] = pl[s * l_stride];
       a[k] = *reinterpret_cast<const float4*>(po + s * o_stride);
@@ -545,7 +544,7 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
     }
     float mx = M;
 #pragma unroll
-    for (int k = 0; k < kMergeBatch; ++k) {
+    for (int k = 0; k < KB; ++k) {
       if (s0 + 4 * k >= ns) {
         ls[k] = -INFINITY;
         a[k] = b[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -559,7 +558,7 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] *= f0;
 #pragma unroll
-    for (int k = 0; k < kMergeBatch; ++k) {
+    for (int k = 0; k < KB; ++k) {
       const float f = fast_exp2(ls[k] - ref);
       L += f;
       const float v[8] = {a[k].x, a[k].y, a[k].z, a[k].w, b[k].x, b[k].y, b[k].z, b[k].w};
@@ -597,8 +596,10 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ po, int
 }
 
 // Combines the partial results of each (request, head): one work group per request and 512 / D
-// heads. Splits past the end of the request's kv range wrote nothing and are not read.
-template <int D>
+// heads. Splits past the end of the request's kv range wrote nothing and are not read. KB: plans of at
+// most four splits need one load per wave; with eight (seven of them repeats of it) a decode layer of 45
+// requests at 3 splits took 69.1 us, 68.0 with one.
+template <int D, int KB>
 __global__ __launch_bounds__(256) void attn_merge_kernel(PagedKV kv, int window_left, int Hq, int splits,
                                                          const float* __restrict__ part_o,
                                                          const float* __restrict__ part_lse,
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(PagedKV kv, int window_
   const int ns = split_count(len, splits);
   const int64_t first = (int64_t)b * splits * Hq + hl;
   float acc[8], L, M;
-  merge_partials<D>(part_o + first * D + 8 * c, (int64_t)Hq * D, part_lse + first, Hq, ns, splits, acc, L, M);
+  merge_partials<D, KB>(part_o + first * D + 8 * c, (int64_t)Hq * D, part_lse + first, Hq, ns, splits, acc, L, M);
   if (threadIdx.x >= 64 || hq >= Hq) return;
   if (M != -INFINITY) L += sink_mass(sinks, hq, M);
   const float inv = L > 0.f ? 1.f / L : 0.f;
@@ -1464,7 +1465,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
   const int64_t first = ((int64_t)slot * n_kv_heads + kvh) * kPrefillRows + (R - row0);
   const int64_t step = (int64_t)n_kv_heads * kPrefillRows;
   float acc[8], L, M;
-  merge_partials<D>(part_o + first * D + 8 * c, step * D, part_lse + first, step, pieces, pieces, acc, L, M);
+  merge_partials<D, 8>(part_o + first * D + 8 * c, step * D, part_lse + first, step, pieces, pieces, acc, L, M);
   if (threadIdx.x >= 64 || row0 + rl0 + lane / CH >= rows) return;
   const int tok = R / G, hq = kvh * G + (R - tok * G);
   if (M != -INFINITY) L += sink_mass(sinks, hq, M);
@@ -1537,8 +1538,9 @@ static void launch_decode(hipStream_t st, const uint16_t* q, int64_t q_ts, int64
   hipLaunchKernelGGL(attn_decode_kernel<D>, dim3(B * splits * Hkv), dim3(256), 0, st, q, q_ts, q_hs, kv,
                      B, G, Hq, sl2, splits, window_left, out, o_ts, o_hs, po, pl, sinks);
   if (splits > 1)
-    hipLaunchKernelGGL(attn_merge_kernel<D>, dim3(B, (Hq + 64 / (D / 8) - 1) / (64 / (D / 8))), dim3(256), 0,
-                       st, kv, window_left, Hq, splits, po, pl, out, o_ts, o_hs, sinks);
+    hipLaunchKernelGGL((splits <= 4 ? attn_merge_kernel<D, 1> : attn_merge_kernel<D, 8>),
+                       dim3(B, (Hq + 64 / (D / 8) - 1) / (64 / (D / 8))), dim3(256), 0, st, kv, window_left, Hq, splits,
+                       po, pl, out, o_ts, o_hs, sinks);
 }
 
 static int attention_decode_impl(
