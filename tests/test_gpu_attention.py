@@ -416,9 +416,9 @@ def test_prefill_items_cut_over_kv(dev, D, Hq, Hkv, P, mode):
 
 @pytest.mark.parametrize("D", [64, 128, 256])
 def test_prefill_cut_plan_captured_and_on_two_streams(dev, D):
-    """A cut plan's partial results are shared by its runs. Head dims 64 and 256: a captured run,
-    and one made while another stream's run is in flight, take the uncut items, so both give the
-    eager result up to rounding; head dim 128 replays the cut run and refuses the overlap."""
+    """A cut plan's partial results are shared by its runs. Captured runs (head dims 64 and 256: of the
+    uncut items; 128: of the cut ones) replay to the eager result up to rounding, and so do, for 64 and
+    256, runs issued in turn on two streams, whichever items each of them takes."""
     a = wl.attn_batch([6000, 9000], [20, 7], Hq=8, Hkv=2, D=D, page_size=16, seed=77)
     pb = a["batch"]
     w = attention.BatchPrefillWithPagedKVCacheWrapper(_workspace(dev), "NHD")

@@ -38,6 +38,17 @@ def _both(monkeypatch, call):
         assert torch.equal(g.view(torch.int16), w.view(torch.int16))
 
 
+def _both_refuse(monkeypatch, call):
+    """call() raises the same exception with the native path and without it."""
+    with pytest.raises(Exception) as got:
+        call()
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "fast", None)
+        with pytest.raises(Exception) as want:
+            call()
+    assert got.type is want.type and str(got.value) == str(want.value)
+
+
 def _rows(dev, kind, n, cols):
     if kind == "2d":
         return _x(dev, n, cols)
@@ -67,6 +78,11 @@ def test_row_ops(dev, monkeypatch, kind, n, cols):
         _both(monkeypatch, lambda: f2(x, r, w, 1, out=new(), residual_out=new()))
     out = torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
     assert ops.rmsnorm(x, w, 1e-5, out=out) is out
+    wide = torch.empty((*x.shape[:-1], cols + 1), dtype=torch.bfloat16, device=dev)
+    for f in (lambda: ops.rmsnorm(x, w[1:]), lambda: ops.rmsnorm(x.float(), w), lambda: ops.rmsnorm(x, w.cpu()),
+              lambda: ops.rmsnorm(x, w, 1e-5, out=wide), lambda: ops.add_rms_norm(x, wide, w),
+              lambda: ops.silu_and_mul(wide if cols % 2 == 0 else x), lambda: ops.silu_and_mul(x.cpu())):
+        _both_refuse(monkeypatch, f)
     if cols % 2 == 0:
         _both(monkeypatch, lambda: ops.silu_and_mul(x))
         _both(monkeypatch, lambda: ops.gelu_tanh_and_mul(x))
@@ -110,8 +126,7 @@ def test_prologue_and_attention(dev, monkeypatch, layout, as_pair):
         out = torch.empty_like(qs)
         assert w.run(qs, kv, out=out) is out
         for bad in (qs[:2], qs.float(), qs.cpu(), qs[:, :, ::2]):
-            with pytest.raises((ValueError, RuntimeError)):
-                w.run(bad, kv)
+            _both_refuse(monkeypatch, lambda: w.run(bad, kv))
 
 
 def test_modes_and_subclasses_take_the_general_path(dev):

@@ -341,49 +341,48 @@ def test_sample_one_read_and_fallbacks(dev, mode, case):
     assert (got == want).all(), f"{got} vs {want}"
 
 
-def _one_launch(probs, mode, **kw):
+def _one_launch(probs, mode, top_p=None):
     """The draw by the one-launch entry point (no workspace)."""
     B, V = probs.shape
     out = torch.empty(B, dtype=torch.int32, device=probs.device)
     p = lambda t: t.data_ptr() if t is not None else None
-    _lib.call("pie_hip_sample", probs.data_ptr(), probs.stride(0), B, V, B, None, mode, p(kw.get("top_k")), 0,
-              p(kw.get("top_p")), 0.0, p(kw.get("min_p")), 0.0, None, C.c_uint64(11), C.c_uint64(5), out.data_ptr(),
+    _lib.call("pie_hip_sample", probs.data_ptr(), probs.stride(0), B, V, B, None, mode, None, 0,
+              p(top_p), 0.0, None, 0.0, None, C.c_uint64(11), C.c_uint64(5), out.data_ptr(),
               torch.cuda.current_stream().cuda_stream)
     return out
 
 
 @pytest.mark.parametrize("B,V", [(1, 65536), (2, 70003), (9, 151936), (16, 100277), (33, 128256), (64, 65539)])
-@pytest.mark.parametrize("kind", ["peaked", "flat", "ties", "sparse"])
+@pytest.mark.parametrize("kind", ["peaked", "flat", "ties", "sparse", "block"])
 def test_sliced_draws_equal_the_one_launch(dev, B, V, kind):
     """Few long rows of top_p and plain sampling run over several work groups per row: the same
-    tokens as one work group per row (the other samplers keep it), rows of few and of all tokens kept, ties, and mostly zero rows."""
+    tokens as one work group per row, for rows of few and of all tokens kept, ties, mostly zero rows, and
+    rows whose kept tokens lie together, more than one wave's share of a slice's list holds. (The other
+    samplers have no sliced form.)"""
     print(f"sliced draws B={B} V={V} {kind}", flush=True)
     assert _lib.load().pie_hip_sample_workspace(B, V, 1) > 0
     assert (_lib.load().pie_hip_sample_workspace(B, V, 0) > 0) == (B <= 32)
+    assert all(_lib.load().pie_hip_sample_workspace(B, V, mode) == 0 for mode in (2, 3, 4))
     g = torch.Generator(device=dev).manual_seed(B + V)
-    x = torch.randn((B, V), generator=g, device=dev) * {"peaked": 4.0, "flat": 0.01, "ties": 1.0, "sparse": 2.0}[kind]
+    scale = {"peaked": 4.0, "flat": 0.01, "ties": 1.0, "sparse": 2.0, "block": 0.01}[kind]
+    x = torch.randn((B, V), generator=g, device=dev) * scale
     if kind == "ties":
         x = x.round()
     if kind == "sparse":
         x[:, 7:-9] = -float("inf")
         x[0] = -float("inf")
         x[0, V // 2] = 0.0
+    if kind == "block":
+        x[:, :V // 3] = x[:, V // 3 + 3000:] = -float("inf")
     probs = torch.softmax(x, -1)
     if kind == "sparse" and B > 1:
         probs[1] = 0.0  # nothing to draw
-    u = lambda: torch.rand(B, generator=g, device=dev)
-    tk = (1 + 300 * u()).int()
-    tk[-1] = 0
+    tp = torch.rand(B, generator=g, device=dev)
+    if kind == "block":
+        tp = 0.9 + 0.1 * tp
     kw = dict(seed=11, offset=5)
-    tp, mp = u(), 0.5 * u()
-    for got, want in (
-            (sampling.sampling_from_probs(probs, **kw), _one_launch(probs, 0)),
-            (sampling.top_p_sampling_from_probs(probs, tp, **kw), _one_launch(probs, 1, top_p=tp)),
-            (sampling.top_k_sampling_from_probs(probs, tk, **kw), _one_launch(probs, 2, top_k=tk)),
-            (sampling.min_p_sampling_from_probs(probs, mp, **kw), _one_launch(probs, 3, min_p=mp)),
-            (sampling.top_k_top_p_sampling_from_probs(probs, tk, tp, **kw),
-             _one_launch(probs, 4, top_k=tk, top_p=tp))):
-        assert torch.equal(got, want)
+    assert torch.equal(sampling.sampling_from_probs(probs, **kw), _one_launch(probs, 0))
+    assert torch.equal(sampling.top_p_sampling_from_probs(probs, tp, **kw), _one_launch(probs, 1, top_p=tp))
 
 
 @pytest.mark.parametrize("B,V", [(1, 131080), (5, 140003), (9, 151936), (64, 131073)])
