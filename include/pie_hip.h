@@ -425,17 +425,18 @@ int pie_hip_attention_prefill(const pie_bf16* q, int64_t q_tok_stride, int64_t q
 /*
  * The prefill form with items cut over their kv range, for batches that would leave most of the
  * chip idle (a few query tokens over long contexts). pie_hip_attention_prefill_split_plan takes the
- * plan's arguments, the run's window_left, the device's compute units (0: 256) and the bytes of
- * the workspace that will hold the plan, then (mode 2) the packed mask and the extents, each
- * 16-byte aligned, then the run's scratch. It writes the same plan and, after it, a list with the
- * longest items cut, where that pays and plan_capacity (8 words more per piece) and the workspace
- * hold it: split[5] = {word of the cut items, their number (0: no cut), word of the merge list,
- * its entries, scratch bytes}. pie_hip_attention_prefill_split takes pie_hip_attention_prefill's
- * arguments, that array and 16-byte-aligned scratch; a cut plan runs at its own head_dim and
- * num_kv_heads only (PIE_HIP_EINVAL otherwise), and at any mode and window_left. Runs of one plan
- * share its scratch: for head_dim 128 overlapping runs are refused as above; for 64 and 256 a run
- * that is captured, or made while another stream's run uses the scratch, runs the uncut items; so
- * does, at any head_dim, one made while another thread makes a run of the plan on the same stream.
+ * plan's arguments, the run's window_left, the device's compute units (0: 256) and the bytes of the
+ * workspace that will hold the plan, then (mode 2) the packed mask and the extents, each 16-byte
+ * aligned, then the run's scratch. It writes the same plan and, after it, a list with the longest
+ * items cut, where that pays and plan_capacity (8 words more per piece) and the workspace hold it:
+ * split[7] = {word of the cut items, their number (0: no cut), word of the merge list, its entries,
+ * scratch bytes, mode, window_left (-1: none)}. pie_hip_attention_prefill_split takes
+ * pie_hip_attention_prefill's arguments, that array and 16-byte-aligned scratch; a cut plan runs at
+ * its own head_dim and num_kv_heads only (PIE_HIP_EINVAL otherwise); at another mode or window_left
+ * its uncut items run. Runs of one plan share its scratch: for head_dim 128 overlapping runs are
+ * refused as above; for 64 and 256 a run that is captured, or made while another stream's run uses
+ * the scratch, runs the uncut items; so does, at any head_dim, one made while another thread makes
+ * a run of the plan on the same stream.
  */
 int pie_hip_attention_prefill_split_plan(const int32_t* qo_indptr, const int32_t* kv_indptr,
                                          const int32_t* kv_last_page_len, int64_t batch,

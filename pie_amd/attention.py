@@ -242,7 +242,7 @@ class BatchPrefillWithPagedKVCacheWrapper:
         cap = 16 + 8 * n_items + 4 * batch + 8 + 8 * (2 * n_items + 4 * (cus or 256))
         plan = np.empty(cap, dtype=np.int32)
         words, items, mbytes, mwords = C.c_int64(0), C.c_int64(0), C.c_int64(0), C.c_int64(0)
-        split = (C.c_int64 * 5)()
+        split = (C.c_int64 * 7)()
         _lib.call("pie_hip_attention_prefill_split_plan", qo_h.data_ptr(), kv_h.data_ptr(), ll_h.data_ptr(),
                   batch, page_size, num_qo_heads, num_kv_heads, head_dim_qk, mode, window_left, cus, ws_bytes,
                   plan.ctypes.data, cap, C.byref(words), C.byref(items), C.byref(mbytes), C.byref(mwords), split)

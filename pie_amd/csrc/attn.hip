@@ -669,12 +669,8 @@ constexpr int kPlanQueueWord = 8, kPlanDoneWord = 7;
 // words per work item: request b, first packed row, the request's q0 (first query token),
 // qo_len, kv_len and first page-table slot, so the kernels' prologue reads one 32-byte item
 // instead of chasing b through qo_indptr / kv_indptr / kv_last_page_len; then, for an item split
-// over its kv range, the piece's index (kLastPiece set in the item's last) and 1 + its
-// partial-result slot (0: not split)
+// over its kv range, the piece's index and 1 + its partial-result slot (0: not split)
 constexpr int kPlanItemWords = 8;
-// The last piece ends where the item's kv range does, whatever mode and window the run has: pieces
-// planned for a shorter range than the run's are longer at the end, not short of it.
-constexpr int kLastPiece = 1 << 30;
 // words per merge entry of a split plan: first packed row, q0, qo_len, first slot, pieces
 constexpr int kPlanMergeWords = 8;
 
@@ -831,8 +827,8 @@ __global__ __launch_bounds__(256, prefill_groups<D>()) void attn_prefill_kernel(
   int kv_begin = window_left >= 0 ? max(0, kv_len - qo_len + row0 / G - window_left) & ~31 : 0;
   if (slot >= 0) {
     const int chunk = uniform(plan[kPlanChunkWord]);
-    kv_begin += (piece & (kLastPiece - 1)) * chunk;
-    if (!(piece & kLastPiece)) kv_end = min(kv_end, kv_begin + chunk);
+    kv_begin += piece * chunk;
+    kv_end = min(kv_end, kv_begin + chunk);
   }
   const int nw = (kv_len + 31) / 32;
   const uint32_t* mword = mode == 2 ? packed + word_off[b] + (int64_t)max(row_tok, 0) * nw : nullptr;
@@ -1811,7 +1807,7 @@ static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr,
       const int32_t w8[kPlanMergeWords] = {it.row0, it.q0, it.qo, slot, n, 0, 0, 0};
       memcpy(m, w8, sizeof(w8));
       m += kPlanMergeWords;
-      for (int32_t i = 0; i < n; ++i) { put(p, it, i + 1 < n ? i : i | kLastPiece, ++slot); p += kPlanItemWords; }
+      for (int32_t i = 0; i < n; ++i) { put(p, it, i, ++slot); p += kPlanItemWords; }
     }
   }
   return PIE_HIP_OK;
@@ -1846,6 +1842,8 @@ extern "C" int pie_hip_attention_prefill_split_plan(
   split[2] = sp.merges_word;
   split[3] = sp.num_merges;
   split[4] = sp.scratch_bytes;
+  split[5] = mode;
+  split[6] = std::max<int64_t>(window_left, -1);
   return PIE_HIP_OK;
 }
 
@@ -1984,6 +1982,8 @@ static int attention_prefill_impl(
     PIE_REQUIRE(split[4] == prefill_scratch_bytes(split[1] - (num_items - split[3]), num_kv_heads, head_dim),
                 "attention_prefill: the split plan is for another head_dim or num_kv_heads than %lld, %lld",
                 (long long)head_dim, (long long)num_kv_heads);
+    // the pieces cover the kv range of the plan's mode and window; at others the uncut items run
+    cut = split[5] == mode && split[6] == std::max<int64_t>(window_left, -1);
   }
   if (num_items == 0) return PIE_HIP_OK;
   // The head-dim-128 kernel counts its work in the plan's header words, so runs of one plan must not

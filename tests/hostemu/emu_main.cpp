@@ -586,7 +586,7 @@ static void case_attn_prefill(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int
   const int64_t cap = 16 + 8 * (T * Hq / 32 + 2 * B + 2) + 4 * B + 8 + (T * Hq / 32 + 2 * B + 2) * Hkv + 4096;
   Buf<int32_t> plan(cap);
   int64_t words = 0, items = 0, mb = 0, mw = 0;
-  int64_t split[5] = {0, 0, 0, 0, 0};
+  int64_t split[7] = {};
   if (cut_cus)
     rc_ok(pie_hip_attention_prefill_split_plan(qi.p, ip.p, ll.p, B, P, Hq, Hkv, D, mode, window, cut_cus, 1ll << 30,
                                                plan.p, cap, &words, &items, &mb, &mw, split),
@@ -675,7 +675,7 @@ struct CutPrefill {
   const int64_t Hq = 2, Hkv = 1, P = 16, D, kv, qo;
   Buf<int32_t> qi{2}, ip{2}, ll{1}, idx, plan;
   Buf<uint16_t> cache;
-  int64_t words = 0, items = 0, mb = 0, mw = 0, split[5] = {0, 0, 0, 0, 0};
+  int64_t words = 0, items = 0, mb = 0, mw = 0, split[7] = {};
   CutPrefill(int64_t D_, int64_t kv_ = 790, int64_t qo_ = 3, int64_t window = -1)
       : D(D_), kv(kv_), qo(qo_), idx(pages()), plan(4096), cache(pages() * 2 * P * Hkv * D) {
     qi[0] = ip[0] = 0;
@@ -736,7 +736,7 @@ static void case_prefill_two_threads(int64_t D, int at, bool same_stream) {
   }
 }
 
-// A cut plan's run covers its own kv range whatever mode and window the plan was made for.
+// A run covers its own kv range whatever mode and window its cut plan was made for.
 static void case_prefill_cut_plan_other_range(int64_t D) {
   printf("prefill, cut plans run at another mode or window: D=%lld\n", (long long)D);
   struct { int64_t kv, qo, planned; int mode; int64_t window; } runs[] = {
