@@ -644,18 +644,19 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(PagedKV kv, int window_
 // rescale factor are its own (one exchange with lane ^ 32 for the max), and no factor has to be
 // broadcast to other lanes.
 //
-// What bounds it (rocprofv3 counters, 8 x 8192 tokens at head dim 128): MFMA 37% busy, VALU 40%, LDS
-// 28%, no bank conflicts; a wave waits 36% of its time, for the tile's loads (without them the
-// kernel takes 22% less) and at the barrier. Work groups of four 32-row waves in 64-token tiles,
-// each MFMA's V operands read a step ahead, against the four 2 x 16-row waves on 16x16x32 MFMAs in
-// 32-token tiles before: head dim 64, 4 x 4000 tokens 1,531 -> 827 us (674 TFLOP/s); head dim 256
-// (one 16-row tile per wave before) 1,858 -> 922 us (568 TFLOP/s). At head dim 256 one wave fits a
-// SIMD and nothing runs under its softmax.
+// What bounds it (rocprofv3 counters, 4 x 4000 causal tokens, shares of a SIMD's cycles). Head dim 64:
+// VALU 66%, MFMA 32%, LDS 12%; waves wait 26% of their time: a tile's softmax costs twice its MFMAs,
+// and the two hardly overlap. Head dim 256: MFMA 22%, VALU 30%, LDS 8%: one wave fits a SIMD and nothing
+// runs under its softmax and waits. No bank conflicts at either. Work groups of four 32-row waves in
+// 64-token tiles, each MFMA's V operands read a step ahead, against the four 2 x 16-row waves on
+// 16x16x32 MFMAs in 32-token tiles before (4 x 4000 causal tokens, 8 kv heads): head dim 64, 64 heads
+// 1,331 -> 690 us (760 TFLOP/s); head dim 256, 16 heads (one 16-row tile per wave before) 1,852 -> 934
+// us (562 TFLOP/s).
 constexpr int kPrefillRows = 128;
 // kv tokens per tile: 64, or 32 at head dim 256, whose accumulators fill the registers
 template <int D>
 constexpr int prefill_tile() { return D == 256 ? 32 : 64; }
-// work groups per CU the registers are budgeted for
+// work groups per CU the registers are budgeted for (at head dim 64 three fit: 164 registers, 34 KiB)
 template <int D>
 constexpr int prefill_groups() { return D == 256 ? 1 : 2; }
 constexpr int kPlanHeader = 16;  // plan words before the items: [0] items, [1] batch, [2] rows per item
@@ -1061,9 +1062,9 @@ __global__ __launch_bounds__(256, prefill_groups<D>()) void attn_prefill_kernel(
       }
       const float m_use = m_run == -INFINITY ? 0.f : m_run;
       // O^T += V^T P^T, 16 tokens at a time. Step j's MFMAs, the next step's V reads and its
-      // exponentials are independent, and pinned together: the reads first, then an equal share of
-      // the exponentials behind each MFMA. Left to itself the compiler reads each V operand right
-      // before its MFMA and waits for it there.
+      // exponentials are independent and stay together, the reads pinned before the MFMAs: left to
+      // itself the compiler reads each V operand right before its MFMA and waits for it there. (The
+      // exponentials are the compiler's to place: each pinned behind an MFMA is 2-4% slower.)
       float ps[2 * H2];
       u32x4_t pb[2];
       const auto probs = [&](int j) {
@@ -1084,10 +1085,7 @@ __global__ __launch_bounds__(256, prefill_groups<D>()) void attn_prefill_kernel(
         for (int bb = 0; bb < NB; ++bb) o[bb] = mfma_32x32x16(va[j & 1][bb], pb[j & 1], o[bb]);
         if (more) sched_group(0x100, 2 * NB);
 #pragma unroll
-        for (int bb = 0; bb < NB; ++bb) {
-          sched_group(0x008, 1);
-          
-        }
+        for (int bb = 0; bb < NB; ++bb) sched_group(0x008, 1);
         __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (H2 == 2) l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);
@@ -1675,10 +1673,13 @@ struct PrefillSplit {
 
 // The rule of the split list. Without it a request's rows walk its whole context in one work group:
 // 13 drafted tokens each over 4 contexts of 1-9k tokens took 253 us on 32 work groups and take 32 us
-// in 256-to-320-token pieces; one 700-token prompt 100 us, and 30 us. A launch fills num_cus * groups work groups; their mean share of the
-// kv tokens (over all items and kv heads) is the length a piece aims at, at least kSplitMinChunk,
-// below which a piece is mostly set-up. Items are cut only when the longest exceeds its pieces by
-// kSplitMinGain tokens: less than that the merge launch costs more than the cut saves.
+// in 256-to-320-token pieces; one 700-token prompt 100 us, and 30 us. A launch is counted as
+// num_cus * prefill_groups work groups (head dim 64 as 128, two per CU, although three fit); their mean
+// share of the kv tokens (over all items and kv heads) is the length a piece aims at, at least
+// kSplitMinChunk, below which a piece is mostly set-up. A custom mask is not looked at: its items count
+// their whole context, also where the mask is causal and the kernel stops sooner. Items are cut only
+// when the longest exceeds its pieces by kSplitMinGain tokens: less than that the merge launch costs
+// more than the cut saves.
 constexpr int64_t kSplitMinChunk = 256, kSplitMinGain = 512;
 
 // Bytes of the partial results of `pieces` pieces: kPrefillRows rows of D outputs and a log-sum-exp each.
