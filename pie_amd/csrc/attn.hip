@@ -672,8 +672,10 @@ constexpr int kPlanQueueWord = 8, kPlanDoneWord = 7;
 // instead of chasing b through qo_indptr / kv_indptr / kv_last_page_len; then, for an item split
 // over its kv range, the piece's index and 1 + its partial-result slot (0: not split)
 constexpr int kPlanItemWords = 8;
-// words per merge entry of a split plan: first packed row, q0, qo_len, first slot, pieces
+// words per merge entry of a split plan: first packed row, q0, qo_len, first slot, pieces, and
+// kMergeTag + the plan's rows word
 constexpr int kPlanMergeWords = 8;
+constexpr int kMergeTag = 0x4d520000;
 
 // XCD-aware order of the prefill grid: work groups are dispatched round-robin over the 8 XCDs
 // (id mod 8), each with its own L2, so XCD x takes the contiguous run [x * per, (x + 1) * per) of
@@ -1448,10 +1450,10 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
     const float* __restrict__ part_lse, uint16_t* __restrict__ out, int64_t o_ts, int64_t o_hs,
     const float* __restrict__ sinks) {
   constexpr int CH = D / 8;
-  if (plan[2] != plan_rows_word(D)) return;
   const int e = blockIdx.x / n_kv_heads, kvh = blockIdx.x - e * n_kv_heads;
   const int32_t* m = plan + merges_word + kPlanMergeWords * e;
   const int row0 = m[0], q0 = m[1], rows = m[2] * G, slot = m[3], pieces = m[4];
+  if (m[5] != kMergeTag + plan_rows_word(D)) return;  // (in the entry: the header is a load more to wait for)
   const int lane = threadIdx.x & 63, c = lane % CH;
   const int rl0 = blockIdx.y * (64 / CH);
   if (row0 + rl0 >= rows) return;
@@ -1805,7 +1807,7 @@ static int prefill_plan_impl(const int32_t* qo_indptr, const int32_t* kv_indptr,
     for (const Item& it : items) {
       const int32_t n = (int32_t)((it.span + chunk - 1) / chunk);
       if (n <= 1) { put(p, it, 0, 0); p += kPlanItemWords; continue; }
-      const int32_t w8[kPlanMergeWords] = {it.row0, it.q0, it.qo, slot, n, 0, 0, 0};
+      const int32_t w8[kPlanMergeWords] = {it.row0, it.q0, it.qo, slot, n, kMergeTag + plan_rows_word(head_dim), 0, 0};
       memcpy(m, w8, sizeof(w8));
       m += kPlanMergeWords;
       for (int32_t i = 0; i < n; ++i) { put(p, it, i, ++slot); p += kPlanItemWords; }
